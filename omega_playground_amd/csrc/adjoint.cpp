@@ -520,7 +520,7 @@ void restore(omega_tape_s *T, int slot, omega_state_s *S, hipStream_t s) {
 
 void advance(omega_tape_s *T, omega_state_s *S, int from, int count, hipStream_t s) {
   for (int i = 0; i < count; ++i)
-    do_step_maybe_graph(T->stepper, S, T->t0 + (from + i) * T->dt, T->dt, s);
+    do_step_maybe_graph(T->stepper, S, T->t0 + (from + i) * T->dt, T->dt, s, false);
   T->forward_steps += count;
 }
 
@@ -604,7 +604,7 @@ void tape_forward(omega_tape_s *T, double t0, double dt, omega_state_s *S, hipSt
   store(T, 0, S, s);
   size_t next = 0;
   for (int i = 0; i < T->nsteps; ++i) {
-    do_step_maybe_graph(T->stepper, S, t0 + i * dt, dt, s);
+    do_step_maybe_graph(T->stepper, S, t0 + i * dt, dt, s, i + 1 == T->nsteps);
     ++T->forward_steps;
     if (next < T->descent.size() && T->descent[next].first == i + 1)
       store(T, T->descent[next++].second, S, s);

@@ -498,6 +498,7 @@ int omega_model_set_f_vertex(omega_model_t M, const double *f) {
     for (int i = 0; i < dm.host.nvertices; ++i) tmp[i] = f[dm.vert_n2o[i]];
     M->f_v.upload(tmp);
     M->f_uniform = rows_equal(tmp, 1);
+    M->f_value = tmp.empty() ? 0 : tmp[0];
     M->touch();
   });
 }
@@ -922,7 +923,7 @@ int omega_stepper_run(omega_stepper_t St, double t0, double dt, int nsteps, int 
     OMEGA_REQUIRE(nsteps >= 0, "nsteps must be >= 0");
     check_state(St->model, S, "run");
     for (int i = 0; i < nsteps; ++i)
-      do_step_maybe_graph(St, S, t0 + (i + t_offset) * dt, dt, as_stream(stream));
+      do_step_maybe_graph(St, S, t0 + (i + t_offset) * dt, dt, as_stream(stream), i + 1 == nsteps);
   });
 }
 

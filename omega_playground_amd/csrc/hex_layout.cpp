@@ -7,7 +7,9 @@
 // cell edge must list the cell second for j < 3 and first for j >= 3.  Any
 // mismatch leaves hex_ok false and the general kernels are used.
 #include <algorithm>
+#include <cmath>
 
+#include "hex_lattice.hpp"
 #include "hex_pattern.hpp"
 #include "internal.hpp"
 
@@ -140,6 +142,122 @@ bool build_hex_records(DeviceMesh &dm) {
   }
   dm.hexu_ok = true;
   return true;
+}
+
+// Every table the one-launch stage kernels replace by lattice arithmetic is
+// checked here: neighbours that step back and round a corner as on the
+// lattice (then the cell at an offset does not depend on the path to it),
+// edges, vertices and edges-on-edge at their lattice places, and one
+// magnitude per coefficient kind with the signs and TRiSK multiples of
+// hex_lattice.hpp, bit for bit.
+void build_hex_stage(DeviceMesh &dm) {
+  dm.stage_ok = false;
+  dm.hexc_h.clear();
+  const HostMesh &m = dm.host;
+  const int NC = m.ncells, ME = m.max_edges;
+  if (!dm.hex_ok || !dm.coef_uni || !dm.off32 || dm.me2 != hex::kSlots) return;
+  namespace hl = hexl;
+  HexCoef &q = dm.stage_coef;
+  const double C = dm.cdiv_h[3], ke = dm.cke_h[0], R = dm.crv_h[0], th = dm.cth_h[0];
+  const double w1 = dm.w_h[1];
+  for (int j = 0; j < 6; ++j)
+    if (dm.cdiv_h[j] != (j < 3 ? -C : C) || dm.cke_h[j] != ke) return;
+  for (int x = 0; x < 2; ++x)
+    for (int j = 0; j < 3; ++j)
+      if (dm.crv_h[3 * x + j] != hl::vert(x).s[j] * R || dm.cth_h[3 * x + j] != th) return;
+  for (int K = 0; K < 3; ++K)
+    for (int j = 0; j < 10; ++j)
+      if (dm.w_h[K * 10 + j] != hl::pv_mult(K, j) * w1) return;
+  // products by powers of two must be exact: no tiny coefficients
+  for (double x : {C, ke, R, th, w1})
+    if (!(std::fabs(x) > 1e-200 && std::fabs(x) < 1e200)) return;
+  const int *coc = dm.coc_h.data();
+  for (int c = 0; c < NC; ++c)
+    for (int d = 0; d < 6; ++d) {
+      const int n = coc[6 * (size_t)c + d];
+      if (coc[6 * (size_t)n + (d + 3) % 6] != c) return;
+      if (coc[6 * (size_t)n + (d + 2) % 6] != coc[6 * (size_t)c + (d + 1) % 6]) return;
+    }
+  dm.hexc_h.assign((size_t)NC * hl::kRec, 0);
+  for (int c = 0; c < NC; ++c) {
+    int *r = &dm.hexc_h[(size_t)c * hl::kRec];
+    r[0] = c;
+    for (int d = 0; d < 6; ++d) r[1 + d] = coc[6 * (size_t)c + d];
+    for (int d = 0; d < 6; ++d) {
+      r[7 + 2 * d] = coc[6 * (size_t)r[1 + d] + d];
+      r[8 + 2 * d] = coc[6 * (size_t)r[1 + d] + (d + 1) % 6];
+    }
+    auto eid = [&](int e) { return 3 * r[e / 3] + e % 3; };
+    auto vid = [&](int v) { return 2 * r[v / 2] + v % 2; };
+    bool ok = true;
+    for (int d = 0; d < 6; ++d) ok = ok && dm.eoc_h[(size_t)c * ME + d] == eid(hl::cell_edge(0, d));
+    for (int K = 0; K < 3; ++K) {
+      const size_t e = 3 * (size_t)c + K;
+      const hl::Edge t = hl::edge(K);
+      for (int s = 0; s < 2; ++s)
+        ok = ok && dm.coe_h[2 * e + s] == r[t.c[s]] && dm.voe_h[2 * e + s] == vid(t.v[s]);
+      for (int j = 0; j < 10; ++j) ok = ok && dm.eoe_h[e * 10 + j] == eid(hl::pv_edge(K, j));
+    }
+    for (int x = 0; x < 2; ++x) {
+      const size_t v = 2 * (size_t)c + x;
+      const hl::Vert t = hl::vert(x);
+      for (int j = 0; j < 3; ++j)
+        ok = ok && dm.eov_h[3 * v + j] == eid(t.e[j]) && dm.cov_h[3 * v + j] == r[t.c[j]];
+    }
+    if (!ok) {
+      dm.hexc_h.clear();
+      return;
+    }
+  }
+  q.crv = R;
+  q.cth = th;
+  q.w = w1;
+  q.w2 = w1 / 2;
+  q.cke = ke;
+  q.cdiv = C;
+  q.hdiv = C / 2;
+  q.qdiv = C / 4;
+  q.idc = dm.inv_dc_h[0];
+  q.idv = dm.inv_dv_h[0];
+  q.idv4 = dm.inv_dv4_h[0];
+  q.s2 = dm.s2_h[0];
+  q.ml = dm.maxlev_h[0];
+  // place every cell on the lattice: rows of nx cells running E, the next row
+  // NE of an even one and NW of an odd one
+  int nx = 0;
+  for (int c = 0; nx == 0 || c != 0; c = coc[6 * (size_t)c + 3], ++nx)
+    if (nx > NC) return;
+  if (NC % nx || (NC / nx) % 2) return;
+  const int ny = NC / nx;
+  std::vector<int> at((size_t)NC), seen((size_t)NC, 0);
+  for (int r = 0, first = 0; r < ny; ++r) {
+    for (int i = 0, c = first; i < nx; ++i, c = coc[6 * (size_t)c + 3]) {
+      at[(size_t)r * nx + i] = c;
+      if (seen[c]++) return;
+    }
+    first = coc[6 * (size_t)first + (r % 2 ? 5 : 4)];
+    if (r + 1 == ny && first != 0) return; // the rows close without a shift
+  }
+  // block shape: four lanes of two levels and 8 x 8 cells; with fewer lanes
+  // of levels more cells
+  TileView &t = dm.tile;
+  const int lanes = m.nlayers % 2 == 0 ? m.nlayers / 2 : m.nlayers;
+  t.lx = lanes >= 3 ? 4 : lanes;
+  t.tw = t.lx == 4 ? 8 : 16;
+  t.th = t.lx == 1 ? 16 : 8;
+  t.nx = nx;
+  t.ny = ny;
+  const int tx = (nx + t.tw - 1) / t.tw, ty = (ny + t.th - 1) / t.th;
+  dm.tile_h.clear();
+  dm.tile_h.reserve((size_t)tx * ty * (t.tw + 4) * (t.th + 4));
+  for (int j = 0; j < ty; ++j)
+    for (int i = 0; i < tx; ++i)
+      for (int y = -2; y < t.th + 2; ++y)
+        for (int x = -2; x < t.tw + 2; ++x) {
+          const int r = ((j * t.th + y) % ny + ny) % ny, q = ((i * t.tw + x) % nx + nx) % nx;
+          dm.tile_h.push_back(at[(size_t)r * nx + q]);
+        }
+  dm.stage_ok = true;
 }
 
 } // namespace omega_hip

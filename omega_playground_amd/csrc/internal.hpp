@@ -101,6 +101,14 @@ void build_planar_hex(HostMesh &m, int nx, int ny, double dc, int nlayers);
 // ---------------------------------------------------------------------------
 // Device mesh: reordered connectivity plus host-precomputed coefficients.
 // ---------------------------------------------------------------------------
+// Tiles of the lattice for the kernels that stage a tile in LDS: tw x th
+// cells (th even) and lx lanes per block, tiles row by row; ids holds each
+// tile's cells with two rings of halo, [tiles][(th + 4)(tw + 4)]
+struct TileView {
+  const int *ids;
+  int nx, ny, tw, th, lx;
+};
+
 struct MeshView {
   int nc, ne, nv, L;
   int me;   // row length of per-cell tables
@@ -130,6 +138,20 @@ struct MeshView {
   const int *hexrec;            // [ne][30]
   const int *hexu;              // [nc][49] per-cell union stencil (hex_pattern.hpp)
   const int *coc;               // cells_on_cell [nc][6]
+  const int *hexc;              // [nc][20] neighbourhood cells (hex_lattice.hpp)
+  TileView tile;                // ids null where the mesh has no tiles
+};
+
+// Coefficients of the one-launch stage kernels (hex_stage.hpp): one value per
+// kind for the whole mesh, with the stencils' constant factors folded in
+struct HexCoef {
+  Real crv, cth;       // |crv|, cth
+  Real w, w2;          // smallest nonzero TRiSK weight, and half of it
+  Real cke, cdiv, hdiv, qdiv; // cke, |cdiv|, |cdiv| / 2, |cdiv| / 4
+  Real idc, idv, idv4; // 1/dc, 1/dv, 1/max(dv, dc/4)
+  Real f, grav, cv2, cv4;
+  Real ct2, s2, ct4;   // |ct2| / 2, mesh_scaling_del2, |ct4|
+  int ml;              // max_level_edge_top
 };
 
 struct DeviceMesh {
@@ -153,8 +175,15 @@ struct DeviceMesh {
   bool coef_uni = false; // coefficient tables equal at every stencil slot
   bool off32 = false;    // 32-bit byte offsets suffice for every row array
   bool hexd_ok = false; // owned vertices follow the diagnostics maps (hexd)
-  std::vector<int> hexrec_h, coc_h, hexu_h;
-  DBuf<int> hexrec, coc, hexu;
+  std::vector<int> hexrec_h, coc_h, hexu_h, hexc_h;
+  DBuf<int> hexrec, coc, hexu, hexc;
+  // the mesh is the lattice of hex_lattice.hpp with one value per coefficient
+  // kind (stage_coef holds the mesh's share); hexc_h its neighbourhood records
+  bool stage_ok = false;
+  std::vector<int> tile_h;
+  DBuf<int> tile_ids;
+  TileView tile{};
+  HexCoef stage_coef{};
 
   bool uploaded = false;
 
@@ -167,6 +196,9 @@ struct DeviceMesh {
 std::vector<int> order_cells(const HostMesh &m, int ordering);
 // Builds and verifies the regular-hexagon records (hex_layout.cpp).
 bool build_hex_records(DeviceMesh &dm);
+// Neighbourhood records and uniform coefficients of the one-launch stage
+// kernels (hex_layout.cpp); sets stage_ok.
+void build_hex_stage(DeviceMesh &dm);
 
 // ---------------------------------------------------------------------------
 // Launch configuration and kernel parameter blocks
@@ -212,6 +244,7 @@ struct DiagOut {
   Real *trdel2_c;              // [ntr][nc][L]
   Real *vdel2_e;               // [ne][L]  (momentum del4 pre-pass)
   Real *vdel2_rv_v, *vdel2_div_c;
+  Real *vdel4_e;               // [ne][L]  del4 term of the stage kernels
 };
 
 struct ModelCoef {
@@ -282,6 +315,12 @@ void launch_diag_hex(const MeshView &m, const Launch &lc, int terms, int ntr, co
                      const Real *vn, const Real *tr, const DiagOut &d, hipStream_t s);
 void launch_tend_hex(const MeshView &m, const Launch &lc, const ModelCoef &mc, const StageArgs &a,
                      const DiagOut &d, hipStream_t s, const PreOut *pre = nullptr);
+// Stage on the lattice mesh with uniform coefficients, without a diagnostics
+// launch (kernels_stage.hip): tendencies and stage update of every field.
+// emit: also write the stage input's diagnostics to d; d's momentum del4 rows
+// (vdel2_e, vdel4_e) are scratch in any case.
+void launch_stage_hex(const MeshView &m, const Launch &lc, const HexCoef &q, const StageArgs &a,
+                      const DiagOut &d, bool emit, hipStream_t s);
 // y += alpha*x elementwise
 void launch_axpy(Real *y, Real alpha, const Real *x, size_t n, hipStream_t s);
 // y = x + alpha*z elementwise

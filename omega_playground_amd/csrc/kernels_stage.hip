@@ -1,0 +1,415 @@
+// Forward stage on the regular hexagonal mesh with uniform coefficients, any
+// layer count: one launch for momentum and thickness (hex_stage.hpp), one for
+// the tracers, two more before them with momentum del4.  No diagnostics
+// launch: each kernel forms what it needs from the prognostic rows.
+//
+// Against a diagnostics launch and a tendency launch that gather about 260
+// rows per cell (nx=512, 64 layers, 4 tracers, del2 viscosity, tracer del4):
+// 2.37 -> 1.57 ms per RK4 stage, 68 -> 44 rows per cell through HBM.  At 60
+// layers, where that pair ran the general kernels, 0.250 -> 0.077 ms (150 x
+// 94 cells, 3 tracers); one layer, 512 x 384 cells: 0.135 -> 0.019 ms.
+#include <algorithm>
+
+#include "hex_stage.hpp"
+
+namespace omega_hip {
+
+namespace {
+
+using namespace stage;
+
+struct StageLaunch {
+  HexCoef q;
+  const int *rec;
+  int nc, L, ncb, tiles, per_xcd;
+  StageArgs a;
+  DiagOut d;
+  const double *x; // k_stage_lap: the edge field, its result
+  double *y;
+};
+
+// Block b runs on XCD b mod 8 (workgroups are dealt round-robin) and takes
+// that XCD's contiguous range of (level chunk, cell block) pairs, so that
+// neighbouring cells' rows are re-read from one L2.  False: no work here.
+__device__ __forceinline__ bool stage_place(const StageLaunch &p, int N, int &c, Ctx &x) {
+  const int tile = ((int)blockIdx.x & 7) * p.per_xcd + ((int)blockIdx.x >> 3);
+  if (tile >= p.tiles) return false;
+  const int ch = p.tiles == p.ncb ? 0 : uniform(tile / p.ncb);
+  c = (tile - ch * p.ncb) * (int)blockDim.y + (int)threadIdx.y;
+  const int k = (ch * (int)blockDim.x + (int)threadIdx.x) * N;
+  x = Ctx{p.L, (unsigned)p.L * 8u, (unsigned)k * 8u, k};
+  return c < p.nc && k < p.L;
+}
+
+// Momentum and thickness.  Two levels per lane at two waves per SIMD (228
+// registers) take 0.70 ms at nx=512, 64 layers (3.6 TB/s; the vector units
+// half busy, the rest latency), one level per lane at four waves 0.83 ms (the
+// same rows in twice the load instructions).
+// V4: subtract the del4 rows (p.x) the Laplacian launches left.
+template <int N, bool V2, bool V4, bool EMIT>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N == 1 ? 4 : 2)))
+    k_stage_mom(StageLaunch p) {
+  int c;
+  Ctx x;
+  if (!stage_place(p, N, c, x)) return;
+  const StageArgs &a = p.a;
+  const int L = x.L, k = x.k;
+  int id[hl::kCells];
+  load_cells(p.rec, c, id);
+  const size_t idx = (size_t)c * L + k, e0 = (size_t)(3 * c) * L + k;
+  MomOut<N> o;
+  momentum<N, V2>(p.q, x, id, a.h.in, a.vn.in, o);
+  if constexpr (EMIT) {
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      const size_t vi = (size_t)(2 * c + w) * L + k;
+      st<N>(p.d.rvort_v + vi, o.rv[w]);
+      st<N>(p.d.inv_thick_v + vi, o.it[w]);
+    }
+    st<N>(p.d.ke_c + idx, o.ke);
+    st<N>(p.d.div_c + idx, o.div);
+  }
+#pragma unroll
+  for (int K = 0; K < 3; ++K) {
+    Vd<N> T = tend_base<N>(a, a.vn, e0 + K * L);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      T[i] = T[i] + o.u[K][i];
+      T[i] = T[i] - o.ke_grad[K][i];
+      T[i] = T[i] - o.ssh_grad[K][i];
+      if constexpr (V2) T[i] = T[i] + o.visc[K][i];
+    }
+    if constexpr (V4) {
+      const Vd<N> y = ld<N>(p.x + e0 + K * L);
+#pragma unroll
+      for (int i = 0; i < N; ++i) T[i] = T[i] - y[i];
+    }
+    epilogue<N>(a, a.vn, e0 + K * L, T);
+  }
+  Vd<N> T = tend_base<N>(a, a.h, idx);
+#pragma unroll
+  for (int i = 0; i < N; ++i) T[i] = T[i] + o.h[i];
+  epilogue<N>(a, a.h, idx, T);
+}
+
+// The edge Laplacian: of the velocity (FINAL false), then of that result,
+// with the masked coefficient applied (FINAL).
+template <int N, bool FINAL, bool EMIT>
+__global__ void __launch_bounds__(256) k_stage_lap(StageLaunch p) {
+  int c;
+  Ctx x;
+  if (!stage_place(p, N, c, x)) return;
+  int id[hl::kCells];
+  load_cells(p.rec, c, id);
+  LapOut<N> o;
+  laplacian<N>(p.q, FINAL ? p.q.idv : p.q.idv4, x, id, p.x, o);
+  const size_t e0 = (size_t)(3 * c) * x.L + x.k;
+#pragma unroll
+  for (int K = 0; K < 3; ++K) {
+    if constexpr (FINAL) {
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        o.e[K][i] = ((x.k + i < p.q.ml) ? p.q.cv4 : 0.0) * o.e[K][i];
+    }
+    st<N>(p.y + e0 + K * x.L, o.e[K]);
+  }
+  if constexpr (EMIT) {
+#pragma unroll
+    for (int w = 0; w < 2; ++w) st<N>(p.d.vdel2_rv_v + (size_t)(2 * c + w) * x.L + x.k, o.curl[w]);
+    st<N>(p.d.vdel2_div_c + (size_t)c * x.L + x.k, o.div);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Tracers: a block stages a tile of the lattice, TW x TH cells with one ring
+// of halo (two with del4) and LX lanes of N levels, in LDS, so that a
+// neighbour's tracer ratio and Laplacian are formed once per tile instead of
+// once per cell that reads them: 0.86 ms per stage at nx=512, 64 layers, 4
+// tracers with del4 (0.64 without, 90 % of a copy's rate), against 1.49 ms
+// for one cell per thread with both rings in registers (19 divisions and 19
+// rows per cell and tracer).  A thread computes its own cell's Laplacian and
+// at most one of the ring's, with the sums of its cell's thicknesses kept in
+// registers for all tracers.  Tiles of 64-byte rows (LX = 4, N = 2) ran
+// faster than 128-byte ones (6.3 against 7.2 ms per step), three waves per
+// SIMD faster than four with 13 registers spilled (6.3 against 7.0).
+// ---------------------------------------------------------------------------
+struct TileLaunch {
+  HexCoef q;
+  const int *ids; // [tiles][(TH + 4)(TW + 4)] cell at each place, row-major
+  int nx, ny, tiles_x, nch, work, per_xcd, nc, L, per_block;
+  StageArgs a;
+  DiagOut d;
+};
+
+template <int N, int LX, int TW, int TH, bool D2, bool D4, bool EMIT>
+__global__ void __launch_bounds__(LX *TW *TH) __attribute__((amdgpu_waves_per_eu(N == 2 ? 3 : 4)))
+    k_stage_tile(TileLaunch p) {
+  constexpr int HALO = D4 ? 2 : 1, PW = TW + 2 * HALO, PH = TH + 2 * HALO, NP = PW * PH;
+  constexpr int CELLS = TW * TH, R = (NP + CELLS - 1) / CELLS;
+  constexpr int RING = 2 * (TW + 2) + 2 * TH; // the first ring round the tile
+  static_assert(RING <= CELLS, "one place of the ring per row of lanes");
+  constexpr int S = LX * N, PLANE = NP * S; // doubles per place and per array
+  __shared__ double Hs[PLANE], Ns[PLANE], Ds[D4 ? PLANE : 1];
+  __shared__ int ids[NP];
+  const int w = ((int)blockIdx.x & 7) * p.per_xcd + ((int)blockIdx.x >> 3);
+  if (w >= p.work) return;
+  const int tile = uniform(w / p.nch), ch = w - tile * p.nch;
+  const int ln = (int)threadIdx.x % LX, row = (int)threadIdx.x / LX;
+  const int L = p.L, k = (ch * LX + ln) * N;
+  const bool lev = k < L;
+  const unsigned L8 = (unsigned)L * 8u, k8 = (unsigned)k * 8u;
+  const size_t sp = (size_t)p.nc * L;
+  const StageArgs &a = p.a;
+  const HexCoef &q = p.q;
+  const int *tid = p.ids + (size_t)tile * ((TW + 4) * (TH + 4));
+  for (int i = (int)threadIdx.x; i < NP; i += LX * CELLS)
+    ids[i] = tid[(i / PW + 2 - HALO) * (TW + 4) + i % PW + 2 - HALO];
+  __syncthreads();
+  const int l0 = (int)blockIdx.y * p.per_block, l1 = min(l0 + p.per_block, a.ntr);
+  // the places this thread stages: thickness, its inverse, the first tracer
+  Vd<N> inv[R], t[R];
+  unsigned off[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int pos = row + r * CELLS;
+    if (pos < NP && lev) {
+      off[r] = __umul24((unsigned)ids[pos], L8) + k8;
+      inv[r] = ldo<N>(a.h.in, off[r]);
+      t[r] = ldo<N>(a.tr.in + l0 * sp, off[r]);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int pos = row + r * CELLS;
+    if (pos < NP && lev) {
+      st<N>(Hs + pos * S + ln * N, inv[r]);
+#pragma unroll
+      for (int i = 0; i < N; ++i) inv[r][i] = 1.0 / inv[r][i];
+    }
+  }
+  // A place's neighbours W, SW, SE, E, NE, NW are at fixed distances from it,
+  // those of other rows one place further right in odd rows: two bases,
+  // lowered by a row so that every distance is positive
+  struct Place {
+    int same, other; // index of the element a row below and one left
+  };
+  auto place = [&](int x, int y) {
+    const int i = ((y - 1) * PW + x - 1) * S + ln * N;
+    return Place{i, i + ((y + HALO) & 1) * S};
+  };
+  auto get = [&](const double *A, const Place &o, auto J) {
+    constexpr int j = J; // 0 the place itself, 1 + d its neighbour in direction d
+    constexpr int by[7] = {PW + 1, PW, 0, 1, PW + 2, 2 * PW + 1, 2 * PW};
+    constexpr bool same = j < 2 || j == 4;
+    return ld<N>(A + (same ? o.same : o.other) + by[j] * S);
+  };
+  // the thread's own cell (tile rows start at even rows of the lattice, and
+  // so do staged rows)
+  const int cy = row / TW, cx = row % TW;
+  const Place own = place(cx + HALO, cy + HALO);
+  const int self = (cy + HALO) * PW + cx + HALO;
+  const bool mine = lev && (tile % p.tiles_x) * TW + cx < p.nx && (tile / p.tiles_x) * TH + cy < p.ny;
+  Vd<N> v[6];
+  if (mine) {
+    const int odd = cy & 1;
+    const int c4[6] = {ids[self], ids[self], ids[self], ids[self + 1], ids[self + PW + odd],
+                       ids[self + PW - 1 + odd]};
+#pragma unroll
+    for (int j = 0; j < 6; ++j)
+      v[j] = ldo<N>(a.vn.in + (j % 3) * L, __umul24((unsigned)c4[j], 3u * L8) + k8);
+  }
+  __syncthreads();
+  Vd<N> f[6];
+  {
+    const Vd<N> h0 = get(Hs, own, std::integral_constant<int, 0>{});
+    each<6>([&](auto J) {
+      const Vd<N> hj = get(Hs, own, std::integral_constant<int, 1 + J>{});
+#pragma unroll
+      for (int i = 0; i < N; ++i) f[J][i] = hj[i] + h0[i];
+    });
+  }
+  const int c = ids[self];
+  // this thread's place on the ring: the rows below and above, then the sides
+  const int rr = row < RING ? row : 0, side = rr - 2 * (TW + 2);
+  const Place ring = side < 0 ? place(rr % (TW + 2) + 1, rr < TW + 2 ? 1 : TH + 2)
+                             : place(side & 1 ? TW + 2 : 1, side / 2 + 2);
+  for (int l = l0; l < l1; ++l) {
+    if (l > l0) __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int pos = row + r * CELLS;
+      if (pos < NP && lev) {
+        Vd<N> n;
+#pragma unroll
+        for (int i = 0; i < N; ++i) n[i] = t[r][i] * inv[r][i];
+        st<N>(Ns + pos * S + ln * N, n);
+        if (l + 1 < l1) t[r] = ldo<N>(a.tr.in + (l + 1) * sp, off[r]);
+      }
+    }
+    const size_t idx = ((size_t)l * p.nc + c) * L + k;
+    EpiIn<N> e;
+    if (mine) e = epi_prefetch<N>(a, a.tr, idx);
+    __syncthreads();
+    // the cell's tracer Laplacian (D4) and advection, from its neighbours' ratios
+    const double qdiv = each_time(q.qdiv), hdiv = each_time(q.hdiv);
+    const Vd<N> n0 = get(Ns, own, std::integral_constant<int, 0>{});
+    Vd<N> d0 = zero<N>(), adv = zero<N>(), dif = zero<N>(), hyp = zero<N>();
+    each<6>([&](auto J) {
+      constexpr int j = J;
+      const Vd<N> nj = get(Ns, own, std::integral_constant<int, 1 + j>{});
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const double g = (j < 3 ? n0[i] - nj[i] : nj[i] - n0[i]) * q.idc;
+        const double x = (qdiv * f[j][i]) * (nj[i] + n0[i]) * v[j][i];
+        adv[i] = j < 3 ? adv[i] + x : adv[i] - x;
+        if constexpr (D2) {
+          const double y = q.ct2 * f[j][i] * q.s2 * g;
+          dif[i] = j < 3 ? dif[i] - y : dif[i] + y;
+        }
+        if constexpr (D4) {
+          const double z = (hdiv * f[j][i]) * g;
+          d0[i] = j < 3 ? d0[i] - z : d0[i] + z;
+        }
+      }
+    });
+    pin(adv);
+    if constexpr (D2) pin(dif);
+    if constexpr (D4) {
+      st<N>(Ds + own.same + (PW + 1) * S, d0);
+      if (row < RING) {
+        Place rim = ring;
+        rim.same = (int)again((unsigned)rim.same);
+        rim.other = (int)again((unsigned)rim.other);
+        const Vd<N> h0 = get(Hs, rim, std::integral_constant<int, 0>{});
+        const Vd<N> r0 = get(Ns, rim, std::integral_constant<int, 0>{});
+        Vd<N> d = zero<N>();
+        each<6>([&](auto J) {
+          constexpr int j = J;
+          const Vd<N> hj = get(Hs, rim, std::integral_constant<int, 1 + j>{});
+          const Vd<N> nj = get(Ns, rim, std::integral_constant<int, 1 + j>{});
+#pragma unroll
+          for (int i = 0; i < N; ++i) {
+            const double m = hdiv * (hj[i] + h0[i]);
+            const double y = m * ((j < 3 ? r0[i] - nj[i] : nj[i] - r0[i]) * q.idc);
+            d[i] = j < 3 ? d[i] - y : d[i] + y;
+          }
+        });
+        st<N>(Ds + rim.same + (PW + 1) * S, d);
+      }
+      __syncthreads();
+      each<6>([&](auto J) {
+        constexpr int j = J;
+        const Vd<N> dj = get(Ds, own, std::integral_constant<int, 1 + j>{});
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          const double z = q.ct4 * ((j < 3 ? d0[i] - dj[i] : dj[i] - d0[i]) * q.idc);
+          hyp[i] = j < 3 ? hyp[i] + z : hyp[i] - z;
+        }
+      });
+      pin(hyp);
+    }
+    if (mine) {
+      Vd<N> T;
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        T[i] = e.base[i] + adv[i];
+        if constexpr (D2) T[i] = T[i] + dif[i];
+        if constexpr (D4) T[i] = T[i] + hyp[i];
+      }
+      if constexpr (EMIT && D4) st<N>(p.d.trdel2_c + idx, d0);
+      epi_finish<N>(a, a.tr, idx, T, e);
+    }
+  }
+}
+
+using StageFn = void (*)(StageLaunch);
+using TileFn = void (*)(TileLaunch);
+
+template <int N, bool EMIT> StageFn pick_mom(bool v2, bool v4) {
+  if (v4) return v2 ? k_stage_mom<N, true, true, EMIT> : k_stage_mom<N, false, true, EMIT>;
+  return v2 ? k_stage_mom<N, true, false, EMIT> : k_stage_mom<N, false, false, EMIT>;
+}
+
+// without del4 there is no Laplacian to emit
+template <int N, int LX, int TW, int TH, bool EMIT> TileFn pick_shape(bool d2, bool d4) {
+  if (d4)
+    return d2 ? k_stage_tile<N, LX, TW, TH, true, true, EMIT>
+              : k_stage_tile<N, LX, TW, TH, false, true, EMIT>;
+  return d2 ? k_stage_tile<N, LX, TW, TH, true, false, false>
+            : k_stage_tile<N, LX, TW, TH, false, false, false>;
+}
+template <int N, bool EMIT> TileFn pick_tile(const TileView &t, bool d2, bool d4) {
+  if (t.lx == 4) return pick_shape<N, 4, 8, 8, EMIT>(d2, d4);
+  if (t.lx == 2) return pick_shape<N, 2, 16, 8, EMIT>(d2, d4);
+  return pick_shape<N, 1, 16, 16, EMIT>(d2, d4);
+}
+
+} // namespace
+
+void launch_stage_hex(const MeshView &m, const Launch &lc, const HexCoef &q, const StageArgs &a,
+                      const DiagOut &d, bool emit, hipStream_t s) {
+  TimerScope ts("tend", s);
+  const int N = lc.lpt == 2 && m.L % 2 == 0 ? 2 : 1;
+  const int lanes = (m.L + N - 1) / N;
+  // cells' lanes per block: up to 16 (32 levels), so that a block's cells
+  // share more of their neighbours' rows in L1 (2.81 against 2.85 ms per step
+  // for momentum alone at nx=512, 64 layers with 32, 2.94 with 8)
+  const int want = lc.chunk > 0 ? std::min(std::max(1, lc.chunk / N), 64) : 16;
+  const int nch = (lanes + want - 1) / want, lx = (lanes + nch - 1) / nch;
+  const int rows = lc.rows > 0 ? std::min(lc.rows, 256 / lx) : 256 / lx;
+  StageLaunch p{};
+  p.q = q;
+  p.rec = m.hexc;
+  p.nc = m.nc;
+  p.L = m.L;
+  p.ncb = (m.nc + rows - 1) / rows;
+  p.tiles = p.ncb * nch;
+  p.per_xcd = (p.tiles + 7) / 8;
+  p.a = a;
+  p.d = d;
+  const dim3 grid(8 * p.per_xcd), block(lx, rows);
+  const bool v4 = a.terms & T_VDEL4;
+  if (v4) {
+    p.x = a.vn.in;
+    p.y = d.vdel2_e;
+    hipLaunchKernelGGL((N == 2 ? k_stage_lap<2, false, false> : k_stage_lap<1, false, false>), grid,
+                       block, 0, s, p);
+    p.x = d.vdel2_e;
+    p.y = d.vdel4_e;
+    const StageFn k = N == 2 ? (emit ? k_stage_lap<2, true, true> : k_stage_lap<2, true, false>)
+                             : (emit ? k_stage_lap<1, true, true> : k_stage_lap<1, true, false>);
+    hipLaunchKernelGGL(k, grid, block, 0, s, p);
+    p.x = d.vdel4_e;
+  }
+  const bool v2 = a.terms & T_VDEL2, d2 = a.terms & T_TDEL2, d4 = a.terms & T_TDEL4;
+  const StageFn k = N == 2 ? (emit ? pick_mom<2, true>(v2, v4) : pick_mom<2, false>(v2, v4))
+                           : (emit ? pick_mom<1, true>(v2, v4) : pick_mom<1, false>(v2, v4));
+  hipLaunchKernelGGL(k, grid, block, 0, s, p);
+  if (a.ntr > 0) {
+    const TileView &tv = m.tile;
+    TileLaunch t{};
+    t.q = q;
+    t.ids = tv.ids;
+    t.nx = tv.nx;
+    t.ny = tv.ny;
+    t.tiles_x = (tv.nx + tv.tw - 1) / tv.tw;
+    t.nch = (lanes + tv.lx - 1) / tv.lx;
+    t.work = t.tiles_x * ((tv.ny + tv.th - 1) / tv.th) * t.nch;
+    t.per_xcd = (t.work + 7) / 8;
+    t.nc = m.nc;
+    t.L = m.L;
+    // one block takes all tracers of its tile, keeping the tile's thicknesses
+    // and velocities; where the tiles alone leave the chip short of blocks
+    // (fewer than 512) each tracer has its own
+    t.per_block = t.work >= 512 ? a.ntr : 1;
+    t.a = a;
+    t.d = d;
+    const TileFn kt = N == 2 ? (emit ? pick_tile<2, true>(tv, d2, d4) : pick_tile<2, false>(tv, d2, d4))
+                             : (emit ? pick_tile<1, true>(tv, d2, d4) : pick_tile<1, false>(tv, d2, d4));
+    hipLaunchKernelGGL(kt, dim3(8 * t.per_xcd, (a.ntr + t.per_block - 1) / t.per_block),
+                       dim3(tv.lx * tv.tw * tv.th), 0, s, t);
+  }
+  OMEGA_HIP_CHECK(hipGetLastError());
+}
+
+} // namespace omega_hip

@@ -431,6 +431,7 @@ void DeviceMesh::build_device(int ord) {
              rows_equal(cke_h, ME) && rows_equal(crv_h, 6) && rows_equal(cth_h, 6);
   const size_t rows = std::max({(size_t)NC, (size_t)NE, (size_t)NV});
   off32 = rows < (size_t(1) << 24) && rows * (size_t)L * sizeof(double) < (size_t(1) << 32);
+  build_hex_stage(*this);
   uploaded = false;
 }
 
@@ -450,6 +451,10 @@ void DeviceMesh::upload() {
     hexrec.upload(hexrec_h);
     if (hexu_ok) hexu.upload(hexu_h);
     coc.upload(coc_h);
+    if (stage_ok) {
+      hexc.upload(hexc_h);
+      tile_ids.upload(tile_h);
+    }
   }
 
   auto perm_upload = [](DBuf<Real> &dst, const std::vector<double> &src,
@@ -509,6 +514,9 @@ MeshView DeviceMesh::view() const {
   v.hexrec = hexrec.p;
   v.hexu = hexu.p;
   v.coc = coc.p;
+  v.hexc = hexc.p;
+  v.tile = tile;
+  v.tile.ids = tile_ids.p;
   return v;
 }
 

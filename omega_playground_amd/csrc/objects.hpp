@@ -67,6 +67,7 @@ struct omega_model_s {
   const Real *aux_h = nullptr, *aux_vn = nullptr, *aux_tr = nullptr;
   DBuf<Real> f_v, cv2, cv4, ct2, ct4;
   DBuf<Real> rvort_v, inv_thick_v, ke_c, div_c, trdel2_c, vdel2_e, vdel2_rv_v, vdel2_div_c;
+  DBuf<Real> vdel4_e; // scratch of the stage kernels with momentum del4
   DBuf<Real> partial, result;
   omega_additional_tendency_fn add_fn = nullptr;
   void *add_user = nullptr;
@@ -104,6 +105,10 @@ struct omega_model_s {
     if (!(forms & 4)) v.term_sets = 0;
     return v;
   }
+  // coefficients of the stage kernels without a diagnostics launch; false where this model's
+  // mesh, coefficients, terms or kernel forms need the other kernels
+  bool stage_coef(omega_hip::HexCoef &q) const;
+  Real f_value = 0; // the Coriolis parameter where f_uniform
   ModelCoef coef() const {
     return ModelCoef{params.grav, f_v.p, cv2.p, cv4.p, ct2.p, ct4.p,
                      f_uniform && mix_uniform ? 1 : 0, params.drag_coeff};
@@ -126,26 +131,29 @@ struct omega_model_s {
     if (diag_slot > 0) {
       DiagSet &d = diag_sets[diag_slot - 1];
       return DiagOut{d.rvort_v.p, d.inv_thick_v.p, d.ke_c.p, d.div_c.p, d.trdel2_c.p,
-                     d.vdel2_e.p, d.vdel2_rv_v.p, d.vdel2_div_c.p};
+                     d.vdel2_e.p, d.vdel2_rv_v.p, d.vdel2_div_c.p, vdel4_e.p};
     }
     return DiagOut{rvort_v.p, inv_thick_v.p, ke_c.p, div_c.p, trdel2_c.p,
-                   vdel2_e.p, vdel2_rv_v.p, vdel2_div_c.p};
+                   vdel2_e.p, vdel2_rv_v.p, vdel2_div_c.p, vdel4_e.p};
   }
 };
 
 // A captured step is valid only for the exact device buffers and model
-// configuration it recorded: the key holds dt, the buffer parity, the
+// configuration it recorded: the key holds dt, the buffer parity, whether
+// the step leaves its last stage's diagnostics, the
 // model's configuration generation and every buffer address the step
 // touches, so a reallocated buffer or a changed setting never replays a
 // stale graph.
 struct GraphKey {
   double dt;
   int cur;
+  bool emit;
   uint64_t gen;
   std::vector<const void *> bufs;
   bool operator<(const GraphKey &o) const {
     if (dt != o.dt) return dt < o.dt;
     if (cur != o.cur) return cur < o.cur;
+    if (emit != o.emit) return emit < o.emit;
     if (gen != o.gen) return gen < o.gen;
     return bufs < o.bufs;
   }
@@ -205,7 +213,8 @@ void run_diag(omega_model_s *M, const Real *h, const Real *vn, const Real *tr, h
 // pre: also write the tendency VJP's rows at the stage input (only where
 // stage_writes_pre says the model's stage kernel can)
 void run_stage(omega_model_s *M, StageArgs a, hipStream_t s, int fields = 7,
-               bool with_diag = true, const omega_hip::PreOut *pre = nullptr);
+               bool with_diag = true, const omega_hip::PreOut *pre = nullptr,
+               bool emit = true);
 bool stage_writes_pre(omega_model_s *M);
 // true when the model's terms need the general kernels (bottom drag)
 bool general_only(const omega_model_s *M);
@@ -230,8 +239,9 @@ void compute_tendency_ptrs(omega_model_s *M, Real *ht, Real *vt, Real *tt, const
 // RK4 tableau (rk4.cpp:14-25) or the low-storage coefficients (lsrk.cpp:16-33)
 void stepper_coefficients(int kind, int nstages, std::vector<Real> &rka, std::vector<Real> &rkb,
                           std::vector<Real> &rkc);
-void step_once(omega_stepper_s *St, omega_state_s *S, double t, double dt, hipStream_t s);
+void step_once(omega_stepper_s *St, omega_state_s *S, double t, double dt, hipStream_t s,
+               bool emit = true);
 void do_step_maybe_graph(omega_stepper_s *St, omega_state_s *S, double t, double dt,
-                         hipStream_t s);
+                         hipStream_t s, bool emit = true);
 
 } // namespace omega_hip

@@ -9,6 +9,15 @@
 
 namespace omega_hip {
 
+// The stage kernels (kernels_stage.hip) take models whose every coefficient is one
+// value per stencil slot and sign (the mesh's by build_hex_stage, the model's
+// here) and whose momentum has its three basic terms and both tendencies on.
+bool stage_terms(const omega_model_s *M) {
+  constexpr int basic = T_PV | T_KE | T_SSH;
+  return (M->terms & basic) == basic && !(M->terms & T_DRAG) &&
+         !M->params.disable_h_tendency && !M->params.disable_vn_tendency;
+}
+
 void model_build_coefficients(omega_model_s *M) {
   const DeviceMesh &dm = M->mesh->dm;
   const HostMesh &hm = dm.host;
@@ -45,6 +54,7 @@ void model_build_coefficients(omega_model_s *M) {
   M->ct4_h = ct4;
   M->ct4.upload(ct4);
   M->f_uniform = rows_equal(f, 1);
+  M->f_value = M->params.f0;
   M->mix_uniform = rows_equal(cv2, 1) && rows_equal(cv4, 1) && rows_equal(ct2, ME) &&
                    rows_equal(ct4, ME);
   M->rvort_v.alloc((size_t)NV * L);
@@ -84,6 +94,7 @@ void ensure_vdel4(omega_model_s *M) {
     M->vdel2_rv_v.alloc((size_t)hm.nvertices * L);
     M->vdel2_div_c.alloc((size_t)hm.ncells * L);
   }
+  if (M->mesh->dm.stage_ok && !M->vdel4_e.p) M->vdel4_e.alloc((size_t)hm.nedges * L);
 }
 
 hipStream_t capture_stream() {
@@ -152,7 +163,13 @@ void run_stage_into(omega_model_s *M, StageArgs a, hipStream_t s, int fields,
     return;
   }
   if (dx) {
-    // caller-provided diagnostics buffers
+    // caller-provided diagnostics buffers; without momentum del4 the stage
+    // kernels need none
+    HexCoef q;
+    if (fields == 7 && !(M->terms & T_VDEL4) && M->stage_coef(q)) {
+      launch_stage_hex(mv, M->lc, q, a, *dx, false, s);
+      return;
+    }
     run_diag_into(M, a.h.in, a.vn.in, a.tr.in, *dx, s);
     if (hex_usable(mv, M->lc) && !general_only(M)) launch_tend_hex(mv, M->lc, mc, a, *dx, s);
     else launch_tend(mv, M->lc, mc, a, *dx, s);
@@ -172,7 +189,7 @@ bool stage_writes_pre(omega_model_s *M) {
 }
 
 void run_stage(omega_model_s *M, StageArgs a, hipStream_t s, int fields, bool with_diag,
-               const PreOut *pre) {
+               const PreOut *pre, bool emit) {
   const MeshView mv = M->view();
   const ModelCoef mc = M->coef();
   a.terms = M->terms;
@@ -181,6 +198,15 @@ void run_stage(omega_model_s *M, StageArgs a, hipStream_t s, int fields, bool wi
   a.ntr = (fields & 4) ? M->params.ntracers : 0;
   if (M->linear) {
     launch_tend_linear(mv, M->lc, M->lin_coef(), a, s);
+    return;
+  }
+  HexCoef q;
+  if (with_diag && !pre && fields == 7 && M->stage_coef(q)) {
+    M->aux_h = a.h.in;
+    M->aux_vn = a.vn.in;
+    M->aux_tr = a.tr.in;
+    if (M->terms & T_VDEL4) ensure_vdel4(M);
+    launch_stage_hex(mv, M->lc, q, a, M->diag(), emit, s);
     return;
   }
   if (with_diag) run_diag(M, a.h.in, a.vn.in, a.tr.in, s);
@@ -269,7 +295,7 @@ void stepper_coefficients(int kind, int nstages, std::vector<Real> &rka, std::ve
 
 // RK4 with a fused tendency + update per stage (rk4.cpp:28-104 reorganised:
 // the accumulator lives in acc until the last stage writes the state).
-void rk4_fused_step(omega_stepper_s *St, omega_state_s *S, double dt, hipStream_t s) {
+void rk4_fused_step(omega_stepper_s *St, omega_state_s *S, double dt, hipStream_t s, bool emit) {
   omega_model_s *M = St->model;
   ensure3(St->acc, S);
   ensure3(St->p1, S);
@@ -289,7 +315,7 @@ void rk4_fused_step(omega_stepper_s *St, omega_state_s *S, double dt, hipStream_
     a.h = fio(in[0], nullptr, A[0], Y[0], out[0]);
     a.vn = fio(in[1], nullptr, A[1], Y[1], out[1]);
     a.tr = fio(in[2], nullptr, A[2], Y[2], out[2]);
-    run_stage(M, a, s);
+    run_stage(M, a, s, 7, true, nullptr, emit && stage == 3);
   }
 }
 
@@ -333,7 +359,7 @@ void carry_extra_tracers(omega_model_s *M, omega_state_s *S, hipStream_t s) {
 
 // Low-storage RK with the state alternating between two buffers per stage
 // (lsrk.cpp:36-89 fused: tend = a*tend + F(y); y' = y + dt*b*tend).
-void lsrk_fused_step(omega_stepper_s *St, omega_state_s *S, double dt, hipStream_t s) {
+void lsrk_fused_step(omega_stepper_s *St, omega_state_s *S, double dt, hipStream_t s, bool emit) {
   omega_model_s *M = St->model;
   ensure3(St->tend, S);
   carry_extra_tracers(M, S, s);
@@ -348,7 +374,7 @@ void lsrk_fused_step(omega_stepper_s *St, omega_state_s *S, double dt, hipStream
     a.h = fio(in[0], St->tend[0].p, nullptr, nullptr, out[0]);
     a.vn = fio(in[1], St->tend[1].p, nullptr, nullptr, out[1]);
     a.tr = fio(in[2], St->tend[2].p, nullptr, nullptr, out[2]);
-    run_stage(M, a, s);
+    run_stage(M, a, s, 7, true, nullptr, emit && stage + 1 == St->nstages);
     S->cur = 1 - S->cur;
   }
 }
@@ -367,22 +393,25 @@ void lsrk_unfused_step(omega_stepper_s *St, omega_state_s *S, double t, double d
   }
 }
 
-void step_once(omega_stepper_s *St, omega_state_s *S, double t, double dt, hipStream_t s) {
+// emit: leave the last stage's diagnostics in the model's buffers, where the
+// auxiliary-state calls read them
+void step_once(omega_stepper_s *St, omega_state_s *S, double t, double dt, hipStream_t s,
+               bool emit) {
   const bool fused = St->model->add_fn == nullptr;
   if (St->kind == OMEGA_STEPPER_RK4) {
-    if (fused) rk4_fused_step(St, S, dt, s);
+    if (fused) rk4_fused_step(St, S, dt, s, emit);
     else rk4_unfused_step(St, S, t, dt, s);
   } else {
-    if (fused) lsrk_fused_step(St, S, dt, s);
+    if (fused) lsrk_fused_step(St, S, dt, s, emit);
     else lsrk_unfused_step(St, S, t, dt, s);
   }
 }
 
 void do_step_maybe_graph(omega_stepper_s *St, omega_state_s *S, double t, double dt,
-                         hipStream_t s) {
+                         hipStream_t s, bool emit) {
   const bool graphable = St->use_graph && St->model->add_fn == nullptr && !stream_capturing(s);
   if (!graphable) {
-    step_once(St, S, t, dt, s);
+    step_once(St, S, t, dt, s, emit);
     return;
   }
   if (St->kind == OMEGA_STEPPER_LSRK) {
@@ -399,14 +428,14 @@ void do_step_maybe_graph(omega_stepper_s *St, omega_state_s *S, double t, double
   }
   omega_model_s *M = St->model;
   if (M->terms & T_VDEL4) ensure_vdel4(M);
-  GraphKey key{dt, S->cur, M->gen, {}};
+  GraphKey key{dt, S->cur, emit, M->gen, {}};
   for (int f = 0; f < 3; ++f)
     key.bufs.insert(key.bufs.end(), {S->buf[0][f].p, S->buf[1][f].p, St->acc[f].p,
                                      St->p1[f].p, St->p2[f].p, St->tend[f].p});
   key.bufs.insert(key.bufs.end(), {M->vdel2_e.p, M->trdel2_c.p, M->f_v.p});
   const DiagOut dk = M->diag();
   key.bufs.insert(key.bufs.end(), {dk.rvort_v, dk.inv_thick_v, dk.ke_c, dk.div_c, dk.trdel2_c,
-                                   dk.vdel2_e, dk.vdel2_rv_v, dk.vdel2_div_c});
+                                   dk.vdel2_e, dk.vdel2_rv_v, dk.vdel2_div_c, dk.vdel4_e});
   auto it = St->graphs.find(key);
   if (it == St->graphs.end()) {
     // bound the cache: states created and destroyed in a loop (the adjoint's
@@ -419,7 +448,7 @@ void do_step_maybe_graph(omega_stepper_s *St, omega_state_s *S, double t, double
     hipGraph_t g;
     OMEGA_HIP_CHECK(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
     try {
-      step_once(St, S, t, dt, cs);
+      step_once(St, S, t, dt, cs, emit);
     } catch (...) {
       hipGraph_t dummy;
       (void)hipStreamEndCapture(cs, &dummy);
@@ -437,5 +466,24 @@ void do_step_maybe_graph(omega_stepper_s *St, omega_state_s *S, double t, double
   if (St->kind == OMEGA_STEPPER_LSRK && (St->nstages % 2 == 1)) S->cur = 1 - S->cur;
 }
 
-
 } // namespace omega_hip
+
+bool omega_model_s::stage_coef(omega_hip::HexCoef &q) const {
+  using namespace omega_hip;
+  const DeviceMesh &dm = mesh->dm;
+  if (!dm.stage_ok || linear || (forms & 7) != 7 || lc.variant != 0 || !f_uniform ||
+      !mix_uniform || !stage_terms(this))
+    return false;
+  q = dm.stage_coef;
+  // ct2, ct4: one magnitude, negative at the cell's first three sides
+  const double c2 = ct2_h[3], c4 = ct4_h[3];
+  for (int j = 0; j < 6; ++j)
+    if (ct2_h[j] != (j < 3 ? -c2 : c2) || ct4_h[j] != (j < 3 ? -c4 : c4)) return false;
+  q.f = f_value;
+  q.grav = params.grav;
+  q.cv2 = params.visc_del2 * dm.s2_h[0];
+  q.cv4 = params.visc_del4 * dm.s4_h[0];
+  q.ct2 = c2 / 2;
+  q.ct4 = c4;
+  return true;
+}

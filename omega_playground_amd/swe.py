@@ -572,12 +572,16 @@ class ShallowWaterModel:
     def set_kernel_forms(self, forms: int = 15):
         """Allow (bits set) or forbid the shared-coefficient (bit 0),
         32-bit-offset (bit 1) and compiled-in term-set (bit 2) forms of the
-        pair kernels, and a step adjoint's stage recomputation writing the
+        pair kernels (the stage kernels without stored diagnostics need all
+        three), and a step adjoint's stage recomputation writing the
         rows its tendency VJPs linearise about (bit 3)."""
         check(lib().omega_model_set_kernel_forms(self._h, int(forms)))
 
     def kernel_variant(self) -> int:
-        """6 linear model, 2 pattern-specialised, 1 general kernels."""
+        """6 linear model, 2 pattern-specialised, 1 general kernels: the family
+        of the kernels with stored diagnostics for this layer count (forward
+        stages of a regular mesh with uniform coefficients store none, at any
+        layer count)."""
         v = C.c_int()
         check(lib().omega_model_kernel_variant(self._h, C.byref(v)))
         return v.value
