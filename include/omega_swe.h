@@ -486,7 +486,10 @@ int omega_batch_set_graph(omega_batch_t batch, int enable);
  * and levels per lane (1 or 2).  Each stage phase (diagnostics, momentum
  * del4 pre-pass, tendency + update) is one launch over every member; members
  * on the regular hexagonal mesh run the pattern-specialised operators and
- * the others the general ones inside it. */
+ * the others the general ones inside it.  Members whose models take the stage
+ * kernels without stored diagnostics (regular mesh, uniform coefficients, no
+ * momentum del4) have launches of their own, one for momentum and one for
+ * tracers per set of terms, with the shape their models' launches have. */
 int omega_batch_set_launch(omega_batch_t batch, int threads, int levels_per_thread);
 int omega_batch_get_launch(omega_batch_t batch, int *threads, int *levels_per_thread);
 /* Persistent grid: 0 (default) launches one block per table entry (a

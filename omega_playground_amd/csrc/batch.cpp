@@ -1,6 +1,9 @@
 // Ensembles (no reference counterpart): independent members -- each its own
 // mesh, layer count, tracer count, coefficients and time step -- advanced
-// together.  Every stage phase (diagnostics, momentum del4 pre-pass,
+// together.  Members on the stage kernels without stored diagnostics
+// (kernels_stage.hip) have one momentum and one tracer launch per stage and
+// set of terms (16 mixed members, 64 layers at most, LSRK5: 2.05 -> 1.23 ms
+// per step against the launches below).  For the others every stage phase (diagnostics, momentum del4 pre-pass,
 // tendency + update) is one launch over all members' blocks, driven by a
 // table of per-member descriptors built once per (step parity, stage); the
 // step can be captured in a HIP graph.  The stage updates are the fused
@@ -14,6 +17,7 @@
 
 #include "batch.hpp"
 #include "objects.hpp"
+#include "stage_launch.hpp"
 
 using namespace omega_hip;
 
@@ -37,12 +41,24 @@ struct omega_batch_s {
   bool built = false;
   int parity = 0;
   // one table over all members; member kinds share each launch
-  int nblocks = 0;
+  int nblocks = 0; // entries of a stage's first launches, ntable in the table
+  int ntable = 0;
   int kinds = 0; // bit 0 general-kernel members, bit 1 pattern-specialised
   int tset = 0;  // term set compiled into the pair tendency launch (0: none)
   bool any_vdel4 = false;
   DBuf<int> blk;
   DBuf<BatchMember> desc; // [parity][stage][member]
+  // members on the stage kernels without stored diagnostics, by what their
+  // launches have compiled in; the tables above hold the others
+  struct Group {
+    StageKind kind;
+    std::vector<int> members;
+    int nmom = 0, ntile = 0;     // entries of the two launches
+    DBuf<int> wmom, wtile;       // member (of the group) of each entry
+    DBuf<StageLaunch> mom;       // [parity][stage][member]
+    DBuf<TileLaunch> tile;
+  };
+  std::vector<std::unique_ptr<Group>> groups;
   bool use_graph = false;
   std::map<int, hipGraphExec_t> graphs;
 
@@ -79,6 +95,9 @@ void build_tables(omega_batch_s *B) {
   const int nm = (int)B->mem.size(), ns = B->nstages, N = B->N, T = B->threads;
   std::vector<int> blk;
   std::vector<BatchMember> geo(nm);
+  std::vector<int> own(nm, -1); // group of a member on the stage kernels
+  std::vector<HexCoef> coef(nm);
+  B->groups.clear();
   B->any_vdel4 = false;
   for (int i = 0; i < nm; ++i) {
     auto &mb = *B->mem[i];
@@ -96,6 +115,22 @@ void build_tables(omega_batch_s *B) {
       ensure3(mb.p2, S);
     } else {
       ensure3(mb.tend, S);
+    }
+    mb.cur0 = S->cur;
+    mb.gen = M->gen;
+    if (!(M->terms & T_VDEL4) && M->stage_coef(coef[i])) {
+      const MeshView mv = M->view();
+      const StageKind k{stage_levels(mv, M->lc), mv.tile.lx, (M->terms & T_VDEL2) != 0,
+                        (M->terms & T_TDEL2) != 0, (M->terms & T_TDEL4) != 0};
+      size_t j = 0;
+      while (j < B->groups.size() && !(B->groups[j]->kind == k)) ++j;
+      if (j == B->groups.size()) {
+        B->groups.push_back(std::make_unique<omega_batch_s::Group>());
+        B->groups[j]->kind = k;
+      }
+      B->groups[j]->members.push_back(i);
+      own[i] = (int)j;
+      continue;
     }
     BatchMember &g = geo[i];
     // 16 or 32 layers run the pattern kernels with several cells per
@@ -130,12 +165,11 @@ void build_tables(omega_batch_s *B) {
     g.dterms = need_diag ? (do_vn ? M->terms : (M->terms & T_TDEL4)) : 0;
     g.vdel4 = do_vn && (M->terms & T_VDEL4);
     B->any_vdel4 = B->any_vdel4 || g.vdel4;
-    mb.cur0 = S->cur;
-    mb.gen = M->gen;
   }
-  B->nblocks = (int)blk.size();
+  B->nblocks = B->ntable = (int)blk.size();
   B->kinds = 0;
-  for (const BatchMember &g : geo) B->kinds |= g.hex ? 2 : 1;
+  for (int i = 0; i < nm; ++i)
+    if (own[i] < 0) B->kinds |= geo[i].hex ? 2 : 1;
   // the members' term set, compiled into the tendency launch when they all
   // share it (the 64k-layer members' pair operators also need the
   // shared-coefficient, 32-bit-offset forms and the vertex-union records)
@@ -144,6 +178,7 @@ void build_tables(omega_batch_s *B) {
     int ts = 0;
     bool ok = true;
     for (int i = 0; i < nm && ok; ++i) {
+      if (own[i] >= 0) continue;
       omega_model_s *M = B->mem[i]->M;
       const MeshView v = M->view();
       const ModelCoef c = M->coef();
@@ -154,6 +189,20 @@ void build_tables(omega_batch_s *B) {
       ts = M->terms;
     }
     if (ok) B->tset = ts;
+  }
+  // entries of the groups' launches
+  struct Tables {
+    std::vector<StageLaunch> mom;
+    std::vector<TileLaunch> tile;
+    std::vector<int> wmom, wtile;
+  };
+  std::vector<Tables> gt(B->groups.size());
+  std::vector<int> place(nm, 0);
+  for (size_t j = 0; j < gt.size(); ++j) {
+    const std::vector<int> &mem = B->groups[j]->members;
+    gt[j].mom.resize((size_t)2 * ns * mem.size());
+    gt[j].tile.resize((size_t)2 * ns * mem.size());
+    for (size_t q = 0; q < mem.size(); ++q) place[mem[q]] = (int)q;
   }
   std::vector<BatchMember> tab((size_t)2 * ns * nm);
   for (int p = 0; p < 2; ++p)
@@ -209,9 +258,36 @@ void build_tables(omega_batch_s *B) {
           a.vn = fio(in[1], mb.tend[1].p, nullptr, nullptr, out[1]);
           a.tr = fio(in[2], mb.tend[2].p, nullptr, nullptr, out[2]);
         }
+        if (own[i] >= 0) {
+          Tables &T = gt[own[i]];
+          const size_t ng = B->groups[own[i]]->members.size();
+          const size_t at = ((size_t)p * ns + s) * ng + place[i];
+          stage_launch(g.m, M->lc, B->groups[own[i]]->kind.N, coef[i], a, g.d, T.mom[at], T.tile[at]);
+          // the first table's entries give every table's numbering
+          if (p == 0 && s == 0) {
+            T.mom[at].block0 = (int)T.wmom.size();
+            T.tile[at].block0 = (int)T.wtile.size();
+            T.wmom.insert(T.wmom.end(), T.mom[at].tiles, place[i]);
+            T.wtile.insert(T.wtile.end(), T.tile[at].work, place[i]);
+          } else {
+            T.mom[at].block0 = T.mom[place[i]].block0;
+            T.tile[at].block0 = T.tile[place[i]].block0;
+          }
+          continue;
+        }
         g.a = a;
         tab[((size_t)p * ns + s) * nm + i] = g;
       }
+  for (size_t j = 0; j < gt.size(); ++j) {
+    omega_batch_s::Group &G = *B->groups[j];
+    G.nmom = (int)gt[j].wmom.size();
+    G.ntile = (int)gt[j].wtile.size();
+    G.wmom.upload(gt[j].wmom);
+    G.wtile.upload(gt[j].wtile);
+    G.mom.upload(gt[j].mom);
+    G.tile.upload(gt[j].tile);
+    B->nblocks += G.nmom;
+  }
   B->blk.upload(blk);
   if (B->desc.n != tab.size()) B->desc.alloc(tab.size());
   OMEGA_HIP_CHECK(hipMemcpy(B->desc.p, tab.data(), tab.size() * sizeof(BatchMember),
@@ -252,7 +328,16 @@ void step_launches(omega_batch_s *B, int parity, hipStream_t s) {
   for (int st = 0; st < B->nstages; ++st) {
     const BatchMember *d = B->desc.p + ((size_t)parity * B->nstages + st) * nm;
     const int *g = B->blk.p;
-    const int n = B->nblocks;
+    const int n = B->ntable;
+    for (auto &gp : B->groups) {
+      // the last stage leaves its input's diagnostics in the models' buffers
+      const omega_batch_s::Group &G = *gp;
+      const size_t at = ((size_t)parity * B->nstages + st) * G.members.size();
+      const bool emit = st + 1 == B->nstages;
+      launch_stage_batch(G.kind, G.mom.p + at, G.wmom.p, G.nmom, emit, s);
+      if (G.ntile) launch_tile_batch(G.kind, G.tile.p + at, G.wtile.p, G.ntile, emit, s);
+    }
+    if (!n) continue;
     launch_batch_diag(d, g, n, B->threads, B->N, pers, B->kinds, s);
     if (B->any_vdel4) launch_batch_vdel4(d, g, n, B->threads, B->N, pers, s);
     launch_batch_tend(d, g, n, B->threads, B->N, pers, B->kinds, B->tset, s);

@@ -11,6 +11,7 @@
 #include <algorithm>
 
 #include "hex_stage.hpp"
+#include "stage_launch.hpp"
 
 namespace omega_hip {
 
@@ -18,27 +19,20 @@ namespace {
 
 using namespace stage;
 
-struct StageLaunch {
-  HexCoef q;
-  const int *rec;
-  int nc, L, ncb, tiles, per_xcd;
-  StageArgs a;
-  DiagOut d;
-  const double *x; // k_stage_lap: the edge field, its result
-  double *y;
-};
+// Entry b of n for this block: workgroups are dealt to the 8 XCDs
+// round-robin, and each XCD takes a contiguous range of entries, so that
+// neighbouring cells' rows are re-read from one L2.
+__device__ __forceinline__ int xcd_entry(int n) { return logical_block((int)blockIdx.x, n, 1); }
 
-// Block b runs on XCD b mod 8 (workgroups are dealt round-robin) and takes
-// that XCD's contiguous range of (level chunk, cell block) pairs, so that
-// neighbouring cells' rows are re-read from one L2.  False: no work here.
-__device__ __forceinline__ bool stage_place(const StageLaunch &p, int N, int &c, Ctx &x) {
-  const int tile = ((int)blockIdx.x & 7) * p.per_xcd + ((int)blockIdx.x >> 3);
-  if (tile >= p.tiles) return false;
-  const int ch = p.tiles == p.ncb ? 0 : uniform(tile / p.ncb);
-  c = (tile - ch * p.ncb) * (int)blockDim.y + (int)threadIdx.y;
-  const int k = (ch * (int)blockDim.x + (int)threadIdx.x) * N;
+// The cell and levels of this thread at an entry (level chunk, cell block);
+// false: no work here.
+__device__ __forceinline__ bool stage_place(const StageLaunch &p, int entry, int N, int &c, Ctx &x) {
+  const int ch = p.tiles == p.ncb ? 0 : uniform(entry / p.ncb);
+  const int row = (int)threadIdx.x / p.lx, ln = (int)threadIdx.x - row * p.lx;
+  c = (entry - ch * p.ncb) * p.rows + row;
+  const int k = (ch * p.lx + ln) * N;
   x = Ctx{p.L, (unsigned)p.L * 8u, (unsigned)k * 8u, k};
-  return c < p.nc && k < p.L;
+  return row < p.rows && c < p.nc && k < p.L;
 }
 
 // Momentum and thickness.  Two levels per lane at two waves per SIMD (228
@@ -47,11 +41,10 @@ __device__ __forceinline__ bool stage_place(const StageLaunch &p, int N, int &c,
 // same rows in twice the load instructions).
 // V4: subtract the del4 rows (p.x) the Laplacian launches left.
 template <int N, bool V2, bool V4, bool EMIT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N == 1 ? 4 : 2)))
-    k_stage_mom(StageLaunch p) {
+__device__ __forceinline__ void stage_mom(const StageLaunch &p, int entry) {
   int c;
   Ctx x;
-  if (!stage_place(p, N, c, x)) return;
+  if (!stage_place(p, entry, N, c, x)) return;
   const StageArgs &a = p.a;
   const int L = x.L, k = x.k;
   int id[hl::kCells];
@@ -92,13 +85,29 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N == 1
   epilogue<N>(a, a.h, idx, T);
 }
 
+template <int N, bool V2, bool V4, bool EMIT>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N == 1 ? 4 : 2)))
+    k_stage_mom(StageLaunch p) {
+  stage_mom<N, V2, V4, EMIT>(p, xcd_entry(p.tiles));
+}
+
+// Ensemble forms: entry b of n belongs to member who[b], whose parameter
+// block is read in place through scalar loads.
+template <int N, bool V2, bool EMIT>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N == 1 ? 4 : 2)))
+    k_batch_mom(const StageLaunch *__restrict__ desc, const int *__restrict__ who, int n) {
+  const int b = xcd_entry(n);
+  const StageLaunch &p = desc[uniform(who[b])];
+  stage_mom<N, V2, false, EMIT>(p, b - p.block0);
+}
+
 // The edge Laplacian: of the velocity (FINAL false), then of that result,
 // with the masked coefficient applied (FINAL).
 template <int N, bool FINAL, bool EMIT>
 __global__ void __launch_bounds__(256) k_stage_lap(StageLaunch p) {
   int c;
   Ctx x;
-  if (!stage_place(p, N, c, x)) return;
+  if (!stage_place(p, xcd_entry(p.tiles), N, c, x)) return;
   int id[hl::kCells];
   load_cells(p.rec, c, id);
   LapOut<N> o;
@@ -133,17 +142,8 @@ __global__ void __launch_bounds__(256) k_stage_lap(StageLaunch p) {
 // faster than 128-byte ones (6.3 against 7.2 ms per step), three waves per
 // SIMD faster than four with 13 registers spilled (6.3 against 7.0).
 // ---------------------------------------------------------------------------
-struct TileLaunch {
-  HexCoef q;
-  const int *ids; // [tiles][(TH + 4)(TW + 4)] cell at each place, row-major
-  int nx, ny, tiles_x, nch, work, per_xcd, nc, L, per_block;
-  StageArgs a;
-  DiagOut d;
-};
-
 template <int N, int LX, int TW, int TH, bool D2, bool D4, bool EMIT>
-__global__ void __launch_bounds__(LX *TW *TH) __attribute__((amdgpu_waves_per_eu(N == 2 ? 3 : 4)))
-    k_stage_tile(TileLaunch p) {
+__device__ __forceinline__ void stage_tile(const TileLaunch &p, int w) {
   constexpr int HALO = D4 ? 2 : 1, PW = TW + 2 * HALO, PH = TH + 2 * HALO, NP = PW * PH;
   constexpr int CELLS = TW * TH, R = (NP + CELLS - 1) / CELLS;
   constexpr int RING = 2 * (TW + 2) + 2 * TH; // the first ring round the tile
@@ -151,8 +151,6 @@ __global__ void __launch_bounds__(LX *TW *TH) __attribute__((amdgpu_waves_per_eu
   constexpr int S = LX * N, PLANE = NP * S; // doubles per place and per array
   __shared__ double Hs[PLANE], Ns[PLANE], Ds[D4 ? PLANE : 1];
   __shared__ int ids[NP];
-  const int w = ((int)blockIdx.x & 7) * p.per_xcd + ((int)blockIdx.x >> 3);
-  if (w >= p.work) return;
   const int tile = uniform(w / p.nch), ch = w - tile * p.nch;
   const int ln = (int)threadIdx.x % LX, row = (int)threadIdx.x / LX;
   const int L = p.L, k = (ch * LX + ln) * N;
@@ -322,8 +320,21 @@ __global__ void __launch_bounds__(LX *TW *TH) __attribute__((amdgpu_waves_per_eu
   }
 }
 
+template <int N, int LX, int TW, int TH, bool D2, bool D4, bool EMIT>
+__global__ void __launch_bounds__(LX *TW *TH) __attribute__((amdgpu_waves_per_eu(N == 2 ? 3 : 4)))
+    k_stage_tile(TileLaunch p) {
+  stage_tile<N, LX, TW, TH, D2, D4, EMIT>(p, xcd_entry(p.work));
+}
+
+template <int N, int LX, int TW, int TH, bool D2, bool D4, bool EMIT>
+__global__ void __launch_bounds__(LX *TW *TH) __attribute__((amdgpu_waves_per_eu(N == 2 ? 3 : 4)))
+    k_batch_tile(const TileLaunch *__restrict__ desc, const int *__restrict__ who, int n) {
+  const int b = xcd_entry(n);
+  const TileLaunch &p = desc[uniform(who[b])];
+  stage_tile<N, LX, TW, TH, D2, D4, EMIT>(p, b - p.block0);
+}
+
 using StageFn = void (*)(StageLaunch);
-using TileFn = void (*)(TileLaunch);
 
 template <int N, bool EMIT> StageFn pick_mom(bool v2, bool v4) {
   if (v4) return v2 ? k_stage_mom<N, true, true, EMIT> : k_stage_mom<N, false, true, EMIT>;
@@ -331,43 +342,88 @@ template <int N, bool EMIT> StageFn pick_mom(bool v2, bool v4) {
 }
 
 // without del4 there is no Laplacian to emit
-template <int N, int LX, int TW, int TH, bool EMIT> TileFn pick_shape(bool d2, bool d4) {
-  if (d4)
-    return d2 ? k_stage_tile<N, LX, TW, TH, true, true, EMIT>
-              : k_stage_tile<N, LX, TW, TH, false, true, EMIT>;
-  return d2 ? k_stage_tile<N, LX, TW, TH, true, false, false>
-            : k_stage_tile<N, LX, TW, TH, false, false, false>;
+template <int N, int LX, int TW, int TH, bool EMIT, bool BATCH> auto pick_shape(bool d2, bool d4) {
+  if constexpr (BATCH) {
+    if (d4)
+      return d2 ? k_batch_tile<N, LX, TW, TH, true, true, EMIT>
+                : k_batch_tile<N, LX, TW, TH, false, true, EMIT>;
+    return d2 ? k_batch_tile<N, LX, TW, TH, true, false, false>
+              : k_batch_tile<N, LX, TW, TH, false, false, false>;
+  } else {
+    if (d4)
+      return d2 ? k_stage_tile<N, LX, TW, TH, true, true, EMIT>
+                : k_stage_tile<N, LX, TW, TH, false, true, EMIT>;
+    return d2 ? k_stage_tile<N, LX, TW, TH, true, false, false>
+              : k_stage_tile<N, LX, TW, TH, false, false, false>;
+  }
 }
-template <int N, bool EMIT> TileFn pick_tile(const TileView &t, bool d2, bool d4) {
-  if (t.lx == 4) return pick_shape<N, 4, 8, 8, EMIT>(d2, d4);
-  if (t.lx == 2) return pick_shape<N, 2, 16, 8, EMIT>(d2, d4);
-  return pick_shape<N, 1, 16, 16, EMIT>(d2, d4);
+template <bool BATCH, int N, bool EMIT> auto pick_tile_of(int lx, bool d2, bool d4) {
+  if (lx == 4) return pick_shape<N, 4, 8, 8, EMIT, BATCH>(d2, d4);
+  if (lx == 2) return pick_shape<N, 2, 16, 8, EMIT, BATCH>(d2, d4);
+  return pick_shape<N, 1, 16, 16, EMIT, BATCH>(d2, d4);
 }
+template <bool BATCH> auto pick_tile(int N, int lx, bool d2, bool d4, bool emit) {
+  if (N == 2) return emit ? pick_tile_of<BATCH, 2, true>(lx, d2, d4) : pick_tile_of<BATCH, 2, false>(lx, d2, d4);
+  return emit ? pick_tile_of<BATCH, 1, true>(lx, d2, d4) : pick_tile_of<BATCH, 1, false>(lx, d2, d4);
+}
+
+template <int N> auto pick_batch_mom(bool v2, bool emit) {
+  if (emit) return v2 ? k_batch_mom<N, true, true> : k_batch_mom<N, false, true>;
+  return v2 ? k_batch_mom<N, true, false> : k_batch_mom<N, false, false>;
+}
+
+constexpr int kTileThreads = 256; // every tile shape's
 
 } // namespace
 
-void launch_stage_hex(const MeshView &m, const Launch &lc, const HexCoef &q, const StageArgs &a,
-                      const DiagOut &d, bool emit, hipStream_t s) {
-  TimerScope ts("tend", s);
-  const int N = lc.lpt == 2 && m.L % 2 == 0 ? 2 : 1;
+int stage_levels(const MeshView &m, const Launch &lc) {
+  return lc.lpt == 2 && m.L % 2 == 0 ? 2 : 1;
+}
+
+void stage_launch(const MeshView &m, const Launch &lc, int N, const HexCoef &q, const StageArgs &a,
+                  const DiagOut &d, StageLaunch &p, TileLaunch &t) {
   const int lanes = (m.L + N - 1) / N;
-  // cells' lanes per block: up to 16 (32 levels), so that a block's cells
+  // lanes per cell and block: up to 16 (32 levels), so that a block's cells
   // share more of their neighbours' rows in L1 (2.81 against 2.85 ms per step
   // for momentum alone at nx=512, 64 layers with 32, 2.94 with 8)
   const int want = lc.chunk > 0 ? std::min(std::max(1, lc.chunk / N), 64) : 16;
-  const int nch = (lanes + want - 1) / want, lx = (lanes + nch - 1) / nch;
-  const int rows = lc.rows > 0 ? std::min(lc.rows, 256 / lx) : 256 / lx;
-  StageLaunch p{};
+  const int nch = (lanes + want - 1) / want;
+  p = StageLaunch{};
   p.q = q;
   p.rec = m.hexc;
   p.nc = m.nc;
   p.L = m.L;
-  p.ncb = (m.nc + rows - 1) / rows;
+  p.lx = (lanes + nch - 1) / nch;
+  p.rows = lc.rows > 0 ? std::min(lc.rows, 256 / p.lx) : 256 / p.lx;
+  p.ncb = (m.nc + p.rows - 1) / p.rows;
   p.tiles = p.ncb * nch;
-  p.per_xcd = (p.tiles + 7) / 8;
   p.a = a;
   p.d = d;
-  const dim3 grid(8 * p.per_xcd), block(lx, rows);
+  t = TileLaunch{};
+  if (a.ntr <= 0) return;
+  const TileView &tv = m.tile;
+  t.q = q;
+  t.ids = tv.ids;
+  t.nx = tv.nx;
+  t.ny = tv.ny;
+  t.tiles_x = (tv.nx + tv.tw - 1) / tv.tw;
+  t.nch = (lanes + tv.lx - 1) / tv.lx;
+  t.work = t.tiles_x * ((tv.ny + tv.th - 1) / tv.th) * t.nch;
+  t.nc = m.nc;
+  t.L = m.L;
+  t.per_block = a.ntr;
+  t.a = a;
+  t.d = d;
+}
+
+void launch_stage_hex(const MeshView &m, const Launch &lc, const HexCoef &q, const StageArgs &a,
+                      const DiagOut &d, bool emit, hipStream_t s) {
+  TimerScope ts("tend", s);
+  const int N = stage_levels(m, lc);
+  StageLaunch p;
+  TileLaunch t;
+  stage_launch(m, lc, N, q, a, d, p, t);
+  const dim3 grid(p.tiles), block(p.lx * p.rows);
   const bool v4 = a.terms & T_VDEL4;
   if (v4) {
     p.x = a.vn.in;
@@ -386,29 +442,31 @@ void launch_stage_hex(const MeshView &m, const Launch &lc, const HexCoef &q, con
                            : (emit ? pick_mom<1, true>(v2, v4) : pick_mom<1, false>(v2, v4));
   hipLaunchKernelGGL(k, grid, block, 0, s, p);
   if (a.ntr > 0) {
-    const TileView &tv = m.tile;
-    TileLaunch t{};
-    t.q = q;
-    t.ids = tv.ids;
-    t.nx = tv.nx;
-    t.ny = tv.ny;
-    t.tiles_x = (tv.nx + tv.tw - 1) / tv.tw;
-    t.nch = (lanes + tv.lx - 1) / tv.lx;
-    t.work = t.tiles_x * ((tv.ny + tv.th - 1) / tv.th) * t.nch;
-    t.per_xcd = (t.work + 7) / 8;
-    t.nc = m.nc;
-    t.L = m.L;
     // one block takes all tracers of its tile, keeping the tile's thicknesses
-    // and velocities; where the tiles alone leave the chip short of blocks
-    // (fewer than 512) each tracer has its own
-    t.per_block = t.work >= 512 ? a.ntr : 1;
-    t.a = a;
-    t.d = d;
-    const TileFn kt = N == 2 ? (emit ? pick_tile<2, true>(tv, d2, d4) : pick_tile<2, false>(tv, d2, d4))
-                             : (emit ? pick_tile<1, true>(tv, d2, d4) : pick_tile<1, false>(tv, d2, d4));
-    hipLaunchKernelGGL(kt, dim3(8 * t.per_xcd, (a.ntr + t.per_block - 1) / t.per_block),
-                       dim3(tv.lx * tv.tw * tv.th), 0, s, t);
+    // and velocities (6.3 against 7.5 ms per step at nx=512, 4 tracers);
+    // where the tiles alone leave the chip short of blocks (fewer than 512)
+    // each tracer has its own
+    if (t.work < 512) t.per_block = 1;
+    hipLaunchKernelGGL(pick_tile<false>(N, m.tile.lx, d2, d4, emit),
+                       dim3(t.work, (a.ntr + t.per_block - 1) / t.per_block), dim3(kTileThreads), 0,
+                       s, t);
   }
+  OMEGA_HIP_CHECK(hipGetLastError());
+}
+
+void launch_stage_batch(const StageKind &k, const StageLaunch *desc, const int *who, int n, bool emit,
+                        hipStream_t s) {
+  TimerScope ts("batch_tend", s);
+  hipLaunchKernelGGL(k.N == 2 ? pick_batch_mom<2>(k.v2, emit) : pick_batch_mom<1>(k.v2, emit),
+                     dim3(n), dim3(256), 0, s, desc, who, n);
+  OMEGA_HIP_CHECK(hipGetLastError());
+}
+
+void launch_tile_batch(const StageKind &k, const TileLaunch *desc, const int *who, int n, bool emit,
+                       hipStream_t s) {
+  TimerScope ts("batch_tracers", s);
+  hipLaunchKernelGGL(pick_tile<true>(k.N, k.lx, k.d2, k.d4, emit), dim3(n), dim3(kTileThreads), 0, s,
+                     desc, who, n);
   OMEGA_HIP_CHECK(hipGetLastError());
 }
 

@@ -1,0 +1,53 @@
+// Parameter blocks of the stage kernels (kernels_stage.hip), passed by value
+// to a single model's launches and kept in tables for an ensemble's.
+#pragma once
+
+#include "internal.hpp"
+
+namespace omega_hip {
+
+// momentum and thickness: rows cells of lx lanes per block, ncb such blocks
+// per level chunk, tiles = ncb * chunks
+struct StageLaunch {
+  HexCoef q;
+  const int *rec; // neighbourhood records
+  int nc, L, lx, rows, ncb, tiles;
+  int block0; // first entry in an ensemble's launch
+  StageArgs a;
+  DiagOut d;
+  const double *x; // momentum del4: the edge field a Laplacian launch reads
+  double *y;       // and writes; the del4 term for the momentum launch
+};
+
+// tracers: work = tiles * level chunks
+struct TileLaunch {
+  HexCoef q;
+  const int *ids; // [tiles][(th + 4)(tw + 4)] cell at each place, row-major
+  int nx, ny, tiles_x, nch, work, nc, L, per_block;
+  int block0;
+  StageArgs a;
+  DiagOut d;
+};
+
+// Fills a stage's parameter blocks (t where a.ntr > 0) for N levels per lane.
+void stage_launch(const MeshView &m, const Launch &lc, int N, const HexCoef &q, const StageArgs &a,
+                  const DiagOut &d, StageLaunch &p, TileLaunch &t);
+int stage_levels(const MeshView &m, const Launch &lc); // N of a model's launches
+
+// What one launch of an ensemble's members has compiled in; members that
+// share it share the launch.
+struct StageKind {
+  int N, lx; // levels per lane, lanes of a tile
+  bool v2, d2, d4;
+  bool operator==(const StageKind &o) const {
+    return N == o.N && lx == o.lx && v2 == o.v2 && d2 == o.d2 && d4 == o.d4;
+  }
+};
+// One launch over n entries; entry b belongs to member who[b], whose
+// parameter block is desc[who[b]].
+void launch_stage_batch(const StageKind &k, const StageLaunch *desc, const int *who, int n, bool emit,
+                        hipStream_t s);
+void launch_tile_batch(const StageKind &k, const TileLaunch *desc, const int *who, int n, bool emit,
+                       hipStream_t s);
+
+} // namespace omega_hip

@@ -118,3 +118,29 @@ def test_stage_nonfinite_rows_spread_as_with_stored_diagnostics(value):
             out.append(gt.download())
         for a, b in zip(*out):
             assert same_bits(a, b), (field, at)
+
+
+@pytest.mark.parametrize("kind,graph", [("rk4", False), ("lsrk", True)])
+def test_stage_ensemble_members_step_as_alone(kind, graph):
+    """An ensemble whose members differ in grid, layer and tracer counts and
+    term sets, with one member on the kernels that store diagnostics: every
+    member ends with the bits of stepping alone."""
+    shapes = [(16, 16, 1, 1, 79), (9, 8, 5, 0, 15), (12, 10, 25, 2, 127 - 16), (8, 6, 60, 3, 79),
+              (10, 8, 64, 1, 7), (6, 4, 130, 2, 79), (10, 10, 16, 2, 127), (17, 6, 2, 1, 39)]
+    batch, alone = swe.Batch(kind, 5), []
+    batch.set_graph(graph)
+    keep = []
+    for i, (nx, ny, L, ntr, terms) in enumerate(shapes):
+        om, omodel, gm, gmodel, state = make_pair(nx, ny, L, ntr, seed=i)
+        gmodel.terms = terms
+        s = upload(gm, ntr, state)
+        batch.add(gmodel, s, 10.0 + i)
+        keep.append((gm, gmodel, s))
+        t = upload(gm, ntr, state)
+        st = swe.RK4Stepper(gmodel) if kind == "rk4" else swe.LSRKStepper(gmodel, 5)
+        alone.append((st, t, 10.0 + i))
+    batch.run(3)
+    for i, ((_, _, s), (st, t, dt)) in enumerate(zip(keep, alone)):
+        got = s.download()
+        st.run(0.0, dt, 3, t)
+        compare(got, t.download(), shapes[i])
