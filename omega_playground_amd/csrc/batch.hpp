@@ -38,4 +38,13 @@ void launch_batch_tend(const BatchMember *desc, const int *blk, int nblocks, int
                        int persistent, int kinds, int tset, hipStream_t s);
 bool term_set_batch(int terms);
 
+// Members' fields <-> the columns of stacked fields (omega_batch_adjoint_run)
+struct StackArgs {
+  static constexpr int kMany = 16;
+  Real *mem[kMany][3], *big[3];
+  size_t n[3]; // elements of a member's fields
+  int count, first, L, wide, to_big;
+};
+void launch_stack(const StackArgs &a, hipStream_t s);
+
 } // namespace omega_hip

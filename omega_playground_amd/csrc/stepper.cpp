@@ -2,6 +2,7 @@
 // (diagnostics + fused tendency/update launch), the RK4 and low-storage RK
 // steppers and their HIP-graph capture.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <mutex>
 
@@ -95,6 +96,11 @@ void ensure_vdel4(omega_model_s *M) {
     M->vdel2_div_c.alloc((size_t)hm.ncells * L);
   }
   if (M->mesh->dm.stage_ok && !M->vdel4_e.p) M->vdel4_e.alloc((size_t)hm.nedges * L);
+}
+
+uint64_t next_uid() {
+  static std::atomic<uint64_t> n{0};
+  return ++n;
 }
 
 hipStream_t capture_stream() {
