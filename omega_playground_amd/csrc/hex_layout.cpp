@@ -17,12 +17,24 @@ namespace omega_hip {
 
 namespace {
 
-int local_index(std::vector<int> &list, int id) {
-  for (size_t i = 0; i < list.size(); ++i)
-    if (list[i] == id) return (int)i;
-  list.push_back(id);
-  return (int)list.size() - 1;
-}
+// Ids numbered in first-appearance order against an expected numbering:
+// expect(k, id) is true when id is the k-th distinct id, known or new; that
+// the ids taken are distinct is checked once at the end.
+template <int most> struct Appear {
+  int id[most], n = 0;
+  bool expect(int k, int x) {
+    if (k < n) return id[k] == x;
+    if (k > n || n == most) return false;
+    id[n++] = x;
+    return true;
+  }
+  bool distinct() const {
+    for (int i = 1; i < n; ++i)
+      for (int j = 0; j < i; ++j)
+        if (id[i] == id[j]) return false;
+    return true;
+  }
+};
 
 } // namespace
 
@@ -48,32 +60,28 @@ bool build_hex_records(DeviceMesh &dm) {
     }
   }
   dm.hexrec_h.assign((size_t)NE * hex::kRecInts, 0);
-  std::vector<int> uv, uc;
   for (int c = 0; c < NC; ++c) {
     for (int k = 0; k < 3; ++k) {
       const int e = dm.eofs_h[c] + k;
       if (dm.noe_h[e] != hex::kSlots) return false;
-      uv.clear();
-      uc.clear();
+      Appear<hex::kUniq> uv, uc;
       int *rec = &dm.hexrec_h[(size_t)e * hex::kRecInts];
       for (int j = 0; j < hex::kSlots; ++j) {
         const int ej = dm.eoe_h[(size_t)e * dm.me2 + j];
         rec[j] = ej;
-        const int v0 = local_index(uv, dm.voe_h[2 * (size_t)ej]);
-        const int v1 = local_index(uv, dm.voe_h[2 * (size_t)ej + 1]);
-        const int q0 = local_index(uc, dm.coe_h[2 * (size_t)ej]);
-        const int q1 = local_index(uc, dm.coe_h[2 * (size_t)ej + 1]);
-        if (v0 != hex::LV0[k][j] || v1 != hex::LV1[k][j] || q0 != hex::LC0[k][j] ||
-            q1 != hex::LC1[k][j])
+        if (!uv.expect(hex::LV0[k][j], dm.voe_h[2 * (size_t)ej]) ||
+            !uv.expect(hex::LV1[k][j], dm.voe_h[2 * (size_t)ej + 1]) ||
+            !uc.expect(hex::LC0[k][j], dm.coe_h[2 * (size_t)ej]) ||
+            !uc.expect(hex::LC1[k][j], dm.coe_h[2 * (size_t)ej + 1]))
           return false;
       }
-      if ((int)uv.size() != hex::kUniq || (int)uc.size() != hex::kUniq) return false;
+      if (uv.n != hex::kUniq || uc.n != hex::kUniq || !uv.distinct() || !uc.distinct()) return false;
       for (int s = 0; s < 2; ++s) {
-        if (uv[hex::OWNV[k][s]] != dm.voe_h[2 * (size_t)e + s]) return false;
-        if (uc[hex::OWNC[k][s]] != dm.coe_h[2 * (size_t)e + s]) return false;
+        if (uv.id[hex::OWNV[k][s]] != dm.voe_h[2 * (size_t)e + s]) return false;
+        if (uc.id[hex::OWNC[k][s]] != dm.coe_h[2 * (size_t)e + s]) return false;
       }
-      std::copy(uv.begin(), uv.end(), rec + 10);
-      std::copy(uc.begin(), uc.end(), rec + 20);
+      std::copy(uv.id, uv.id + hex::kUniq, rec + 10);
+      std::copy(uc.id, uc.id + hex::kUniq, rec + 20);
     }
   }
   dm.hex_ok = true;
@@ -98,47 +106,40 @@ bool build_hex_records(DeviceMesh &dm) {
   // per-cell union stencil: every cell must reproduce the hexu tables
   dm.hexu_ok = false;
   dm.hexu_h.assign((size_t)NC * hexu::kRec, 0);
-  std::vector<int> ue, uv2, uc2;
-  auto check = [](bool ok) {
-    if (!ok) throw 0;
-  };
-  try {
-    for (int c = 0; c < NC; ++c) {
-      ue = {dm.eofs_h[c], dm.eofs_h[c] + 1, dm.eofs_h[c] + 2};
-      uv2.clear();
-      uc2.clear();
-      for (int k = 0; k < 3; ++k) {
-        const int e = dm.eofs_h[c] + k;
-        for (int j = 0; j < hex::kSlots; ++j) {
-          const int ej = dm.eoe_h[(size_t)e * dm.me2 + j];
-          check(local_index(ue, ej) == hexu::TE[k][j]);
-          check(local_index(uv2, dm.voe_h[2 * (size_t)ej]) == hexu::TV0[k][j]);
-          check(local_index(uv2, dm.voe_h[2 * (size_t)ej + 1]) == hexu::TV1[k][j]);
-          check(local_index(uc2, dm.coe_h[2 * (size_t)ej]) == hexu::TC0[k][j]);
-          check(local_index(uc2, dm.coe_h[2 * (size_t)ej + 1]) == hexu::TC1[k][j]);
-        }
-        for (int s = 0; s < 2; ++s) {
-          check(local_index(uv2, dm.voe_h[2 * (size_t)e + s]) == hexu::OV[k][s]);
-          check(local_index(uc2, dm.coe_h[2 * (size_t)e + s]) == hexu::OC[k][s]);
-        }
+  for (int c = 0; c < NC; ++c) {
+    Appear<hexu::kNE> ue;
+    Appear<hexu::kNV> uv;
+    Appear<hexu::kNC> uc;
+    bool ok = true;
+    for (int k = 0; k < 3; ++k) ok = ok && ue.expect(k, dm.eofs_h[c] + k);
+    for (int k = 0; k < 3 && ok; ++k) {
+      const size_t e = dm.eofs_h[c] + k;
+      for (int j = 0; j < hex::kSlots; ++j) {
+        const size_t ej = dm.eoe_h[e * dm.me2 + j];
+        ok = ok && ue.expect(hexu::TE[k][j], (int)ej) && uv.expect(hexu::TV0[k][j], dm.voe_h[2 * ej]) &&
+             uv.expect(hexu::TV1[k][j], dm.voe_h[2 * ej + 1]) &&
+             uc.expect(hexu::TC0[k][j], dm.coe_h[2 * ej]) &&
+             uc.expect(hexu::TC1[k][j], dm.coe_h[2 * ej + 1]);
       }
-      for (int j = 0; j < 6; ++j) {
-        const int e = dm.eoc_h[(size_t)c * ME + j];
-        check(local_index(ue, e) == hexu::CE[j]);
-        check(local_index(uc2, dm.coe_h[2 * (size_t)e]) == hexu::CC0[j]);
-        check(local_index(uc2, dm.coe_h[2 * (size_t)e + 1]) == hexu::CC1[j]);
-      }
-      check(local_index(uc2, c) == hexu::SELF);
-      check((int)ue.size() == hexu::kNE && (int)uv2.size() == hexu::kNV &&
-            (int)uc2.size() == hexu::kNC);
-      int *rec = &dm.hexu_h[(size_t)c * hexu::kRec];
-      std::copy(ue.begin(), ue.end(), rec);
-      std::copy(uv2.begin(), uv2.end(), rec + hexu::kNE);
-      std::copy(uc2.begin(), uc2.end(), rec + hexu::kNE + hexu::kNV);
+      for (int s = 0; s < 2; ++s)
+        ok = ok && uv.expect(hexu::OV[k][s], dm.voe_h[2 * e + s]) &&
+             uc.expect(hexu::OC[k][s], dm.coe_h[2 * e + s]);
     }
-  } catch (int) {
-    dm.hexu_h.clear();
-    return true;
+    for (int j = 0; j < 6 && ok; ++j) {
+      const size_t e = dm.eoc_h[(size_t)c * ME + j];
+      ok = ue.expect(hexu::CE[j], (int)e) && uc.expect(hexu::CC0[j], dm.coe_h[2 * e]) &&
+           uc.expect(hexu::CC1[j], dm.coe_h[2 * e + 1]);
+    }
+    ok = ok && uc.expect(hexu::SELF, c) && ue.n == hexu::kNE && uv.n == hexu::kNV &&
+         uc.n == hexu::kNC && ue.distinct() && uv.distinct() && uc.distinct();
+    if (!ok) {
+      dm.hexu_h.clear();
+      return true;
+    }
+    int *rec = &dm.hexu_h[(size_t)c * hexu::kRec];
+    std::copy(ue.id, ue.id + hexu::kNE, rec);
+    std::copy(uv.id, uv.id + hexu::kNV, rec + hexu::kNE);
+    std::copy(uc.id, uc.id + hexu::kNC, rec + hexu::kNE + hexu::kNV);
   }
   dm.hexu_ok = true;
   return true;
@@ -178,7 +179,17 @@ void build_hex_stage(DeviceMesh &dm) {
       if (coc[6 * (size_t)n + (d + 3) % 6] != c) return;
       if (coc[6 * (size_t)n + (d + 2) % 6] != coc[6 * (size_t)c + (d + 1) % 6]) return;
     }
-  dm.hexc_h.assign((size_t)NC * hl::kRec, 0);
+  // the lattice's places as tables
+  int ce[6], pe[3][10];
+  hl::Edge ed[3];
+  hl::Vert ve[2];
+  for (int d = 0; d < 6; ++d) ce[d] = hl::cell_edge(0, d);
+  for (int K = 0; K < 3; ++K) {
+    ed[K] = hl::edge(K);
+    for (int j = 0; j < 10; ++j) pe[K][j] = hl::pv_edge(K, j);
+  }
+  for (int x = 0; x < 2; ++x) ve[x] = hl::vert(x);
+  dm.hexc_h.resize((size_t)NC * hl::kRec);
   for (int c = 0; c < NC; ++c) {
     int *r = &dm.hexc_h[(size_t)c * hl::kRec];
     r[0] = c;
@@ -187,22 +198,21 @@ void build_hex_stage(DeviceMesh &dm) {
       r[7 + 2 * d] = coc[6 * (size_t)r[1 + d] + d];
       r[8 + 2 * d] = coc[6 * (size_t)r[1 + d] + (d + 1) % 6];
     }
+    r[19] = 0;
     auto eid = [&](int e) { return 3 * r[e / 3] + e % 3; };
     auto vid = [&](int v) { return 2 * r[v / 2] + v % 2; };
     bool ok = true;
-    for (int d = 0; d < 6; ++d) ok = ok && dm.eoc_h[(size_t)c * ME + d] == eid(hl::cell_edge(0, d));
+    for (int d = 0; d < 6; ++d) ok = ok && dm.eoc_h[(size_t)c * ME + d] == eid(ce[d]);
     for (int K = 0; K < 3; ++K) {
       const size_t e = 3 * (size_t)c + K;
-      const hl::Edge t = hl::edge(K);
       for (int s = 0; s < 2; ++s)
-        ok = ok && dm.coe_h[2 * e + s] == r[t.c[s]] && dm.voe_h[2 * e + s] == vid(t.v[s]);
-      for (int j = 0; j < 10; ++j) ok = ok && dm.eoe_h[e * 10 + j] == eid(hl::pv_edge(K, j));
+        ok = ok && dm.coe_h[2 * e + s] == r[ed[K].c[s]] && dm.voe_h[2 * e + s] == vid(ed[K].v[s]);
+      for (int j = 0; j < 10; ++j) ok = ok && dm.eoe_h[e * 10 + j] == eid(pe[K][j]);
     }
     for (int x = 0; x < 2; ++x) {
       const size_t v = 2 * (size_t)c + x;
-      const hl::Vert t = hl::vert(x);
       for (int j = 0; j < 3; ++j)
-        ok = ok && dm.eov_h[3 * v + j] == eid(t.e[j]) && dm.cov_h[3 * v + j] == r[t.c[j]];
+        ok = ok && dm.eov_h[3 * v + j] == eid(ve[x].e[j]) && dm.cov_h[3 * v + j] == r[ve[x].c[j]];
     }
     if (!ok) {
       dm.hexc_h.clear();
@@ -248,15 +258,18 @@ void build_hex_stage(DeviceMesh &dm) {
   t.nx = nx;
   t.ny = ny;
   const int tx = (nx + t.tw - 1) / t.tw, ty = (ny + t.th - 1) / t.th;
-  dm.tile_h.clear();
-  dm.tile_h.reserve((size_t)tx * ty * (t.tw + 4) * (t.th + 4));
+  dm.tile_h.resize((size_t)tx * ty * (t.tw + 4) * (t.th + 4));
+  int *id = dm.tile_h.data();
   for (int j = 0; j < ty; ++j)
     for (int i = 0; i < tx; ++i)
-      for (int y = -2; y < t.th + 2; ++y)
-        for (int x = -2; x < t.tw + 2; ++x) {
-          const int r = ((j * t.th + y) % ny + ny) % ny, q = ((i * t.tw + x) % nx + nx) % nx;
-          dm.tile_h.push_back(at[(size_t)r * nx + q]);
+      for (int y = -2; y < t.th + 2; ++y) {
+        const int *row = &at[(size_t)(((j * t.th + y) % ny + ny) % ny) * nx];
+        int q = ((i * t.tw - 2) % nx + nx) % nx;
+        for (int x = 0; x < t.tw + 4; ++x) {
+          *id++ = row[q];
+          if (++q == nx) q = 0;
         }
+      }
   dm.stage_ok = true;
 }
 

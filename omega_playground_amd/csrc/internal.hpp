@@ -52,12 +52,12 @@ template <class T> struct DBuf {
     return *this;
   }
   ~DBuf() { release(); }
-  void alloc(size_t count) {
+  void alloc(size_t count, bool zero = true) {
     release();
     n = count;
     if (count) {
       OMEGA_HIP_CHECK(hipMalloc(&p, count * sizeof(T)));
-      OMEGA_HIP_CHECK(hipMemset(p, 0, count * sizeof(T)));
+      if (zero) OMEGA_HIP_CHECK(hipMemset(p, 0, count * sizeof(T)));
     }
   }
   void release() {
@@ -66,7 +66,7 @@ template <class T> struct DBuf {
     n = 0;
   }
   void upload(const std::vector<T> &h) {
-    if (n != h.size()) alloc(h.size());
+    if (n != h.size()) alloc(h.size(), false);
     if (n) OMEGA_HIP_CHECK(hipMemcpy(p, h.data(), n * sizeof(T), hipMemcpyHostToDevice));
   }
 };

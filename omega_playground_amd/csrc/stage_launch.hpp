@@ -34,6 +34,14 @@ void stage_launch(const MeshView &m, const Launch &lc, int N, const HexCoef &q, 
                   const DiagOut &d, StageLaunch &p, TileLaunch &t);
 int stage_levels(const MeshView &m, const Launch &lc); // N of a model's launches
 
+// Fewer tiles than this (two blocks per CU) leave the chip short of blocks.
+constexpr int kFewTiles = 512;
+
+// Both in one launch, where that is the faster one (kernels_stage_both.hip);
+// false: nothing launched.
+bool launch_stage_both(int N, int lx, const StageLaunch &p, const TileLaunch &t, bool emit,
+                       hipStream_t s);
+
 // What one launch of an ensemble's members has compiled in; members that
 // share it share the launch.
 struct StageKind {
