@@ -139,6 +139,8 @@ struct MeshView {
   const int *hexu;              // [nc][49] per-cell union stencil (hex_pattern.hpp)
   const int *coc;               // cells_on_cell [nc][6]
   const int *hexc;              // [nc][20] neighbourhood cells (hex_lattice.hpp)
+  const int *ccx;               // [nc][me] cell across each edge, top bit set where
+                                // the cell is the edge's second (null on regular meshes)
   TileView tile;                // ids null where the mesh has no tiles
 };
 
@@ -180,7 +182,8 @@ struct DeviceMesh {
   // the mesh is the lattice of hex_lattice.hpp with one value per coefficient
   // kind (stage_coef holds the mesh's share); hexc_h its neighbourhood records
   bool stage_ok = false;
-  std::vector<int> tile_h;
+  std::vector<int> tile_h, ccx_h;
+  DBuf<int> ccx;
   DBuf<int> tile_ids;
   TileView tile{};
   HexCoef stage_coef{};
@@ -245,6 +248,9 @@ struct DiagOut {
   Real *vdel2_e;               // [ne][L]  (momentum del4 pre-pass)
   Real *vdel2_rv_v, *vdel2_div_c;
   Real *vdel4_e;               // [ne][L]  del4 term of the stage kernels
+  // edge means of the general kernels (mean thickness, relative and planetary
+  // PV, [ne][L]) and 1/h [nc][L]; null: formed where they are read
+  Real *fh_e, *nrv_e, *npv_e, *inv_h_c;
 };
 
 struct ModelCoef {
@@ -281,6 +287,10 @@ void launch_diag(const MeshView &m, const Launch &lc, const ModelCoef &mc, int t
 void launch_vdel4(const MeshView &m, const Launch &lc, const DiagOut &d, hipStream_t s);
 void launch_tend(const MeshView &m, const Launch &lc, const ModelCoef &mc, const StageArgs &a,
                  const DiagOut &d, hipStream_t s);
+// Diagnostics, edge means, tendencies and stage update of a general mesh
+// (d with the means' arrays)
+void launch_stage_means(const MeshView &m, const Launch &lc, const ModelCoef &mc, const StageArgs &a,
+                        const DiagOut &d, hipStream_t s);
 // Linear model (LinearShallowWaterModel): h_t = -h0 div(vn),
 // vn_t = f_e * (TRiSK tangential velocity) - g grad(h), with the stage update
 struct LinCoef {

@@ -27,7 +27,7 @@ using namespace fwd;
 // ---------------------------------------------------------------------------
 // Diagnostics
 // ---------------------------------------------------------------------------
-template <int N>
+template <int N, bool MEANS = false>
 __global__ void __launch_bounds__(256)
     k_diag(MeshView m, int terms, int ntr, const double *__restrict__ h,
            const double *__restrict__ vn, const double *__restrict__ tr, DiagOut d, int swz) {
@@ -42,7 +42,7 @@ __global__ void __launch_bounds__(256)
     const int vb = m.vofs[c0], ve = m.vofs[c1];
     for (int v = vb + (int)threadIdx.y; v < ve; v += R) vertex_diag<N>(m, v, k, h, vn, d);
   }
-  for (int c = c0 + (int)threadIdx.y; c < c1; c += R) cell_diag<N>(m, terms, ntr, c, k, h, vn, tr, d);
+  for (int c = c0 + (int)threadIdx.y; c < c1; c += R) cell_diag<N, MEANS>(m, terms, ntr, c, k, h, vn, tr, d);
 }
 
 // ---------------------------------------------------------------------------
@@ -79,7 +79,28 @@ __global__ void __launch_bounds__(256) k_vdel4_vc(MeshView m, DiagOut d, int swz
 // Tendencies + stage update
 // ---------------------------------------------------------------------------
 
+// Edge means and, with tracer del4, the tracer Laplacians (after k_diag's
+// vertices and 1/h)
 template <int N>
+__global__ void __launch_bounds__(256)
+    k_means(MeshView m, ModelCoef mc, int terms, int ntr, const double *__restrict__ h,
+            const double *__restrict__ tr, DiagOut d, int swz) {
+  const int s = logical_block(blockIdx.x, gridDim.x, swz);
+  const int R = blockDim.y;
+  const int c0 = s * R;
+  if (c0 >= m.nc) return;
+  const int c1 = min(c0 + R, m.nc);
+  const int k = (blockIdx.y * blockDim.x + threadIdx.x) * N;
+  if (k >= m.L) return;
+  const int eb = m.eofs[c0], ee = m.eofs[c1];
+  for (int e = eb + (int)threadIdx.y; e < ee; e += R) edge_means<N>(m, mc, h, d, terms, e, k);
+  if ((terms & T_TDEL4) && ntr > 0)
+    for (int c = c0 + (int)threadIdx.y; c < c1; c += R) cell_del2_means<N>(m, ntr, c, k, h, tr, d);
+}
+
+// MEANS: blockIdx.z 0 the edges, 1 the cells of the block, from the stored
+// means
+template <int N, bool MEANS = false>
 __global__ void __launch_bounds__(256)
     k_tend(MeshView m, ModelCoef mc, StageArgs a, DiagOut d, int swz) {
   const int s = logical_block(blockIdx.x, gridDim.x, swz);
@@ -90,6 +111,13 @@ __global__ void __launch_bounds__(256)
   const int k = (blockIdx.y * blockDim.x + threadIdx.x) * N;
   if (k >= m.L) return;
   const int eb = m.eofs[c0], ee = m.eofs[c1];
+  if constexpr (MEANS) {
+    if (blockIdx.z == 0)
+      for (int e = eb + (int)threadIdx.y; e < ee; e += R) edge_tend<N, true>(m, mc, a, d, e, k);
+    else
+      for (int c = c0 + (int)threadIdx.y; c < c1; c += R) cell_tend_means<N>(m, mc, a, d, c, k);
+    return;
+  }
   for (int e = eb + (int)threadIdx.y; e < ee; e += R) edge_tend<N>(m, mc, a, d, e, k);
   for (int c = c0 + (int)threadIdx.y; c < c1; c += R) cell_tend<N>(m, mc, a, d, c, k);
 }
@@ -276,6 +304,27 @@ void launch_tend(const MeshView &m, const Launch &lc, const ModelCoef &mc, const
     hipLaunchKernelGGL(k_tend<2>, g.grid, g.block, 0, s, m, mc, a, d, lc.swizzle);
   else
     hipLaunchKernelGGL(k_tend<1>, g.grid, g.block, 0, s, m, mc, a, d, lc.swizzle);
+  OMEGA_HIP_CHECK(hipGetLastError());
+}
+
+void launch_stage_means(const MeshView &m, const Launch &lc, const ModelCoef &mc, const StageArgs &a,
+                        const DiagOut &d, hipStream_t s) {
+  const int N = (lc.lpt == 2 && m.L % 2 == 0) ? 2 : 1;
+  Launch ld = lc; // the diagnostics launch may have its own block height
+  if (ld.drows >= 0) ld.rows = ld.drows;
+  const Geo g = geometry(m, lc, N), gd = geometry(m, ld, N);
+  {
+    TimerScope ts("diag", s);
+    hipLaunchKernelGGL((N == 2 ? k_diag<2, true> : k_diag<1, true>), gd.grid, gd.block, 0, s, m,
+                       a.terms, a.ntr, a.h.in, a.vn.in, a.tr.in, d, lc.swizzle);
+    hipLaunchKernelGGL((N == 2 ? k_means<2> : k_means<1>), gd.grid, gd.block, 0, s, m, mc, a.terms,
+                       a.ntr, a.h.in, a.tr.in, d, lc.swizzle);
+  }
+  if (a.terms & T_VDEL4) launch_vdel4(m, lc, d, s);
+  TimerScope ts("tend", s);
+  const dim3 grid(g.grid.x, g.grid.y, 2);
+  hipLaunchKernelGGL((N == 2 ? k_tend<2, true> : k_tend<1, true>), grid, g.block, 0, s, m, mc, a, d,
+                     lc.swizzle);
   OMEGA_HIP_CHECK(hipGetLastError());
 }
 

@@ -1,5 +1,6 @@
 // Host-side mesh construction, space-filling-curve ordering and upload.
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <numeric>
@@ -432,6 +433,16 @@ void DeviceMesh::build_device(int ord) {
   const size_t rows = std::max({(size_t)NC, (size_t)NE, (size_t)NV});
   off32 = rows < (size_t(1) << 24) && rows * (size_t)L * sizeof(double) < (size_t(1) << 32);
   build_hex_stage(*this);
+  ccx_h.clear();
+  if (!hex_ok) {
+    ccx_h.assign((size_t)NC * ME, 0);
+    for (int c = 0; c < NC; ++c)
+      for (int j = 0; j < noc_h[c]; ++j) {
+        const size_t e = eoc_h[(size_t)c * ME + j];
+        const bool second = coe_h[2 * e] != c;
+        ccx_h[(size_t)c * ME + j] = coe_h[2 * e + (second ? 0 : 1)] | (second ? INT_MIN : 0);
+      }
+  }
   uploaded = false;
 }
 
@@ -447,6 +458,7 @@ void DeviceMesh::upload() {
   s2.upload(s2_h); s4.upload(s4_h); maxlev_e.upload(maxlev_h);
   eov.upload(eov_h); cov.upload(cov_h); crv.upload(crv_h); cth.upload(cth_h);
   eofs.upload(eofs_h); vofs.upload(vofs_h);
+  if (!hex_ok) ccx.upload(ccx_h);
   if (hex_ok) {
     hexrec.upload(hexrec_h);
     if (hexu_ok) hexu.upload(hexu_h);
@@ -515,6 +527,7 @@ MeshView DeviceMesh::view() const {
   v.hexu = hexu.p;
   v.coc = coc.p;
   v.hexc = hexc.p;
+  v.ccx = ccx.p;
   v.tile = tile;
   v.tile.ids = tile_ids.p;
   return v;

@@ -75,6 +75,7 @@ struct omega_model_s {
   const Real *aux_h = nullptr, *aux_vn = nullptr, *aux_tr = nullptr;
   DBuf<Real> f_v, cv2, cv4, ct2, ct4;
   DBuf<Real> rvort_v, inv_thick_v, ke_c, div_c, trdel2_c, vdel2_e, vdel2_rv_v, vdel2_div_c;
+  DBuf<Real> fh_e, nrv_e, npv_e, inv_h_c; // edge means of the general kernels
   DBuf<Real> vdel4_e; // scratch of the stage kernels with momentum del4
   DBuf<Real> partial, result;
   omega_additional_tendency_fn add_fn = nullptr;
@@ -139,10 +140,12 @@ struct omega_model_s {
     if (diag_slot > 0) {
       DiagSet &d = diag_sets[diag_slot - 1];
       return DiagOut{d.rvort_v.p, d.inv_thick_v.p, d.ke_c.p, d.div_c.p, d.trdel2_c.p,
-                     d.vdel2_e.p, d.vdel2_rv_v.p, d.vdel2_div_c.p, vdel4_e.p};
+                     d.vdel2_e.p, d.vdel2_rv_v.p, d.vdel2_div_c.p, vdel4_e.p,
+                     fh_e.p, nrv_e.p, npv_e.p, inv_h_c.p};
     }
     return DiagOut{rvort_v.p, inv_thick_v.p, ke_c.p, div_c.p, trdel2_c.p,
-                   vdel2_e.p, vdel2_rv_v.p, vdel2_div_c.p, vdel4_e.p};
+                   vdel2_e.p, vdel2_rv_v.p, vdel2_div_c.p, vdel4_e.p,
+                   fh_e.p, nrv_e.p, npv_e.p, inv_h_c.p};
   }
 };
 

@@ -63,6 +63,10 @@ void model_build_coefficients(omega_model_s *M) {
   M->ke_c.alloc((size_t)NC * L);
   M->div_c.alloc((size_t)NC * L);
   if (ntr > 0) M->trdel2_c.alloc(ntr * NC * L);
+  if (!dm.hex_ok && !M->linear) {
+    for (DBuf<Real> *b : {&M->fh_e, &M->nrv_e, &M->npv_e}) b->alloc((size_t)NE * L, false);
+    M->inv_h_c.alloc((size_t)NC * L, false);
+  }
   M->partial.alloc((size_t)reduce_blocks(std::max(NC, NV)) + 1);
   M->result.alloc(4);
 }
@@ -213,6 +217,14 @@ void run_stage(omega_model_s *M, StageArgs a, hipStream_t s, int fields, bool wi
     M->aux_tr = a.tr.in;
     if (M->terms & T_VDEL4) ensure_vdel4(M);
     launch_stage_hex(mv, M->lc, q, a, M->diag(), emit, s);
+    return;
+  }
+  if (with_diag && !pre && fields == 7 && mv.ccx && M->fh_e.p && a.do_h && a.do_vn) {
+    M->aux_h = a.h.in;
+    M->aux_vn = a.vn.in;
+    M->aux_tr = a.tr.in;
+    if (M->terms & T_VDEL4) ensure_vdel4(M);
+    launch_stage_means(mv, M->lc, mc, a, M->diag(), s);
     return;
   }
   if (with_diag) run_diag(M, a.h.in, a.vn.in, a.tr.in, s);

@@ -144,3 +144,33 @@ def test_stage_ensemble_members_step_as_alone(kind, graph):
         got = s.download()
         st.run(0.0, dt, 3, t)
         compare(got, t.download(), shapes[i])
+
+
+@pytest.mark.parametrize("L,ntr,terms", [(1, 1, 127), (2, 5, 127), (5, 0, 31), (33, 4, 79), (66, 9, 111),
+                                         (130, 1, 255)])
+def test_general_mesh_edge_means_bitwise(L, ntr, terms):
+    """General meshes (pentagons; 9 and 10 edges on edge) through the stored
+    edge means, at odd and even layer counts, tracer groups and level chunks,
+    with bottom drag: the oracle's bits, and the auxiliary state the per-field
+    tendencies read afterwards."""
+    from test_gpu_general_mesh import DT, make
+    om, omodel, gm, gmodel, pd, state = make(2, L, ntr, terms=terms, seed=L)
+    ref = omodel.new_state()
+    omodel.compute_tendency(ref, state, 0.0)
+    gs, gt = upload(gm, ntr, state), swe.ShallowWaterState(gm, ntr)
+    gmodel.compute_tendency(gt, gs, 0.0)
+    compare(gt.download(), ref, "tendency")
+    h, vn, tr = gs.device_ptrs()
+    fields = gt.device_ptrs()
+    gmodel.compute_h_tendency_dev(fields[0], h, vn)
+    gmodel.compute_vn_tendency_dev(fields[1], h, vn)
+    if ntr:
+        gmodel.compute_tr_tendency_dev(fields[2], tr, vn)
+    compare(gt.download(), ref, "fields")
+    for kind, graph in (("rk4", True), ("lsrk", False)):
+        st = swe.RK4Stepper(gmodel) if kind == "rk4" else swe.LSRKStepper(gmodel, 5)
+        st.set_graph(graph)
+        s, r = upload(gm, ntr, state), tuple(a.copy() for a in state)
+        st.run(0.0, DT, 2, s)
+        po.Stepper(omodel, kind, 5).run(0.0, DT, 2, r)
+        compare(s.download(), r, kind)
