@@ -117,6 +117,8 @@ template <int N> struct MomOut {
   Vd<N> u[3], ke_grad[3], ssh_grad[3], visc[3];
   Vd<N> h; // thickness tendency
   Vd<N> rv[2], it[2], ke, div; // the cell's own diagnostics
+  // PRE: the rows of the owned edges a tendency VJP reads here (PreOut)
+  Vd<N> se[3], fu[3], own[3];
 };
 
 // The walk keeps few rows live at a time: the four vertices of the owned
@@ -128,15 +130,17 @@ template <int N> struct MomOut {
 // them, and FENCE keeps the scheduler from hoisting a later leg's rows above
 // an earlier one's arithmetic; without these the walk needs 180 registers
 // and half the wavefronts.
-template <int N, bool V2>
+// early(o): called once o's rv, it, se and fu are set, to store them before
+// the walk goes on.
+template <int N, bool V2, bool PRE, class Early>
 __device__ __forceinline__ void momentum(const HexCoef &q, const Ctx &x,
                                          const int (&id)[hl::kCells], const double *__restrict__ h,
-                                         const double *__restrict__ vn, MomOut<N> &o) {
+                                         const double *__restrict__ vn, MomOut<N> &o, Early early) {
   const unsigned L8 = x.L8;
   unsigned k8 = x.k8;
   Vd<N> hv[hl::kCells], v[hl::kEdges];
   Vd<N> P[hl::kVerts], Q[hl::kVerts], rvort[hl::kVerts];
-  Vd<N> S[hl::kEdges], T[hl::kEdges], G[hl::kEdges], G2[hl::kEdges];
+  Vd<N> S[hl::kEdges], T[hl::kEdges], G[hl::kEdges], G2[hl::kEdges], F[hl::kEdges];
   Vd<N> ke[4], dv[4], qs[3], qt[3], curl[3];
   auto H = [&](auto... I) {
     ((hv[I] = ldo<N>(h, __umul24((unsigned)id[I], L8) + k8)), ...);
@@ -179,6 +183,7 @@ __device__ __forceinline__ void momentum(const HexCoef &q, const Ctx &x,
       const double s = hv[t.c[0]][i] + hv[t.c[1]][i];
       G[e][i] = (q.w2 * s) * v[e][i];
       G2[e][i] = (q.w * s) * v[e][i];
+      if constexpr (PRE) F[e][i] = (0.5 * s) * v[e][i];
     }
   };
   // slot j of the PV stencil of owned edge K (the slots of weight zero too: an
@@ -192,6 +197,13 @@ __device__ __forceinline__ void momentum(const HexCoef &q, const Ctx &x,
       if constexpr (m > 0) qt[K][i] = qt[K][i] + t;
       else if constexpr (m < 0) qt[K][i] = qt[K][i] - t;
       else qt[K][i] = __builtin_fma(t, 0.0, qt[K][i]);
+      if constexpr (PRE) {
+        // flux-weighted sum: weight times flux, in slot order
+        const double x = ((m == 2 || m == -2 ? 2 * q.w : q.w) * F[e][i]);
+        if constexpr (m > 0) o.own[K][i] = o.own[K][i] + x;
+        else if constexpr (m < 0) o.own[K][i] = o.own[K][i] - x;
+        else o.own[K][i] = __builtin_fma(F[e][i], 0.0, o.own[K][i]);
+      }
     }
   };
   // kinetic energy and divergence of cell b
@@ -230,10 +242,16 @@ __device__ __forceinline__ void momentum(const HexCoef &q, const Ctx &x,
       qs[K][i] = (P[t.v[0]][i] + P[t.v[1]][i]) + (Q[t.v[0]][i] + Q[t.v[1]][i]);
       qt[K][i] = 0.0;
       curl[K][i] = (rvort[t.v[1]][i] - rvort[t.v[0]][i]) * q.idv;
+      if constexpr (PRE) {
+        o.se[K][i] = 2.0 * qs[K][i];
+        o.own[K][i] = 0.0;
+        o.fu[K][i] = 0.5 * (hv[t.c[0]][i] + hv[t.c[1]][i]) * v[K][i];
+      }
     }
   });
   pin(P[0], Q[0], P[1], Q[1], P[6], Q[6], P[9], Q[9], qs[0], qs[1], qs[2], qt[0], qt[1], qt[2]);
   if constexpr (V2) pin(curl[0], curl[1], curl[2]);
+  early(o);
   FENCE();
   // round W: its sides NE, NW, (W), SW, SE
   V(HEXC(7), HEXC(8), HEXC(26), HEXC(10), HEXC(30));
@@ -256,6 +274,7 @@ __device__ __forceinline__ void momentum(const HexCoef &q, const Ctx &x,
   pv(HEXC(1), HEXC(0));
   cell(c1, HEXC(1));
   pin(qt[0], qt[1], ke[1], P[4], Q[4]);
+  if constexpr (PRE) pin(o.own[0], o.own[1]);
   if constexpr (V2) pin(dv[1]);
   FENCE();
   // round SW: its sides W, (SW), SE, E
@@ -276,6 +295,7 @@ __device__ __forceinline__ void momentum(const HexCoef &q, const Ctx &x,
   pv(HEXC(2), HEXC(0));
   cell(c2, HEXC(2));
   pin(qt[1], qt[2], ke[2], P[7], Q[7]);
+  if constexpr (PRE) pin(o.own[1], o.own[2]);
   if constexpr (V2) pin(dv[2]);
   FENCE();
   // round SE: its sides W, (SW), SE, E, NE
@@ -297,6 +317,7 @@ __device__ __forceinline__ void momentum(const HexCoef &q, const Ctx &x,
   H(HEXC(4), HEXC(5), HEXC(6));
   V(HEXC(17), HEXC(15), HEXC(12), HEXC(16), HEXC(20));
   pin(qt[2], ke[3]);
+  if constexpr (PRE) pin(o.own[2]);
   if constexpr (V2) pin(dv[3]);
   FENCE();
   const LegCoef c4 = leg_coef<4>(q);

@@ -253,6 +253,13 @@ struct DiagOut {
   Real *fh_e, *nrv_e, *npv_e, *inv_h_c;
 };
 
+// Rows a tendency VJP reads at its linearisation state ([ne][L] each): the
+// edge PV sum Q_e + P_e, the edge thickness flux F_e u_e and the flux-weighted
+// edges-on-edge sum sum_j w_ej F_j u_j.  A stage kernel that evaluates the
+// tendency at that state can write them (the adjoint's stage recomputation).
+struct PreOut {
+  Real *se, *fu, *own;
+};
 struct ModelCoef {
   Real grav;
   const Real *f_v;   // [nv]
@@ -302,13 +309,6 @@ struct LinCoef {
 };
 void launch_tend_linear(const MeshView &m, const Launch &lc, const LinCoef &lin,
                         const StageArgs &a, hipStream_t s);
-// Rows a tendency VJP reads at its linearisation state ([ne][L] each): the
-// edge PV sum Q_e + P_e, the edge thickness flux F_e u_e and the flux-weighted
-// edges-on-edge sum sum_j w_ej F_j u_j.  A stage kernel that evaluates the
-// tendency at that state can write them (the adjoint's stage recomputation).
-struct PreOut {
-  Real *se, *fu, *own;
-};
 // Pattern-specialised kernels for the regular hexagonal mesh (kernels_hex.hip)
 bool hex_usable(const MeshView &m, const Launch &lc);
 // launch_tend_hex writes PreOut rows for this mesh, launch shape and
@@ -328,9 +328,10 @@ void launch_tend_hex(const MeshView &m, const Launch &lc, const ModelCoef &mc, c
 // Stage on the lattice mesh with uniform coefficients, without a diagnostics
 // launch (kernels_stage.hip): tendencies and stage update of every field.
 // emit: also write the stage input's diagnostics to d; d's momentum del4 rows
-// (vdel2_e, vdel4_e) are scratch in any case.
+// (vdel2_e, vdel4_e) are scratch in any case.  pre: also write the tendency
+// VJP's rows at the stage input (with emit).
 void launch_stage_hex(const MeshView &m, const Launch &lc, const HexCoef &q, const StageArgs &a,
-                      const DiagOut &d, bool emit, hipStream_t s);
+                      const DiagOut &d, bool emit, hipStream_t s, const PreOut *pre = nullptr);
 // y += alpha*x elementwise
 void launch_axpy(Real *y, Real alpha, const Real *x, size_t n, hipStream_t s);
 // y = x + alpha*z elementwise

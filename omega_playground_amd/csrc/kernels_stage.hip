@@ -24,6 +24,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N == 1
   stage_mom<N, V2, V4, EMIT>(p, xcd_entry(p.tiles));
 }
 
+// The same leaving the stage input's diagnostics and the rows its tendency
+// VJP reads (the adjoint's stage recomputation): 137 us at nx=256, 32 layers
+// with del2 viscosity, against 309 for a diagnostics and a tendency launch
+// that gather the stored rows (with the tracers, 47 us here).  Two levels per
+// lane spill up to 12 registers and are still the faster form (2.27 against
+// 2.34 ms per step adjoint).
+template <int N, bool V2, bool V4>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N == 1 ? 3 : 2)))
+    k_stage_mom_pre(StageLaunch p) {
+  stage_mom<N, V2, V4, true, true>(p, xcd_entry(p.tiles));
+}
+
 // Ensemble forms: entry b of n belongs to member who[b], whose parameter
 // block is read in place through scalar loads.
 template <int N, bool V2, bool EMIT>
@@ -81,6 +93,11 @@ using StageFn = void (*)(StageLaunch);
 template <int N, bool EMIT> StageFn pick_mom(bool v2, bool v4) {
   if (v4) return v2 ? k_stage_mom<N, true, true, EMIT> : k_stage_mom<N, false, true, EMIT>;
   return v2 ? k_stage_mom<N, true, false, EMIT> : k_stage_mom<N, false, false, EMIT>;
+}
+
+template <int N> StageFn pick_pre(bool v2, bool v4) {
+  if (v4) return v2 ? k_stage_mom_pre<N, true, true> : k_stage_mom_pre<N, false, true>;
+  return v2 ? k_stage_mom_pre<N, true, false> : k_stage_mom_pre<N, false, false>;
 }
 
 // without del4 there is no Laplacian to emit
@@ -159,9 +176,10 @@ void stage_launch(const MeshView &m, const Launch &lc, int N, const HexCoef &q, 
 }
 
 void launch_stage_hex(const MeshView &m, const Launch &lc, const HexCoef &q, const StageArgs &a,
-                      const DiagOut &d, bool emit, hipStream_t s) {
+                      const DiagOut &d, bool emit, hipStream_t s, const PreOut *pre) {
   TimerScope ts("tend", s);
   const int N = stage_levels(m, lc);
+  OMEGA_REQUIRE(!pre || emit, "stage launch: the VJP rows come with the diagnostics");
   StageLaunch p;
   TileLaunch t;
   stage_launch(m, lc, N, q, a, d, p, t);
@@ -180,9 +198,11 @@ void launch_stage_hex(const MeshView &m, const Launch &lc, const HexCoef &q, con
     p.x = d.vdel4_e;
   }
   const bool v2 = a.terms & T_VDEL2, d2 = a.terms & T_TDEL2, d4 = a.terms & T_TDEL4;
-  const StageFn k = N == 2 ? (emit ? pick_mom<2, true>(v2, v4) : pick_mom<2, false>(v2, v4))
-                           : (emit ? pick_mom<1, true>(v2, v4) : pick_mom<1, false>(v2, v4));
-  if (a.ntr > 0 && !v4 && launch_stage_both(N, m.tile.lx, p, t, emit, s)) return;
+  if (pre) p.pre = *pre;
+  const StageFn k = pre      ? (N == 2 ? pick_pre<2>(v2, v4) : pick_pre<1>(v2, v4))
+                    : N == 2 ? (emit ? pick_mom<2, true>(v2, v4) : pick_mom<2, false>(v2, v4))
+                             : (emit ? pick_mom<1, true>(v2, v4) : pick_mom<1, false>(v2, v4));
+  if (a.ntr > 0 && !v4 && launch_stage_both(N, m.tile.lx, p, t, emit, pre != nullptr, s)) return;
   hipLaunchKernelGGL(k, grid, block, 0, s, p);
   if (a.ntr > 0) {
     // one block takes all tracers of its tile, keeping the tile's thicknesses

@@ -9,39 +9,48 @@ namespace {
 
 using namespace stage;
 
-template <int N, int LX, int TW, int TH, bool V2, bool D2, bool D4, bool EMIT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N == 1 ? 4 : 2)))
+// what else a stage leaves: nothing, its input's diagnostics, or those and
+// the tendency VJP's rows
+enum Leave { kNothing, kDiag, kPre };
+
+template <int N, int LX, int TW, int TH, bool V2, bool D2, bool D4, Leave E>
+__global__ void __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu(N == 2 ? 2 : E == kPre ? 3 : 4)))
     k_stage_both(StageLaunch p, TileLaunch t) {
   const int b = (int)blockIdx.x;
   if (b < p.tiles) {
-    stage_mom<N, V2, false, EMIT>(p, b);
+    stage_mom<N, V2, false, E != kNothing, E == kPre>(p, b);
   } else {
     // tiles of all tracers of a group, then the next group
     const int w = b - p.tiles, group = uniform(w / t.work);
-    stage_tile<N, LX, TW, TH, D2, D4, EMIT>(t, w - group * t.work, group * t.per_block);
+    stage_tile<N, LX, TW, TH, D2, D4, E != kNothing>(t, w - group * t.work, group * t.per_block);
   }
 }
 
-template <int N, int LX, int TW, int TH, bool V2, bool EMIT> auto pick4(bool d2, bool d4) {
+template <int N, int LX, int TW, int TH, bool V2, Leave E> auto pick4(bool d2, bool d4) {
   if (d4)
-    return d2 ? k_stage_both<N, LX, TW, TH, V2, true, true, EMIT>
-              : k_stage_both<N, LX, TW, TH, V2, false, true, EMIT>;
-  return d2 ? k_stage_both<N, LX, TW, TH, V2, true, false, EMIT>
-            : k_stage_both<N, LX, TW, TH, V2, false, false, EMIT>;
+    return d2 ? k_stage_both<N, LX, TW, TH, V2, true, true, E>
+              : k_stage_both<N, LX, TW, TH, V2, false, true, E>;
+  return d2 ? k_stage_both<N, LX, TW, TH, V2, true, false, E>
+            : k_stage_both<N, LX, TW, TH, V2, false, false, E>;
 }
-template <int N, int LX, int TW, int TH> auto pick3(bool v2, bool d2, bool d4, bool emit) {
-  if (v2) return emit ? pick4<N, LX, TW, TH, true, true>(d2, d4) : pick4<N, LX, TW, TH, true, false>(d2, d4);
-  return emit ? pick4<N, LX, TW, TH, false, true>(d2, d4) : pick4<N, LX, TW, TH, false, false>(d2, d4);
+template <int N, int LX, int TW, int TH, Leave E> auto pick3(bool v2, bool d2, bool d4) {
+  return v2 ? pick4<N, LX, TW, TH, true, E>(d2, d4) : pick4<N, LX, TW, TH, false, E>(d2, d4);
 }
-template <int N> auto pick2(int lx, bool v2, bool d2, bool d4, bool emit) {
-  if (lx == 4) return pick3<N, 4, 8, 8>(v2, d2, d4, emit);
-  if (lx == 2) return pick3<N, 2, 16, 8>(v2, d2, d4, emit);
-  return pick3<N, 1, 16, 16>(v2, d2, d4, emit);
+template <int N, Leave E> auto pick2(int lx, bool v2, bool d2, bool d4) {
+  if (lx == 4) return pick3<N, 4, 8, 8, E>(v2, d2, d4);
+  if (lx == 2) return pick3<N, 2, 16, 8, E>(v2, d2, d4);
+  return pick3<N, 1, 16, 16, E>(v2, d2, d4);
+}
+template <int N> auto pick(int lx, bool v2, bool d2, bool d4, Leave e) {
+  return e == kPre    ? pick2<N, kPre>(lx, v2, d2, d4)
+         : e == kDiag ? pick2<N, kDiag>(lx, v2, d2, d4)
+                      : pick2<N, kNothing>(lx, v2, d2, d4);
 }
 
 } // namespace
 
-bool launch_stage_both(int N, int lx, const StageLaunch &p, const TileLaunch &t0, bool emit,
+bool launch_stage_both(int N, int lx, const StageLaunch &p, const TileLaunch &t0, bool emit, bool pre,
                        hipStream_t s) {
   const StageArgs &a = p.a;
   TileLaunch t = t0;
@@ -55,7 +64,8 @@ bool launch_stage_both(int N, int lx, const StageLaunch &p, const TileLaunch &t0
   // tracers miss the waves they have alone (142 -> 151 at 9216 cells).
   if (p.tiles + t.work * groups > (N == 2 ? 1024 : 2048)) return false;
   const bool v2 = a.terms & T_VDEL2, d2 = a.terms & T_TDEL2, d4 = a.terms & T_TDEL4;
-  hipLaunchKernelGGL(N == 2 ? pick2<2>(lx, v2, d2, d4, emit) : pick2<1>(lx, v2, d2, d4, emit),
+  const Leave e = pre ? kPre : emit ? kDiag : kNothing;
+  hipLaunchKernelGGL(N == 2 ? pick<2>(lx, v2, d2, d4, e) : pick<1>(lx, v2, d2, d4, e),
                      dim3(p.tiles + t.work * groups), dim3(256), 0, s, p, t);
   OMEGA_HIP_CHECK(hipGetLastError());
   return true;

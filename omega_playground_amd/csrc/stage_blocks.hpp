@@ -30,7 +30,7 @@ __device__ __forceinline__ bool stage_place(const StageLaunch &p, int entry, int
 // half busy, the rest latency), one level per lane at four waves 0.83 ms (the
 // same rows in twice the load instructions).
 // V4: subtract the del4 rows (p.x) the Laplacian launches left.
-template <int N, bool V2, bool V4, bool EMIT>
+template <int N, bool V2, bool V4, bool EMIT, bool PRE = false>
 __device__ __forceinline__ void stage_mom(const StageLaunch &p, int entry) {
   int c;
   Ctx x;
@@ -41,16 +41,30 @@ __device__ __forceinline__ void stage_mom(const StageLaunch &p, int entry) {
   load_cells(p.rec, c, id);
   const size_t idx = (size_t)c * L + k, e0 = (size_t)(3 * c) * L + k;
   MomOut<N> o;
-  momentum<N, V2>(p.q, x, id, a.h.in, a.vn.in, o);
-  if constexpr (EMIT) {
+  momentum<N, V2, PRE>(p.q, x, id, a.h.in, a.vn.in, o, [&](const MomOut<N> &o) {
+    if constexpr (EMIT) {
 #pragma unroll
-    for (int w = 0; w < 2; ++w) {
-      const size_t vi = (size_t)(2 * c + w) * L + k;
-      st<N>(p.d.rvort_v + vi, o.rv[w]);
-      st<N>(p.d.inv_thick_v + vi, o.it[w]);
+      for (int w = 0; w < 2; ++w) {
+        const size_t vi = (size_t)(2 * c + w) * L + k;
+        st<N>(p.d.rvort_v + vi, o.rv[w]);
+        st<N>(p.d.inv_thick_v + vi, o.it[w]);
+      }
     }
+    if constexpr (PRE) {
+#pragma unroll
+      for (int K = 0; K < 3; ++K) {
+        st<N>(p.pre.se + e0 + K * L, o.se[K]);
+        st<N>(p.pre.fu + e0 + K * L, o.fu[K]);
+      }
+    }
+  });
+  if constexpr (EMIT) {
     st<N>(p.d.ke_c + idx, o.ke);
     st<N>(p.d.div_c + idx, o.div);
+  }
+  if constexpr (PRE) {
+#pragma unroll
+    for (int K = 0; K < 3; ++K) st<N>(p.pre.own + e0 + K * L, o.own[K]);
   }
 #pragma unroll
   for (int K = 0; K < 3; ++K) {

@@ -17,6 +17,7 @@ struct StageLaunch {
   DiagOut d;
   const double *x; // momentum del4: the edge field a Laplacian launch reads
   double *y;       // and writes; the del4 term for the momentum launch
+  PreOut pre;      // rows for the tendency VJP at this stage input
 };
 
 // tracers: work = tiles * level chunks
@@ -39,7 +40,7 @@ constexpr int kFewTiles = 512;
 
 // Both in one launch, where that is the faster one (kernels_stage_both.hip);
 // false: nothing launched.
-bool launch_stage_both(int N, int lx, const StageLaunch &p, const TileLaunch &t, bool emit,
+bool launch_stage_both(int N, int lx, const StageLaunch &p, const TileLaunch &t, bool emit, bool pre,
                        hipStream_t s);
 
 // What one launch of an ensemble's members has compiled in; members that

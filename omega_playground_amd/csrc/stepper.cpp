@@ -193,9 +193,9 @@ void run_stage_into(omega_model_s *M, StageArgs a, hipStream_t s, int fields,
 // buffers (the per-field tendency calls after compute_aux).
 bool stage_writes_pre(omega_model_s *M) {
   const MeshView mv = M->view();
-  return (M->forms & 8) && !M->linear && !general_only(M) &&
-         !M->params.disable_vn_tendency && hex_usable(mv, M->lc) &&
-         hex_writes_pre(mv, M->lc, M->coef());
+  HexCoef q;
+  if (!(M->forms & 8) || M->linear || general_only(M) || M->params.disable_vn_tendency) return false;
+  return M->stage_coef(q) || (hex_usable(mv, M->lc) && hex_writes_pre(mv, M->lc, M->coef()));
 }
 
 void run_stage(omega_model_s *M, StageArgs a, hipStream_t s, int fields, bool with_diag,
@@ -211,12 +211,12 @@ void run_stage(omega_model_s *M, StageArgs a, hipStream_t s, int fields, bool wi
     return;
   }
   HexCoef q;
-  if (with_diag && !pre && fields == 7 && M->stage_coef(q)) {
+  if (with_diag && fields == 7 && M->stage_coef(q) && (!pre || emit)) {
     M->aux_h = a.h.in;
     M->aux_vn = a.vn.in;
     M->aux_tr = a.tr.in;
     if (M->terms & T_VDEL4) ensure_vdel4(M);
-    launch_stage_hex(mv, M->lc, q, a, M->diag(), emit, s);
+    launch_stage_hex(mv, M->lc, q, a, M->diag(), emit, s, pre);
     return;
   }
   if (with_diag && !pre && fields == 7 && mv.ccx && M->fh_e.p && a.do_h && a.do_vn) {

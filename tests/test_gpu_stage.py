@@ -174,3 +174,26 @@ def test_general_mesh_edge_means_bitwise(L, ntr, terms):
         st.run(0.0, DT, 2, s)
         po.Stepper(omodel, kind, 5).run(0.0, DT, 2, r)
         compare(s.download(), r, kind)
+
+
+@pytest.mark.parametrize("L,ntr", [(1, 1), (5, 2), (20, 1), (60, 0), (66, 3)])
+@pytest.mark.parametrize("terms", [7, 15, 79, 127])
+@pytest.mark.parametrize("kind", ["rk4", "lsrk"])
+def test_step_adjoint_rows_written_by_the_stage_kernels(kind, terms, L, ntr):
+    """Step adjoints whose stage recomputation writes the VJP's rows at any
+    layer count give the bits of the VJP's own pre-pass (forms 7)."""
+    print("case", kind, terms, L, ntr, flush=True)
+    om, omodel, gm, gmodel, state = make_pair(12, 10, L, ntr, seed=L)
+    gmodel.terms = terms
+    rng = np.random.default_rng(terms)
+    cot = tuple(rng.standard_normal(a.shape) for a in state)
+    got = []
+    for forms in (15, 7):
+        gmodel.set_kernel_forms(forms)
+        assert bool(gmodel.kernel_flags() & 16) == (forms == 15)
+        st = swe.RK4Stepper(gmodel) if kind == "rk4" else swe.LSRKStepper(gmodel, 5)
+        gc = upload(gm, ntr, cot)
+        gp = swe.step_vjp(st, 0.0, 30.0, upload(gm, ntr, state), gc)
+        got.append(list(gc.download()) + [gp])
+    for a, b in zip(*got):
+        assert same_bits(a, b)
