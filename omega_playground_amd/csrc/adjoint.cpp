@@ -242,10 +242,13 @@ void add_pgrad(omega_model_s *M, double *param_grad, hipStream_t s) {
 
 void copy_fields(Real *const dst[3], const Real *const src[3], const size_t n[3],
                  hipStream_t s) {
-  for (int f = 0; f < 3; ++f)
-    if (n[f])
-      OMEGA_HIP_CHECK(
-          hipMemcpyAsync(dst[f], src[f], n[f] * sizeof(Real), hipMemcpyDeviceToDevice, s));
+  FieldCopy c;
+  for (int f = 0; f < 3; ++f) {
+    c.src[f] = src[f];
+    c.dst[f] = dst[f];
+    c.n[f] = n[f];
+  }
+  launch_copy_fields(c, s);
 }
 
 void ensure_sized(DBuf<Real> (&b)[3], const size_t n[3]) {
@@ -524,8 +527,8 @@ void advance(omega_tape_s *T, omega_state_s *S, int from, int count, hipStream_t
   T->forward_steps += count;
 }
 
-void step_adjoint_at(omega_tape_s *T, omega_state_s *Y, omega_state_s *C, hipStream_t s) {
-  const auto y = state_ptrs(Y);
+// The step adjoint at y only reads y, so a stored state needs no copy for it.
+void step_adjoint_at(omega_tape_s *T, std::array<Real *, 3> y, omega_state_s *C, hipStream_t s) {
   const std::array<const Real *, 3> yc{y[0], y[1], y[2]};
   const auto c = state_ptrs(C);
   step_vjp_ptrs(T->stepper, yc.data(), c.data(), T->n, T->dt, s);
@@ -538,17 +541,13 @@ void step_adjoint_at(omega_tape_s *T, omega_state_s *Y, omega_state_s *C, hipStr
 void reverse_range(omega_tape_s *T, int a, int b, int sa, int c, bool desc, omega_state_s *C,
                    hipStream_t s) {
   omega_state_s *W = T->work.get();
-  if (b - a == 1) {
-    restore(T, sa, W, s);
-    step_adjoint_at(T, W, C, s);
-    return;
-  }
-  if (c <= 1) {
-    for (int i = b - 1; i >= a; --i) {
+  if (b - a == 1 || c <= 1) {
+    for (int i = b - 1; i > a; --i) {
       restore(T, sa, W, s);
       advance(T, W, a, i - a, s);
-      step_adjoint_at(T, W, C, s);
+      step_adjoint_at(T, state_ptrs(W), C, s);
     }
+    step_adjoint_at(T, slot_ptrs(T->slots[sa]), C, s);
     return;
   }
   const int m = revolve_split(b - a, c);

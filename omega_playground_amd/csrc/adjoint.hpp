@@ -129,6 +129,13 @@ int adj_partial_slots(const MeshView &m, const Launch &lc);
 
 // y[i] = v
 void launch_fill(Real *y, Real v, size_t n, hipStream_t s);
+// dst[f][i] = src[f][i] for three fields that do not overlap, on 16-byte boundaries
+struct FieldCopy {
+  const Real *src[3];
+  Real *dst[3];
+  size_t n[3];
+};
+void launch_copy_fields(const FieldCopy &c, hipStream_t s);
 // y = alpha*x + beta*z (y may alias x or z)
 void launch_lincomb(Real *y, Real alpha, const Real *x, Real beta, const Real *z, size_t n,
                     hipStream_t s);

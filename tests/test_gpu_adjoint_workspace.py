@@ -75,3 +75,24 @@ def test_ensemble_gradient_with_more_members_than_one_copy_launch():
                         tuple(x / 19 for x in (1.0, 0.0, 1.0)), n_snapshots=2)
         for x, y in zip(grads[m].download(), g.download()):
             assert same_bits(x, y), m
+
+
+@pytest.mark.parametrize("L,ntr,snaps", [(1, 0, 1), (3, 1, 2), (5, 4, 3), (16, 2, 6)])
+def test_window_gradient_is_the_chain_of_step_adjoints(L, ntr, snaps):
+    """Stored, restored and directly read checkpoints give the bits of step
+    adjoints at the states of a forward run, at odd sizes and without tracers."""
+    print("case", L, ntr, snaps, flush=True)
+    n, dt = 6, 30.0
+    mesh, pd, ((model, y0, obs),) = make_ensemble(M=1, L=L, ntr=ntr, n=n, dt=dt)
+    st = stepper(model, "rk4")
+    ys = [upload(mesh, ntr, y0) for _ in range(n + 1)]
+    for i, y in enumerate(ys):
+        if i:
+            st.run(0.0, dt, i, y)
+    cot = swe.ShallowWaterState(mesh, ntr)
+    J = swe.misfit(model, ys[n], obs, cot)
+    for y in reversed(ys[:n]):
+        swe.step_vjp(st, 0.0, dt, y, cot)
+    grad = swe.ShallowWaterState(mesh, ntr)
+    Jw, _ = swe.adjoint_run(st, 0.0, dt, n, upload(mesh, ntr, y0), obs, grad, n_snapshots=snaps)
+    assert J == Jw and all(same_bits(a, b) for a, b in zip(grad.download(), cot.download()))
