@@ -168,6 +168,7 @@ void ensure_adjoint(omega_model_s *M) {
     M->a_se.alloc(NE * L);
     M->a_fu.alloc(NE * L);
     M->a_px.alloc(NE * L);
+    if (dm.stage_ok) M->a_own.alloc(NE * L);
     if (ntr) M->a_xa.alloc(ntr * NE * L);
     M->a_sbar.alloc(NE * L);
     M->a_fbar.alloc(NE * L);
@@ -193,6 +194,27 @@ AdjScratch scratch(omega_model_s *M) {
                     M->a_se.p, M->a_fu.p, M->a_px.p, M->a_xa.p};
 }
 
+// Diagnostics and VJP rows at a state whose stage is not run, where one
+// launch of the stage kernels is the faster way to them; false: not done.
+bool run_rows(omega_model_s *M, const Real *h, const Real *vn, const Real *tr, hipStream_t s) {
+  HexCoef q;
+  if (!stage_writes_pre(M) || !M->stage_coef(q)) return false;
+  StageArgs a{};
+  a.terms = M->terms;
+  a.do_h = a.do_vn = 1;
+  a.ntr = M->params.ntracers;
+  a.h.in = h;
+  a.vn.in = vn;
+  a.tr.in = tr;
+  if (!launch_stage_rows(M->view(), M->lc, q, a, M->diag(),
+                         PreOut{M->a_se.p, M->a_fu.p, M->a_own.p}, s))
+    return false;
+  M->aux_h = h;
+  M->aux_vn = vn;
+  M->aux_tr = tr;
+  return true;
+}
+
 // out (+)= J(y)^T k for the tendency at state y (pointers in device numbering;
 // epi says how the result is combined);
 // the mixing-coefficient gradient accumulates in M->a_pgrad.
@@ -203,7 +225,8 @@ void tendency_vjp_ptrs(omega_model_s *M, const Real *const y[3], const Real *con
                        Real *const out[3], hipStream_t s, const AdjEpi &epi = AdjEpi{},
                        bool have_diag = false, const omega_model_s::PreSet *pre = nullptr,
                        int part = 0) {
-  if (!have_diag) run_diag(M, y[0], y[1], y[2], s);
+  const bool rows = !have_diag && run_rows(M, y[0], y[1], y[2], s);
+  if (!have_diag && !rows) run_diag(M, y[0], y[1], y[2], s);
   AdjArgs a{};
   a.terms = M->terms;
   a.do_h = !M->params.disable_h_tendency;
@@ -225,8 +248,9 @@ void tendency_vjp_ptrs(omega_model_s *M, const Real *const y[3], const Real *con
     sc.fu_e = pre->fu.p;
     sc.own_e = pre->own.p;
   }
+  if (rows) sc.own_e = M->a_own.p;
   launch_tendency_vjp(M->view(), M->mesh->adj.view(), M->lc, M->coef(), ac, a, M->diag(), sc,
-                      s, pre != nullptr);
+                      s, pre != nullptr || rows);
 }
 
 void zero_pgrad(omega_model_s *M, hipStream_t s) { launch_fill(M->a_pgrad.p, 0.0, 4, s); }

@@ -230,6 +230,7 @@ enum Epilogue : int {
   EPI_RK4_LAST = 3,  // y = acc + db*T
   EPI_LSRK = 4,      // tend = base + F; yout = yin + db*T
   EPI_PROVIS = 5,    // pout = yold + da*T (stage recomputation for the adjoint)
+  EPI_NONE = 6,      // nothing (stage kernels: their diagnostics alone)
 };
 
 // Buffers of one prognostic field (h, vn, or the tracer block) for a stage.
@@ -332,6 +333,10 @@ void launch_tend_hex(const MeshView &m, const Launch &lc, const ModelCoef &mc, c
 // VJP's rows at the stage input (with emit).
 void launch_stage_hex(const MeshView &m, const Launch &lc, const HexCoef &q, const StageArgs &a,
                       const DiagOut &d, bool emit, hipStream_t s, const PreOut *pre = nullptr);
+// The diagnostics and VJP rows at a state by the same kernels, where that is
+// faster than the diagnostics launch and the VJP's pre-pass; false: nothing launched.
+bool launch_stage_rows(const MeshView &m, const Launch &lc, const HexCoef &q, StageArgs a,
+                       const DiagOut &d, const PreOut &pre, hipStream_t s);
 // y += alpha*x elementwise
 void launch_axpy(Real *y, Real alpha, const Real *x, size_t n, hipStream_t s);
 // y = x + alpha*z elementwise

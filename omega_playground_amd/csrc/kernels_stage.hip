@@ -217,6 +217,28 @@ void launch_stage_hex(const MeshView &m, const Launch &lc, const HexCoef &q, con
   OMEGA_HIP_CHECK(hipGetLastError());
 }
 
+// The momentum body without its update: one launch instead of two, and the
+// adjoint's PV pass then reads the edges-on-edge sums instead of forming them
+// (step adjoint at nx=256, 64 layers, 1 tracer: 2286 -> 2272 us).  The tracers'
+// Laplacian comes along in the same launch (6-step gradient at 1920 cells, 20
+// layers: 1600 -> 1557 us) but is not worth a tile launch of its own.
+bool launch_stage_rows(const MeshView &m, const Launch &lc, const HexCoef &q, StageArgs a,
+                       const DiagOut &d, const PreOut &pre, hipStream_t s) {
+  a.epi = EPI_NONE;
+  a.base_from_tend = 0;
+  // only tracer del4 needs a diagnostic of the tracers
+  if (!(a.terms & T_TDEL4)) a.ntr = 0;
+  if (a.ntr > 0) {
+    StageLaunch p;
+    TileLaunch t;
+    const int N = stage_levels(m, lc);
+    stage_launch(m, lc, N, q, a, d, p, t);
+    if ((a.terms & T_VDEL4) || !stage_one_launch(N, p, t)) return false;
+  }
+  launch_stage_hex(m, lc, q, a, d, true, s, &pre);
+  return true;
+}
+
 void launch_stage_batch(const StageKind &k, const StageLaunch *desc, const int *who, int n, bool emit,
                         hipStream_t s) {
   TimerScope ts("batch_tend", s);

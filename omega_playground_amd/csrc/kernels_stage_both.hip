@@ -50,23 +50,34 @@ template <int N> auto pick(int lx, bool v2, bool d2, bool d4, Leave e) {
 
 } // namespace
 
+namespace {
+// blocks of the tracers: tiles times groups of per_block tracers
+int tile_blocks(const TileLaunch &t, int &per_block) {
+  per_block = t.work < kFewTiles ? 1 : t.per_block;
+  return t.work * ((t.a.ntr + per_block - 1) / per_block);
+}
+} // namespace
+
+// Both bodies hold the momentum's registers here: 2 blocks per CU with two
+// levels per lane, 4 with one, on 256 CUs.  Up to two rounds of those one
+// launch is faster (us per RK4 step, 64 layers, 1 tracer: 49 -> 37 at 576
+// cells, 74 -> 58 at 2304, 80 -> 80 at 4096 where it is two rounds; one
+// layer, 196608 cells, LSRK5: 97 -> 83 at one and a half), beyond them the
+// tracers miss the waves they have alone (142 -> 151 at 9216 cells).
+bool stage_one_launch(int N, const StageLaunch &p, const TileLaunch &t) {
+  int per_block;
+  return p.tiles + tile_blocks(t, per_block) <= (N == 2 ? 1024 : 2048);
+}
+
 bool launch_stage_both(int N, int lx, const StageLaunch &p, const TileLaunch &t0, bool emit, bool pre,
                        hipStream_t s) {
-  const StageArgs &a = p.a;
+  if (!stage_one_launch(N, p, t0)) return false;
   TileLaunch t = t0;
-  if (t.work < kFewTiles) t.per_block = 1;
-  const int groups = (a.ntr + t.per_block - 1) / t.per_block;
-  // Both bodies hold the momentum's registers here: 2 blocks per CU with two
-  // levels per lane, 4 with one, on 256 CUs.  Up to two rounds of those one
-  // launch is faster (us per RK4 step, 64 layers, 1 tracer: 49 -> 37 at 576
-  // cells, 74 -> 58 at 2304, 80 -> 80 at 4096 where it is two rounds; one
-  // layer, 196608 cells, LSRK5: 97 -> 83 at one and a half), beyond them the
-  // tracers miss the waves they have alone (142 -> 151 at 9216 cells).
-  if (p.tiles + t.work * groups > (N == 2 ? 1024 : 2048)) return false;
-  const bool v2 = a.terms & T_VDEL2, d2 = a.terms & T_TDEL2, d4 = a.terms & T_TDEL4;
+  const int blocks = p.tiles + tile_blocks(t0, t.per_block), terms = p.a.terms;
+  const bool v2 = terms & T_VDEL2, d2 = terms & T_TDEL2, d4 = terms & T_TDEL4;
   const Leave e = pre ? kPre : emit ? kDiag : kNothing;
   hipLaunchKernelGGL(N == 2 ? pick<2>(lx, v2, d2, d4, e) : pick<1>(lx, v2, d2, d4, e),
-                     dim3(p.tiles + t.work * groups), dim3(256), 0, s, p, t);
+                     dim3(blocks), dim3(256), 0, s, p, t);
   OMEGA_HIP_CHECK(hipGetLastError());
   return true;
 }

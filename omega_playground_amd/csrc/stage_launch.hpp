@@ -40,6 +40,7 @@ constexpr int kFewTiles = 512;
 
 // Both in one launch, where that is the faster one (kernels_stage_both.hip);
 // false: nothing launched.
+bool stage_one_launch(int N, const StageLaunch &p, const TileLaunch &t);
 bool launch_stage_both(int N, int lx, const StageLaunch &p, const TileLaunch &t, bool emit, bool pre,
                        hipStream_t s);
 

@@ -8,7 +8,7 @@ import pytest
 from oracle import pyoracle as po
 from omega_playground_amd import swe
 
-from helpers import same_bits
+from helpers import params_dict, rich_state, same_bits
 from test_gpu_parity import make_pair, upload
 
 pytestmark = pytest.mark.gpu
@@ -197,3 +197,32 @@ def test_step_adjoint_rows_written_by_the_stage_kernels(kind, terms, L, ntr):
         got.append(list(gc.download()) + [gp])
     for a, b in zip(*got):
         assert same_bits(a, b)
+
+
+@pytest.mark.parametrize("nx,ny,L,ntr", [(12, 10, 3, 1), (10, 8, 64, 0), (64, 64, 64, 1),
+                                         (64, 66, 64, 1), (16, 8, 20, 3)])
+def test_vjp_at_a_state_whose_stage_is_not_run(nx, ny, L, ntr):
+    """The tendency VJP gets its diagnostics and rows from the stage kernels
+    without a stage (with tracer del4 up to the sizes of one launch, with 64
+    layers and one tracer 4096 cells): the bits of the diagnostics launch and
+    the VJP's pre-pass (forms 7), and the same auxiliary state."""
+    mesh = swe.PlanarHexagonalMesh(nx, ny, 10e3, L)
+    model = swe.ShallowWaterModel(mesh, swe.ShallowWaterParams(**params_dict(10e3, ntr)))
+    state = rich_state(mesh, L, ntr, 3)
+    rng = np.random.default_rng(4)
+    cot, out = (tuple(rng.standard_normal(a.shape) for a in state) for _ in range(2))
+    for terms in (7, 15, 23, 79, 127):
+        print("case", nx, ny, L, ntr, terms, flush=True)
+        model.terms = terms
+        got = []
+        for forms in (15, 7):
+            model.set_kernel_forms(forms)
+            so, s = upload(mesh, ntr, out), upload(mesh, ntr, state)
+            gp = swe.tendency_vjp(model, s, upload(mesh, ntr, cot), so)
+            aux = [model.aux_array(n) for n in ("rvort_vertex", "inv_thick_vertex", "ke_cell",
+                                                "vel_div_cell")]
+            if terms & 64 and ntr:
+                aux.append(model.aux_array("tracer_del2_cell"))
+            got.append(list(so.download()) + [gp] + aux)
+        for a, b in zip(*got):
+            assert same_bits(a, b), terms
