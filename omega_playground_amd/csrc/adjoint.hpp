@@ -116,6 +116,7 @@ struct AdjArgs {
   // to reduce (no reduction launch); with either set the block sums carry
   // the vs scaling and the reduction adds them unscaled
   int part_add, part_keep;
+  int cells; // cells of a block in this pass, 0: one per row of lanes
 };
 
 // pre: se_e, fu_e and own_e of s already hold the rows at the linearisation

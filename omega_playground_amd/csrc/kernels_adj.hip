@@ -87,6 +87,11 @@ __device__ void block_partial(const AdjArgs &g, double a, double *out) {
   if (t == 0) put_partial(g, sa[0], out);
 }
 
+// The slot of a block whose term is off (no reduction).
+__device__ void no_partial(const AdjArgs &g, double *out) {
+  if (threadIdx.x == 0 && threadIdx.y == 0) put_partial(g, 0.0, out);
+}
+
 struct Seg {
   int c0, c1, k;
   bool active;
@@ -96,8 +101,11 @@ struct Seg {
 // as in the forward kernels: with a multiple of 8 chunks the chunk runs
 // fastest (XCD x handles chunks x, x + 8, ... of every cell block),
 // otherwise slowest with the optional swizzle over cell blocks.
-template <int N> __device__ __forceinline__ Seg segment(const MeshView &m, int swz) {
+// cells: cells of a block, 0 for one per row.
+template <int N>
+__device__ __forceinline__ Seg segment(const MeshView &m, int swz, int cells = 0) {
   Seg g;
+  if (!cells) cells = (int)blockDim.y;
   const int span = (int)blockDim.x * N;
   const int nch = (m.L + span - 1) / span;
   int s, ch;
@@ -113,8 +121,8 @@ template <int N> __device__ __forceinline__ Seg segment(const MeshView &m, int s
     ch = __builtin_amdgcn_readfirstlane(lb / ncb);
     s = lb - ch * ncb;
   }
-  g.c0 = s * (int)blockDim.y;
-  g.c1 = min(g.c0 + (int)blockDim.y, m.nc);
+  g.c0 = s * cells;
+  g.c1 = min(g.c0 + cells, m.nc);
   g.k = (ch * (int)blockDim.x + (int)threadIdx.x) * N;
   g.active = g.c0 < m.nc && g.k < m.L;
   return g;
@@ -327,7 +335,7 @@ template <int N, int H, int O = 0>
 __global__ void __launch_bounds__(kAB)
     k_adj_pv(MeshView m, AdjMeshView am, ModelCoef mc, AdjArgs a, DiagOut d, AdjScratch s,
              int swz) {
-  const Seg g = segment<N>(m, swz);
+  const Seg g = segment<N>(m, swz, a.cells);
   if (!g.active) return;
   const int L = m.L, k = g.k;
   for (int e = m.eofs[g.c0] + (int)threadIdx.y; e < m.eofs[g.c1]; e += blockDim.y) {
@@ -385,7 +393,7 @@ __global__ void __launch_bounds__(kAB)
   const bool do_vn = TM >= 0 || a.do_vn, do_h = TM >= 0 || a.do_h;
   (void)do_h;
   (void)do_vn;
-  const Seg g = segment<N>(m, swz);
+  const Seg g = segment<N>(m, swz, a.cells);
   const int L = m.L, k = g.k, NC = m.nc;
   const bool pv = do_vn && (terms & T_PV), vd2 = do_vn && (terms & T_VDEL2),
              vd4 = do_vn && (terms & T_VDEL4), ke = do_vn && (terms & T_KE);
@@ -444,7 +452,10 @@ __global__ void __launch_bounds__(kAB)
     });
   }
   const bool td4 = (terms & T_TDEL4) && a.ntr > 0;
-  for (int c = g.c0 + (int)threadIdx.y; g.active && c < g.c1; c += blockDim.y) {
+  // fewer cells than rows: on the rows that the vertices leave free
+  int row = (int)threadIdx.y;
+  if (a.cells) row = row < 2 * a.cells ? row + (int)blockDim.y - 2 * a.cells : row - 2 * a.cells;
+  for (int c = g.c0 + row; g.active && c < g.c1; c += blockDim.y) {
     Vd<N> kb = zero<N>(), db = zero<N>(), ds = zero<N>();
     const int n = H ? 6 : m.noc[c];
     int ec[6];
@@ -517,7 +528,8 @@ __global__ void __launch_bounds__(kAB)
     }
   }
   const int b = blockIdx.x;
-  block_partial(a, p_v2, s.partial + b);
+  if (vd2) block_partial(a, p_v2, s.partial + b);
+  else no_partial(a, s.partial + b);
 }
 
 // ---------------------------------------------------------------------------
@@ -533,7 +545,7 @@ __global__ void __launch_bounds__(kAB) __attribute__((amdgpu_waves_per_eu(4)))
   const bool do_vn = TM >= 0 || a.do_vn, do_h = TM >= 0 || a.do_h;
   (void)do_h;
   (void)do_vn;
-  const Seg g = segment<N>(m, swz);
+  const Seg g = segment<N>(m, swz, a.cells);
   const int L = m.L, k = g.k, NC = m.nc;
   const bool pv = do_vn && (terms & T_PV), vd2 = do_vn && (terms & T_VDEL2),
              vd4 = do_vn && (terms & T_VDEL4), ke = do_vn && (terms & T_KE);
@@ -643,7 +655,8 @@ __global__ void __launch_bounds__(kAB) __attribute__((amdgpu_waves_per_eu(4)))
     });
   }
   const int b = blockIdx.x;
-  block_partial(a, p_v4, s.partial + a.nparts + b);
+  if (vd4) block_partial(a, p_v4, s.partial + a.nparts + b);
+  else no_partial(a, s.partial + a.nparts + b);
 }
 
 // ---------------------------------------------------------------------------
@@ -847,7 +860,13 @@ __global__ void __launch_bounds__(kAB)
     }
   }
   const int b = blockIdx.x;
-  block_partials2(a, p_t2, p_t4, s.partial + 2 * a.nparts + b, s.partial + 3 * a.nparts + b);
+  double *const t2 = s.partial + 2 * a.nparts + b, *const t4 = t2 + a.nparts;
+  if (td2 || td4) {
+    block_partials2(a, p_t2, p_t4, t2, t4);
+  } else {
+    no_partial(a, t2);
+    no_partial(a, t4);
+  }
 }
 
 // pgrad[p] += sum of the block partials of parameter p, in a fixed order
@@ -869,6 +888,8 @@ __global__ void __launch_bounds__(kAB) k_adj_param_reduce(double *partial, int n
 struct AGeo {
   dim3 grid, block;
   int N;
+  int cells; // cells of a block of the edge and vertex passes (AdjArgs::cells)
+  dim3 egrid; // and their grid
 };
 
 AGeo adj_geometry(const MeshView &m, const Launch &lc) {
@@ -879,14 +900,25 @@ AGeo adj_geometry(const MeshView &m, const Launch &lc) {
   while (lx < lanes) lx <<= 1;
   const int rows = kAB / lx;
   const int chunks = (m.L + lx * N - 1) / (lx * N);
-  return AGeo{dim3((m.nc + rows - 1) / rows * chunks), dim3(lx, rows), N};
+  const int blocks = (m.nc + rows - 1) / rows * chunks;
+  // Where the blocks hardly cover the 256 CUs, a thread's three edges (two
+  // vertices and a cell) in a row are what a pass waits for, so a block takes
+  // a third of the cells and each thread one edge, vertex or cell (us per step
+  // adjoint, 64 layers, 2 tracers: 207 -> 168 at 256 cells, 220 -> 189 at
+  // 1024, 269 -> 263 at 2304; 20 layers, 2304 cells: 218 -> 190; one layer,
+  // 65536 cells: 288 -> 268).  From 1.25 blocks per CU on the sharing of rows
+  // within a block weighs as much (292 -> 289 at 338 blocks, 300 -> 303 at
+  // 392, 321 -> 329 at 450).
+  const int cells = blocks <= 320 ? rows / 3 : 0;
+  return AGeo{dim3(blocks), dim3(lx, rows), N, cells,
+              dim3(cells ? (m.nc + cells - 1) / cells * chunks : blocks)};
 }
 
 } // namespace
 
 int adj_partial_slots(const MeshView &m, const Launch &lc) {
   const AGeo g = adj_geometry(m, lc);
-  return (int)(g.grid.x * g.grid.y);
+  return (int)g.egrid.x; // the larger grid
 }
 
 // ---------------------------------------------------------------------------
@@ -1011,10 +1043,13 @@ void launch_sum(const Real *partial, int n, Real *out, int accumulate, hipStream
 }
 
 void launch_tendency_vjp(const MeshView &m, const AdjMeshView &am, const Launch &lc,
-                         const ModelCoef &mc, const AdjCoef &ac, const AdjArgs &a,
+                         const ModelCoef &mc, const AdjCoef &ac, const AdjArgs &args,
                          const DiagOut &d, const AdjScratch &s, hipStream_t st, bool pre) {
   TimerScope ts("adjoint", st);
   const AGeo g = adj_geometry(m, lc);
+  AdjArgs a = args;
+  dim3 grid = g.grid;
+  a.cells = 0;
   const int swz = lc.swizzle;
   const bool vd4 = a.do_vn && (a.terms & T_VDEL4);
   const bool pv = a.do_vn && (a.terms & T_PV);
@@ -1029,34 +1064,34 @@ void launch_tendency_vjp(const MeshView &m, const AdjMeshView &am, const Launch 
 #define OMEGA_ADJ_LAUNCH(K, ...)                                                                \
   do {                                                                                         \
     if (tm == 7)                                                                               \
-      hipLaunchKernelGGL((K<2, 1, 1, 7>), g.grid, g.block, 0, st, __VA_ARGS__);                 \
+      hipLaunchKernelGGL((K<2, 1, 1, 7>), grid, g.block, 0, st, __VA_ARGS__);                 \
     else if (tm == 15)                                                                         \
-      hipLaunchKernelGGL((K<2, 1, 1, 15>), g.grid, g.block, 0, st, __VA_ARGS__);                \
+      hipLaunchKernelGGL((K<2, 1, 1, 15>), grid, g.block, 0, st, __VA_ARGS__);                \
     else if (tm == 79)                                                                         \
-      hipLaunchKernelGGL((K<2, 1, 1, 79>), g.grid, g.block, 0, st, __VA_ARGS__);                \
+      hipLaunchKernelGGL((K<2, 1, 1, 79>), grid, g.block, 0, st, __VA_ARGS__);                \
     else if (tm == 127)                                                                        \
-      hipLaunchKernelGGL((K<2, 1, 1, 127>), g.grid, g.block, 0, st, __VA_ARGS__);               \
+      hipLaunchKernelGGL((K<2, 1, 1, 127>), grid, g.block, 0, st, __VA_ARGS__);               \
     else if (U)                                                                                \
-      hipLaunchKernelGGL((K<2, 1, 1>), g.grid, g.block, 0, st, __VA_ARGS__);                    \
+      hipLaunchKernelGGL((K<2, 1, 1>), grid, g.block, 0, st, __VA_ARGS__);                    \
     else if (g.N == 2 && am.fixed)                                                             \
-      hipLaunchKernelGGL((K<2, 1, 0>), g.grid, g.block, 0, st, __VA_ARGS__);                    \
+      hipLaunchKernelGGL((K<2, 1, 0>), grid, g.block, 0, st, __VA_ARGS__);                    \
     else if (g.N == 2)                                                                         \
-      hipLaunchKernelGGL((K<2, 0, 0>), g.grid, g.block, 0, st, __VA_ARGS__);                    \
+      hipLaunchKernelGGL((K<2, 0, 0>), grid, g.block, 0, st, __VA_ARGS__);                    \
     else if (am.fixed)                                                                         \
-      hipLaunchKernelGGL((K<1, 1, 0>), g.grid, g.block, 0, st, __VA_ARGS__);                    \
+      hipLaunchKernelGGL((K<1, 1, 0>), grid, g.block, 0, st, __VA_ARGS__);                    \
     else                                                                                       \
-      hipLaunchKernelGGL((K<1, 0, 0>), g.grid, g.block, 0, st, __VA_ARGS__);                    \
+      hipLaunchKernelGGL((K<1, 0, 0>), grid, g.block, 0, st, __VA_ARGS__);                    \
   } while (0)
 #define OMEGA_ADJ_LAUNCH2(K, ...)                                                               \
   do {                                                                                         \
     if (g.N == 2 && am.fixed)                                                                  \
-      hipLaunchKernelGGL((K<2, 1>), g.grid, g.block, 0, st, __VA_ARGS__);                       \
+      hipLaunchKernelGGL((K<2, 1>), grid, g.block, 0, st, __VA_ARGS__);                       \
     else if (g.N == 2)                                                                         \
-      hipLaunchKernelGGL((K<2, 0>), g.grid, g.block, 0, st, __VA_ARGS__);                       \
+      hipLaunchKernelGGL((K<2, 0>), grid, g.block, 0, st, __VA_ARGS__);                       \
     else if (am.fixed)                                                                         \
-      hipLaunchKernelGGL((K<1, 1>), g.grid, g.block, 0, st, __VA_ARGS__);                       \
+      hipLaunchKernelGGL((K<1, 1>), grid, g.block, 0, st, __VA_ARGS__);                       \
     else                                                                                       \
-      hipLaunchKernelGGL((K<1, 0>), g.grid, g.block, 0, st, __VA_ARGS__);                       \
+      hipLaunchKernelGGL((K<1, 0>), grid, g.block, 0, st, __VA_ARGS__);                       \
   } while (0)
   if (vd4) {
     OMEGA_ADJ_LAUNCH2(k_adj_v4a, m, mc, a, s, swz);
@@ -1065,16 +1100,18 @@ void launch_tendency_vjp(const MeshView &m, const AdjMeshView &am, const Launch 
   // edge PV sums (PV term) and thickness fluxes (PV term, tracer advection),
   // unless the stage kernel at this state wrote them
   if (!pre && (pv || a.ntr > 0)) OMEGA_ADJ_LAUNCH(k_adj_pre, m, mc, a, d, s, swz);
+  grid = g.egrid;
+  a.cells = g.cells;
   if (pv && pre) {
     OMEGA_REQUIRE(s.own_e != nullptr, "tendency VJP: pre rows without the edges-on-edge sum");
     if (g.N == 2 && am.fixed)
-      hipLaunchKernelGGL((k_adj_pv<2, 1, 1>), g.grid, g.block, 0, st, m, am, mc, a, d, s, swz);
+      hipLaunchKernelGGL((k_adj_pv<2, 1, 1>), grid, g.block, 0, st, m, am, mc, a, d, s, swz);
     else if (g.N == 2)
-      hipLaunchKernelGGL((k_adj_pv<2, 0, 1>), g.grid, g.block, 0, st, m, am, mc, a, d, s, swz);
+      hipLaunchKernelGGL((k_adj_pv<2, 0, 1>), grid, g.block, 0, st, m, am, mc, a, d, s, swz);
     else if (am.fixed)
-      hipLaunchKernelGGL((k_adj_pv<1, 1, 1>), g.grid, g.block, 0, st, m, am, mc, a, d, s, swz);
+      hipLaunchKernelGGL((k_adj_pv<1, 1, 1>), grid, g.block, 0, st, m, am, mc, a, d, s, swz);
     else
-      hipLaunchKernelGGL((k_adj_pv<1, 0, 1>), g.grid, g.block, 0, st, m, am, mc, a, d, s, swz);
+      hipLaunchKernelGGL((k_adj_pv<1, 0, 1>), grid, g.block, 0, st, m, am, mc, a, d, s, swz);
   } else if (pv) {
     OMEGA_ADJ_LAUNCH2(k_adj_pv, m, am, mc, a, d, s, swz);
   }
@@ -1084,25 +1121,30 @@ void launch_tendency_vjp(const MeshView &m, const AdjMeshView &am, const Launch 
 #define OMEGA_ADJ_LAUNCH_X(K, X, TA, TB, ...)                                                   \
   do {                                                                                         \
     if (tm == TA)                                                                              \
-      hipLaunchKernelGGL((K<2, 1, X, 1, TA>), g.grid, g.block, 0, st, __VA_ARGS__);             \
+      hipLaunchKernelGGL((K<2, 1, X, 1, TA>), grid, g.block, 0, st, __VA_ARGS__);             \
     else if (tm == TB)                                                                         \
-      hipLaunchKernelGGL((K<2, 1, X, 1, TB>), g.grid, g.block, 0, st, __VA_ARGS__);             \
+      hipLaunchKernelGGL((K<2, 1, X, 1, TB>), grid, g.block, 0, st, __VA_ARGS__);             \
     else if (U)                                                                                \
-      hipLaunchKernelGGL((K<2, 1, X, 1>), g.grid, g.block, 0, st, __VA_ARGS__);                 \
+      hipLaunchKernelGGL((K<2, 1, X, 1>), grid, g.block, 0, st, __VA_ARGS__);                 \
     else if (g.N == 2 && am.fixed)                                                             \
-      hipLaunchKernelGGL((K<2, 1, X, 0>), g.grid, g.block, 0, st, __VA_ARGS__);                 \
+      hipLaunchKernelGGL((K<2, 1, X, 0>), grid, g.block, 0, st, __VA_ARGS__);                 \
     else if (g.N == 2)                                                                         \
-      hipLaunchKernelGGL((K<2, 0, X, 0>), g.grid, g.block, 0, st, __VA_ARGS__);                 \
+      hipLaunchKernelGGL((K<2, 0, X, 0>), grid, g.block, 0, st, __VA_ARGS__);                 \
     else if (am.fixed)                                                                         \
-      hipLaunchKernelGGL((K<1, 1, X, 0>), g.grid, g.block, 0, st, __VA_ARGS__);                 \
+      hipLaunchKernelGGL((K<1, 1, X, 0>), grid, g.block, 0, st, __VA_ARGS__);                 \
     else                                                                                       \
-      hipLaunchKernelGGL((K<1, 0, X, 0>), g.grid, g.block, 0, st, __VA_ARGS__);                 \
+      hipLaunchKernelGGL((K<1, 0, X, 0>), grid, g.block, 0, st, __VA_ARGS__);                 \
   } while (0)
   if (a.terms & (T_TDEL2 | T_TDEL4)) {
     OMEGA_ADJ_LAUNCH_X(k_adj_edge, 1, 79, 127, m, am, mc, ac, a, d, s, swz);
-    OMEGA_ADJ_LAUNCH_X(k_adj_cell, 1, 79, 127, m, am, mc, ac, a, d, s, swz);
   } else {
     OMEGA_ADJ_LAUNCH_X(k_adj_edge, 0, 7, 15, m, am, mc, ac, a, d, s, swz);
+  }
+  grid = g.grid;
+  a.cells = 0;
+  if (a.terms & (T_TDEL2 | T_TDEL4)) {
+    OMEGA_ADJ_LAUNCH_X(k_adj_cell, 1, 79, 127, m, am, mc, ac, a, d, s, swz);
+  } else {
     OMEGA_ADJ_LAUNCH_X(k_adj_cell, 0, 7, 15, m, am, mc, ac, a, d, s, swz);
   }
 #undef OMEGA_ADJ_LAUNCH_X
@@ -1110,7 +1152,7 @@ void launch_tendency_vjp(const MeshView &m, const AdjMeshView &am, const Launch 
 #undef OMEGA_ADJ_LAUNCH
   if (!a.part_keep)
     hipLaunchKernelGGL(k_adj_param_reduce, dim3(4), dim3(kAB), 0, st, s.partial, a.nparts,
-                       (int)(g.grid.x * g.grid.y), a.part_add ? 1.0 : a.epi.vs, s.pgrad);
+                       (int)g.egrid.x, a.part_add ? 1.0 : a.epi.vs, s.pgrad);
   OMEGA_HIP_CHECK(hipGetLastError());
 }
 

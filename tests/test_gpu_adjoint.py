@@ -703,3 +703,29 @@ def test_step_vjp_without_coefficient_read_back():
         outs.append(gc.download())
     for name, a, b in zip(("h", "vn", "tr"), *outs):
         assert same_bits(a, b), name
+
+
+@pytest.mark.parametrize("many,few", [(64, 4), (65, 5), (66, 20)])
+@pytest.mark.parametrize("forms", [15, 0])
+def test_vjp_of_some_layers_alone(many, few, forms):
+    """The passes give a thread one edge, vertex or cell where the blocks are
+    few and three edges in a row where they are many: the first layers of a
+    model of many give the bits they give alone (no operator couples layers)."""
+    def run(L):
+        mesh = swe.PlanarHexagonalMesh(40, 66, 10e3, L)
+        model = swe.ShallowWaterModel(mesh, swe.ShallowWaterParams(**params_dict(10e3, 2)))
+        model.set_kernel_forms(forms)
+        state = tuple(a[..., :L].copy() for a in full)
+        cot = tuple(a[..., :L].copy() for a in cots)
+        out = swe.ShallowWaterState(mesh, 2)
+        swe.tendency_vjp(model, upload(mesh, 2, state), upload(mesh, 2, cot), out)
+        gc = upload(mesh, 2, cot)
+        swe.step_vjp(swe.LSRKStepper(model, 5), 0.0, 30.0, upload(mesh, 2, state), gc)
+        return list(out.download()) + list(gc.download())
+
+    print("case", many, few, forms, flush=True)
+    full = rich_state(swe.PlanarHexagonalMesh(40, 66, 10e3, many), many, 2, 1)
+    rng = np.random.default_rng(2)
+    cots = tuple(rng.standard_normal(a.shape) for a in full)
+    for a, b in zip(run(many), run(few)):
+        assert same_bits(np.ascontiguousarray(a[..., :few]), b)
