@@ -36,14 +36,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N == 1
   stage_mom<N, V2, V4, true, true>(p, xcd_entry(p.tiles));
 }
 
-// Ensemble forms: entry b of n belongs to member who[b], whose parameter
-// block is read in place through scalar loads.
+// Ensemble forms: block b belongs to member who[b] (-1: none), whose parameter
+// block is read in place through scalar loads and whose blocks start at a
+// multiple of 8, so that each XCD takes a contiguous eighth of every member.
 template <int N, bool V2, bool EMIT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N == 1 ? 4 : 2)))
-    k_batch_mom(const StageLaunch *__restrict__ desc, const int *__restrict__ who, int n) {
-  const int b = xcd_entry(n);
-  const StageLaunch &p = desc[uniform(who[b])];
-  stage_mom<N, V2, false, EMIT>(p, b - p.block0);
+    k_batch_mom(const StageLaunch *__restrict__ desc, const int *__restrict__ who) {
+  const int w = uniform(who[blockIdx.x]);
+  if (w < 0) return;
+  const StageLaunch &p = desc[w];
+  stage_mom<N, V2, false, EMIT>(p, logical_block((int)blockIdx.x - p.block0, p.tiles, 1));
 }
 
 // The edge Laplacian: of the velocity (FINAL false), then of that result,
@@ -82,10 +84,11 @@ __global__ void __launch_bounds__(LX *TW *TH) __attribute__((amdgpu_waves_per_eu
 
 template <int N, int LX, int TW, int TH, bool D2, bool D4, bool EMIT>
 __global__ void __launch_bounds__(LX *TW *TH) __attribute__((amdgpu_waves_per_eu(N == 2 ? 3 : 4)))
-    k_batch_tile(const TileLaunch *__restrict__ desc, const int *__restrict__ who, int n) {
-  const int b = xcd_entry(n);
-  const TileLaunch &p = desc[uniform(who[b])];
-  stage_tile<N, LX, TW, TH, D2, D4, EMIT>(p, b - p.block0, 0);
+    k_batch_tile(const TileLaunch *__restrict__ desc, const int *__restrict__ who) {
+  const int w = uniform(who[blockIdx.x]);
+  if (w < 0) return;
+  const TileLaunch &p = desc[w];
+  stage_tile<N, LX, TW, TH, D2, D4, EMIT>(p, logical_block((int)blockIdx.x - p.block0, p.work, 1), 0);
 }
 
 using StageFn = void (*)(StageLaunch);
@@ -243,7 +246,7 @@ void launch_stage_batch(const StageKind &k, const StageLaunch *desc, const int *
                         hipStream_t s) {
   TimerScope ts("batch_tend", s);
   hipLaunchKernelGGL(k.N == 2 ? pick_batch_mom<2>(k.v2, emit) : pick_batch_mom<1>(k.v2, emit),
-                     dim3(n), dim3(256), 0, s, desc, who, n);
+                     dim3(n), dim3(256), 0, s, desc, who);
   OMEGA_HIP_CHECK(hipGetLastError());
 }
 
@@ -251,7 +254,7 @@ void launch_tile_batch(const StageKind &k, const TileLaunch *desc, const int *wh
                        hipStream_t s) {
   TimerScope ts("batch_tracers", s);
   hipLaunchKernelGGL(pick_tile<true>(k.N, k.lx, k.d2, k.d4, emit), dim3(n), dim3(kTileThreads), 0, s,
-                     desc, who, n);
+                     desc, who);
   OMEGA_HIP_CHECK(hipGetLastError());
 }
 

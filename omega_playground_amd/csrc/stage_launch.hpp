@@ -12,7 +12,7 @@ struct StageLaunch {
   HexCoef q;
   const int *rec; // neighbourhood records
   int nc, L, lx, rows, ncb, tiles;
-  int block0; // first entry in an ensemble's launch
+  int block0; // first block in an ensemble's launch
   StageArgs a;
   DiagOut d;
   const double *x; // momentum del4: the edge field a Laplacian launch reads
@@ -53,8 +53,8 @@ struct StageKind {
     return N == o.N && lx == o.lx && v2 == o.v2 && d2 == o.d2 && d4 == o.d4;
   }
 };
-// One launch over n entries; entry b belongs to member who[b], whose
-// parameter block is desc[who[b]].
+// One launch of n blocks; block b belongs to the member with parameter block
+// desc[who[b]], to none if that is negative.
 void launch_stage_batch(const StageKind &k, const StageLaunch *desc, const int *who, int n, bool emit,
                         hipStream_t s);
 void launch_tile_batch(const StageKind &k, const TileLaunch *desc, const int *who, int n, bool emit,
