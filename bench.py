@@ -563,10 +563,10 @@ def main():
     avg_tend_ms = tend_ms / max(tend_n, 1)
     avg_diag_ms = diag_ms / max(diag_n, 1)
     B = alg_bytes_per_cell_layer_step(ntr, cfg["stepper"])
-    # one RK stage is the unit of launch: its diagnostics launch and its fused
-    # tendency + update launch carry the stage's share of B_alg (a quarter of
-    # the step's for RK4); the headline roofline charges those bytes to the
-    # two kernels' summed average durations
+    # one RK stage is the unit: its launches (momentum and thickness, tracers;
+    # with stored diagnostics a diagnostics launch before) carry the stage's
+    # share of B_alg (a quarter of the step's for RK4); the headline roofline
+    # charges those bytes to their summed average durations
     nlaunch = 4 if cfg["stepper"] == "rk4" else 5
     alg_bytes_launch = B * nc * L / nlaunch
     stage_ms = avg_tend_ms + avg_diag_ms
@@ -634,12 +634,10 @@ def main():
 
     workload_key = f"{args.config}:{args.ordering}:" + ",".join(str(x) for x in model.get_launch())
     traffic = load_traffic("tend", workload_key)
-    dtraffic = load_traffic("diag", workload_key)
-    # measured HBM bytes per stage (rocprofv3 FETCH_SIZE + WRITE_SIZE of both
-    # kernels, committed in profiles/traffic.json) over this run's durations
-    stage_traffic = None
-    if traffic and dtraffic:
-        stage_traffic = traffic["bytes_per_launch"] + dtraffic["bytes_per_launch"]
+    # measured HBM bytes per stage (rocprofv3 FETCH_SIZE + WRITE_SIZE of its
+    # kernels, committed in profiles/traffic.json) over this run's durations;
+    # recorded for the stage kernels, which have no diagnostics launch
+    stage_traffic = traffic["bytes_per_launch"] if traffic and not diag_n else None
     traffic_gbs = stage_traffic / (stage_ms * 1e-3) / 1e9 if stage_traffic else None
     step_traffic_gbs = nlaunch * stage_traffic / (ms_per_step * 1e-3) / 1e9 \
         if stage_traffic else None
@@ -671,8 +669,11 @@ def main():
                                        "WRITE_SIZE; scaled by a plain copy), measured at "
                                        f"launch {traffic['launch']}"
                      if stage_traffic else None,
-                     "kernel": "one RK stage: k_diag (diagnostics) + k_tend (fused tendency + "
-                               "RK4 stage update)",
+                     "kernel": "one RK stage: "
+                               + ("k_diag (diagnostics) + k_tend (fused tendency + RK4 stage "
+                                  "update)" if diag_n else
+                                  "k_stage_mom (momentum, thickness) + k_stage_tile (tracers), "
+                                  "diagnostics in registers, RK4 stage update fused"),
                      "stage_avg_ms": stage_ms,
                      "alg_bytes_per_launch": alg_bytes_launch,
                      "traffic_GBs": traffic_gbs,
@@ -680,9 +681,9 @@ def main():
                      "kernels": {
                          "tend": {"avg_ms": avg_tend_ms, "launches": tend_n,
                                   "alg_frac_if_charged_alone": tend_only / HBM_PEAK_GBS,
-                                  "traffic": traffic["bytes_per_launch"] if traffic else None},
+                                  "traffic": stage_traffic},
                          "diag": {"avg_ms": avg_diag_ms, "launches": diag_n,
-                                  "traffic": dtraffic["bytes_per_launch"] if dtraffic else None}}},
+                                  "traffic": None}}},
         "step_roofline": {"B_alg_per_cell_layer_step": B, "achieved_GBs": step_achieved,
                           "frac": step_achieved / HBM_PEAK_GBS, "diag_kernel_avg_ms": avg_diag_ms,
                           "traffic_GBs": step_traffic_gbs,
