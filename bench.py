@@ -8,9 +8,9 @@ balance, momentum del2 viscosity 1e3 m^2/s, tracer del4 1e9 m^4/s, the step
 captured in a HIP graph.  A step is one full RK4 step (4 tendency
 evaluations + stage updates); the metric counts cell-layer-steps/s.
 
-Prints one JSON line.  `roofline` is measured on one RK stage (its
-diagnostics launch and its fused tendency + stage-update launch) with HIP
-events on their launch stream: the stage's algorithmic bytes over the two
+Prints one JSON line.  `roofline` is measured on one RK stage (its momentum
+and tracer launches, or its diagnostics and tendency launches) with HIP
+events on their launch stream: the stage's algorithmic bytes over the
 kernels' summed average durations; `step_roofline` is the same bytes over
 the whole graph-replayed step.  `cpu_baseline` times the CPU oracle (OpenMP,
 the job's cores, spread binding) on a bounded sample of the same workload.

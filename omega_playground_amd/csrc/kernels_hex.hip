@@ -1,4 +1,9 @@
-// Pattern-specialised forward kernels for the regular hexagonal mesh.
+// Pattern-specialised forward kernels for the regular hexagonal mesh, with
+// stored diagnostics: what the stage kernels (kernels_stage.hip) do not take,
+// such as lattices that close with a shift, models with a tendency or a basic
+// term off, single-field tendencies, and a scratch evaluation with momentum
+// del4.  Times at nx=512, 64 layers: 0.55 ms diagnostics and 1.82 ms tendency
+// per stage, against 1.55 ms for the stage kernels.
 //
 // Each lane carries N consecutive levels of one entity (N = 2: one 16-byte
 // load per lane and row, 32 lanes per 64-level row, two entities per
