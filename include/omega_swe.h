@@ -338,8 +338,9 @@ int omega_model_kernel_variant(omega_model_t model, int *in_use);
 /* Forms of the two-cells-per-wavefront kernels this model runs: bit 0 set
  * when every coefficient table (mesh and model) is bit-identical at each
  * stencil slot, so a wavefront's two cells share one scalar read of each;
- * bit 1 set when all [rows][levels] arrays have < 2^24 rows and < 4 GiB,
- * so row addresses are 32-bit offsets from the array base; bit 2 set when
+ * bit 1 set when all [rows][levels] arrays have < 2^24 rows, each < 2^24
+ * bytes, and < 4 GiB, so row addresses are 32-bit offsets from the array
+ * base; bit 2 set when
  * the tendency VJP runs its slot-uniform form (regular hexagonal
  * numbering, an even layer count, every adjoint table bit-identical at
  * each stencil slot; known after the model's first adjoint call); bit 3

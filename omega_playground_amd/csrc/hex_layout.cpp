@@ -157,6 +157,8 @@ void build_hex_stage(DeviceMesh &dm) {
   const HostMesh &m = dm.host;
   const int NC = m.ncells, ME = m.max_edges;
   if (!dm.hex_ok || !dm.coef_uni || !dm.off32 || dm.me2 != hex::kSlots) return;
+  // a cell's three edge rows are one 24-bit factor of the velocities' offsets
+  if (3 * (size_t)m.nlayers * sizeof(double) >= size_t(1) << 24) return;
   namespace hl = hexl;
   HexCoef &q = dm.stage_coef;
   const double C = dm.cdiv_h[3], ke = dm.cke_h[0], R = dm.crv_h[0], th = dm.cth_h[0];

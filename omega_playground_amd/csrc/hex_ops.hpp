@@ -20,10 +20,10 @@ template <int N> __device__ __forceinline__ int ent(int x) {
 }
 
 // Row e of a [rows][L] array at levels k..k+N-1.  W = false when every
-// array the kernel reads has fewer than 2^24 rows and is below 4 GiB
-// (MeshView::off32, checked on the host): the address is then the array's
-// uniform base plus one 32-bit lane offset (one 24-bit multiply-add instead
-// of 64-bit index arithmetic).
+// array the kernel reads has fewer than 2^24 rows of less than 2^24 bytes and
+// is below 4 GiB (MeshView::off32, checked on the host): the address is then
+// the array's uniform base plus one 32-bit lane offset (one 24-bit
+// multiply-add instead of 64-bit index arithmetic).
 template <int N, bool W = true>
 __device__ __forceinline__ Vd<N> rowv(const double *__restrict__ p, int e, int L, int k) {
   if (W) return ld<N>(p + (size_t)e * L + k);

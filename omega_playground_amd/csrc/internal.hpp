@@ -130,7 +130,8 @@ struct MeshView {
   int hex_ok, hexu_ok, hexd_ok;
   // coef_uni: the mesh's coefficient tables (inv_dc, inv_dv, maxlev_e, s2,
   // s4, w, cdiv, cke, crv, cth) are equal at every stencil slot, bit for
-  // bit; off32: every [rows][L] array has < 2^24 rows and < 4 GiB
+  // bit; off32: every [rows][L] array has < 2^24 rows, each < 2^24
+  // bytes, and < 4 GiB
   int coef_uni, off32;
   // the pair tendency kernel may use its compiled-in term sets (cleared by
   // a model's kernel forms for tests)
@@ -175,7 +176,8 @@ struct DeviceMesh {
   bool hex_ok = false;
   bool hexu_ok = false; // per-cell union records valid (hexu)
   bool coef_uni = false; // coefficient tables equal at every stencil slot
-  bool off32 = false;    // 32-bit byte offsets suffice for every row array
+  bool off32 = false;    // 32-bit byte offsets, as a product of 24-bit factors,
+                         // suffice for every row array
   bool hexd_ok = false; // owned vertices follow the diagnostics maps (hexd)
   std::vector<int> hexrec_h, coc_h, hexu_h, hexc_h;
   DBuf<int> hexrec, coc, hexu, hexc;

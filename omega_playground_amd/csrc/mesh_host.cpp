@@ -431,7 +431,10 @@ void DeviceMesh::build_device(int ord) {
              rows_equal(w_h, 3 * (size_t)me2) && rows_equal(cdiv_h, ME) &&
              rows_equal(cke_h, ME) && rows_equal(crv_h, 6) && rows_equal(cth_h, 6);
   const size_t rows = std::max({(size_t)NC, (size_t)NE, (size_t)NV});
-  off32 = rows < (size_t(1) << 24) && rows * (size_t)L * sizeof(double) < (size_t(1) << 32);
+  // both factors of a row's offset in 24 bits (the kernels' multiply has no
+  // more), the offset in 32
+  off32 = rows < (size_t(1) << 24) && (size_t)L * sizeof(double) < (size_t(1) << 24) &&
+          rows * (size_t)L * sizeof(double) < (size_t(1) << 32);
   build_hex_stage(*this);
   ccx_h.clear();
   if (!hex_ok) {

@@ -226,3 +226,26 @@ def test_vjp_at_a_state_whose_stage_is_not_run(nx, ny, L, ntr):
             got.append(list(so.download()) + [gp] + aux)
         for a, b in zip(*got):
             assert same_bits(a, b), terms
+
+
+# 24 bytes a level in a cell's edge rows: the last count a 24-bit factor holds
+# and the next one, which other kernels take (tests/test_host_side.py)
+@pytest.mark.parametrize("L", [699050, 699051])
+def test_tallest_columns_bitwise(L):
+    print("case", L, flush=True)
+    nx, ny, dc, few = 4, 4, 10e3, 5
+    pd = params_dict(dc, 1, all_terms=False)
+    om = po.Mesh(nx, ny, dc, few)
+    omodel = po.Model(om, **pd)
+    state = rich_state(om, few, 1, 3)
+    ref = omodel.new_state()
+    omodel.compute_tendency(ref, state, 0.0)
+    gm = swe.PlanarHexagonalMesh(nx, ny, dc, L)
+    gmodel = swe.ShallowWaterModel(gm, swe.ShallowWaterParams(**pd))
+
+    def columns(a):  # levels do not see each other: the few, over and over
+        return np.ascontiguousarray(a[..., np.arange(L) % few])
+
+    gs, gt = upload(gm, 1, [columns(a) for a in state]), swe.ShallowWaterState(gm, 1)
+    gmodel.compute_tendency(gt, gs, 0.0)
+    compare(gt.download(), [columns(a) for a in ref], L)
