@@ -511,8 +511,8 @@ int omega_batch_autotune(omega_batch_t batch, int reps, double *best_ms, omega_s
 int omega_batch_info(omega_batch_t batch, int *nmembers, int64_t *blocks_per_launch,
                      int64_t *cell_layers);
 /* Ensemble adjoint with checkpointing under a memory cap.  The members
- * (all on one mesh, with one layer count, tracer count, parameter set and
- * dt; the batch's stepper kind) are stacked along the layer axis, which no
+ * (all on one mesh, with one layer count, tracer count, parameter set,
+ * Coriolis parameter of every vertex and dt; the batch's stepper kind) are stacked along the layer axis, which no
  * operator couples, into one model of nmembers*nlayers layers, so each
  * stage of the forward, recompute and reverse sweeps is one launch per
  * kernel for the whole ensemble.  J = (1/M) sum_m J_m, J_m the misfit of

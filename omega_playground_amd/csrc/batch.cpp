@@ -712,6 +712,8 @@ int omega_batch_adjoint_run(omega_batch_t B, double t0, int nsteps, int n_snapsh
                     "batch adjoint: all members must share one mesh (layers are stacked)");
       OMEGA_REQUIRE(same_params(mb.M->params, M0->params) && mb.M->terms == M0->terms,
                     "batch adjoint: members must share the model parameters and terms");
+      OMEGA_REQUIRE(mb.M->f_h == M0->f_h,
+                    "batch adjoint: members must share the Coriolis parameter of every vertex");
       OMEGA_REQUIRE(mb.dt == dt, "batch adjoint: members must share dt");
       OMEGA_REQUIRE(!mb.M->add_fn, "batch adjoint: members must not have an additional tendency");
       OMEGA_REQUIRE(mb.S->ntr == ntr, "batch adjoint: member state tracer count differs");
@@ -751,6 +753,7 @@ int omega_batch_adjoint_run(omega_batch_t B, double t0, int nsteps, int n_snapsh
       ok(omega_state_create(o->mesh, ntr, &o->obs));
       ok(omega_state_create(o->mesh, ntr, &o->grad));
     }
+    if (o->model->f_h != M0->f_h) model_set_f(o->model, M0->f_h); // same numbering
     std::vector<omega_state_s *> members(M), wanted(obs, obs + M), out(grads, grads + M);
     for (int m = 0; m < M; ++m) members[m] = B->mem[m]->S;
     stack_fields(o->y, members, L, true, s);

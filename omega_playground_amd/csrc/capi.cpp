@@ -496,10 +496,7 @@ int omega_model_set_f_vertex(omega_model_t M, const double *f) {
     const DeviceMesh &dm = M->mesh->dm;
     std::vector<Real> tmp(dm.host.nvertices);
     for (int i = 0; i < dm.host.nvertices; ++i) tmp[i] = f[dm.vert_n2o[i]];
-    M->f_v.upload(tmp);
-    M->f_uniform = rows_equal(tmp, 1);
-    M->f_value = tmp.empty() ? 0 : tmp[0];
-    M->touch();
+    model_set_f(M, tmp);
   });
 }
 

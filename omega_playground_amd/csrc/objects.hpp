@@ -118,6 +118,7 @@ struct omega_model_s {
   // mesh, coefficients, terms or kernel forms need the other kernels
   bool stage_coef(omega_hip::HexCoef &q) const;
   Real f_value = 0; // the Coriolis parameter where f_uniform
+  std::vector<Real> f_h; // at every vertex, in device numbering
   ModelCoef coef() const {
     return ModelCoef{params.grav, f_v.p, cv2.p, cv4.p, ct2.p, ct4.p,
                      f_uniform && mix_uniform ? 1 : 0, params.drag_coeff};
@@ -219,6 +220,8 @@ bool stream_capturing(hipStream_t s);
 hipStream_t capture_stream();
 
 void model_build_coefficients(omega_model_s *M);
+// sets the Coriolis parameter of every vertex (device numbering)
+void model_set_f(omega_model_s *M, const std::vector<Real> &f);
 void ensure_vdel4(omega_model_s *M);
 void model_build_linear(omega_model_s *M);
 void run_diag(omega_model_s *M, const Real *h, const Real *vn, const Real *tr, hipStream_t s);

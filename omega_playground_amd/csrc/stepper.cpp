@@ -19,13 +19,20 @@ bool stage_terms(const omega_model_s *M) {
          !M->params.disable_h_tendency && !M->params.disable_vn_tendency;
 }
 
+void model_set_f(omega_model_s *M, const std::vector<Real> &f) {
+  M->f_v.upload(f);
+  M->f_h = f;
+  M->f_uniform = rows_equal(f, 1);
+  M->f_value = f.empty() ? 0 : f[0];
+  M->touch();
+}
+
 void model_build_coefficients(omega_model_s *M) {
   const DeviceMesh &dm = M->mesh->dm;
   const HostMesh &hm = dm.host;
   const int NC = hm.ncells, NE = hm.nedges, NV = hm.nvertices, ME = hm.max_edges;
   const size_t L = hm.nlayers, ntr = M->params.ntracers;
-  std::vector<Real> f(NV, M->params.f0);
-  M->f_v.upload(f);
+  model_set_f(M, std::vector<Real>(NV, M->params.f0));
   std::vector<Real> cv2(NE), cv4(NE);
   for (int e = 0; e < NE; ++e) {
     // mask*visc*scaling with mask = 1 (vel_diff_edge.hpp:83-84,
@@ -54,8 +61,6 @@ void model_build_coefficients(omega_model_s *M) {
   M->ct2_h = ct2;
   M->ct4_h = ct4;
   M->ct4.upload(ct4);
-  M->f_uniform = rows_equal(f, 1);
-  M->f_value = M->params.f0;
   M->mix_uniform = rows_equal(cv2, 1) && rows_equal(cv4, 1) && rows_equal(ct2, ME) &&
                    rows_equal(ct4, ME);
   M->rvort_v.alloc((size_t)NV * L);

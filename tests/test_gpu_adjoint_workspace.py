@@ -96,3 +96,26 @@ def test_window_gradient_is_the_chain_of_step_adjoints(L, ntr, snaps):
     grad = swe.ShallowWaterState(mesh, ntr)
     Jw, _ = swe.adjoint_run(st, 0.0, dt, n, upload(mesh, ntr, y0), obs, grad, n_snapshots=snaps)
     assert J == Jw and all(same_bits(a, b) for a, b in zip(grad.download(), cot.download()))
+
+
+def test_ensemble_gradient_with_a_coriolis_parameter_per_vertex():
+    """The stacked model has the members' own Coriolis parameter, also after
+    it changed; members that differ in it are refused."""
+    mesh, pd, members = make_ensemble(M=2, L=4, n=3)
+    b, states = make_batch(mesh, 2, members, "rk4", 40.0)
+    grads = [swe.ShallowWaterState(mesh, 2) for _ in members]
+    wanted = [o for _, _, o in members]
+    for seed in (0, 1):
+        f = pd["f0"] * np.random.default_rng(seed).uniform(0.5, 1.5, mesh.nvertices)
+        for model, _, _ in members:
+            model.set_f_vertex(f)
+        b.adjoint_run(0.0, 3, wanted, grads, n_snapshots=2)
+        for m, (model, y0, obs) in enumerate(members):
+            g = swe.ShallowWaterState(mesh, 2)
+            swe.adjoint_run(stepper(model, "rk4"), 0.0, 40.0, 3, upload(mesh, 2, y0), obs, g,
+                            (0.5, 0.0, 0.5), n_snapshots=2)
+            for x, y in zip(grads[m].download(), g.download()):
+                assert same_bits(x, y), (seed, m)
+    members[1][0].set_f_vertex(2 * f)
+    with pytest.raises(RuntimeError, match="Coriolis"):
+        b.adjoint_run(0.0, 3, wanted, grads, n_snapshots=2)
