@@ -100,6 +100,10 @@ Real *state_buf(omega_state_s *S, int c, int f) {
 
 void build_tables(omega_batch_s *B) {
   OMEGA_REQUIRE(!B->mem.empty(), "batch: no members");
+  // a build that fails leaves neither tables to step with nor graphs that
+  // read the ones freed below
+  B->built = false;
+  B->drop_graphs();
   const int nm = (int)B->mem.size(), ns = B->nstages, N = B->N, T = B->threads;
   std::vector<int> blk;
   std::vector<BatchMember> geo(nm);
@@ -313,7 +317,6 @@ void build_tables(omega_batch_s *B) {
   OMEGA_HIP_CHECK(hipMemcpy(B->desc.p, tab.data(), tab.size() * sizeof(BatchMember),
                             hipMemcpyHostToDevice));
   B->parity = 0;
-  B->drop_graphs();
   B->built = true;
 }
 

@@ -35,6 +35,7 @@ struct Launched {
   hipStream_t stream;
 };
 std::vector<Launched> launches;
+std::map<hipGraphExec_t, int> graphs; // live executables and their replays
 } // namespace fake
 
 extern "C" {
@@ -92,6 +93,25 @@ hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *s) {
   return *s = hipStreamCaptureStatusNone, hipSuccess;
 }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return *s = nullptr, hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g) { return *g = nullptr, hipSuccess; }
+hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t, hipGraphNode_t *, char *, size_t) {
+  static char *next = nullptr;
+  *e = reinterpret_cast<hipGraphExec_t>(++next);
+  fake::graphs[*e] = 0;
+  return hipSuccess;
+}
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t e) {
+  CHECK(fake::graphs.erase(e));
+  return hipSuccess;
+}
+hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t) {
+  CHECK(fake::graphs.count(e));
+  ++fake::graphs[e];
+  return hipSuccess;
+}
 hipError_t hipEventCreate(hipEvent_t *e) { return *e = nullptr, hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
@@ -113,8 +133,74 @@ static void tall() {
   }
 }
 
+static void ok(int rc) {
+  if (rc != OMEGA_OK) std::printf("%s\n", omega_last_error());
+  CHECK(rc == OMEGA_OK);
+}
+
+// An ensemble of lattice members for the stage kernels, and its parts
+struct Ensemble {
+  omega_mesh_t mesh = nullptr;
+  std::vector<omega_model_t> models;
+  std::vector<omega_state_t> states;
+  omega_batch_t batch = nullptr;
+
+  Ensemble(int members, int nx, int ny, int L, omega_params p, int kind) {
+    ok(omega_mesh_create_planar_hex(nx, ny, 1e4, L, OMEGA_ORDER_HILBERT, &mesh));
+    ok(omega_batch_create(kind, 5, &batch));
+    for (int i = 0; i < members; ++i) {
+      omega_model_t m;
+      omega_state_t s;
+      ok(omega_model_create(mesh, &p, &m));
+      ok(omega_state_create(mesh, p.ntracers, &s));
+      ok(omega_batch_add(batch, m, s, 10.0, nullptr));
+      models.push_back(m);
+      states.push_back(s);
+    }
+  }
+  ~Ensemble() {
+    ok(omega_batch_destroy(batch));
+    for (auto s : states) ok(omega_state_destroy(s));
+    for (auto m : models) ok(omega_model_destroy(m));
+    ok(omega_mesh_destroy(mesh));
+  }
+  static omega_params params(int ntr) {
+    omega_params p{};
+    p.f0 = 1e-4;
+    p.grav = 9.81;
+    p.ntracers = ntr;
+    return p;
+  }
+};
+
+// A step whose tables cannot be rebuilt fails and leaves no graph of the old
+// ones; the step after it does all of its work.
+static void rebuild() {
+  for (int graph : {0, 1})
+    for (int fail = 0;; ++fail) {
+      Ensemble e(2, 6, 4, 8, Ensemble::params(1), OMEGA_STEPPER_RK4);
+      ok(omega_batch_set_graph(e.batch, graph));
+      ok(omega_batch_step(e.batch, nullptr));
+      fake::launches.clear();
+      ok(omega_model_set_terms(e.models[1], 7 + 8)); // the tables are now out of date
+      fake::fail_after = fail;
+      const bool failed = omega_batch_step(e.batch, nullptr) != OMEGA_OK;
+      fake::fail_after = -1;
+      std::printf("graph %d, allocation %d fails: %d\n", graph, fail, (int)failed);
+      const size_t want = 4 * (2 + 2); // momentum and tracers of two sets of terms per stage
+      if (!failed) {
+        CHECK(fake::launches.size() == want && fail > 0);
+        break;
+      }
+      CHECK(fake::graphs.empty());
+      fake::launches.clear();
+      ok(omega_batch_step(e.batch, nullptr));
+      CHECK(fake::launches.size() == want);
+    }
+}
+
 int main(int argc, char **argv) {
-  const std::map<std::string, std::function<void()>> checks = {{"tall", tall}};
+  const std::map<std::string, std::function<void()>> checks = {{"tall", tall}, {"rebuild", rebuild}};
   CHECK(argc == 2 && checks.count(argv[1]));
   checks.at(argv[1])();
   std::printf("%s ok\n", argv[1]);
