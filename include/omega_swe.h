@@ -457,7 +457,9 @@ int omega_misfit(omega_model_t model, omega_state_t state, omega_state_t obs,
                  const double *weights, omega_state_t cot, double *J, omega_stream_t stream);
 
 /* J(y_nsteps) of omega_misfit after nsteps steps from state (left unchanged),
- * grad = dJ/dy_0 (overwritten), param_grad += dJ/d(coefficients). */
+ * grad = dJ/dy_0 (overwritten), param_grad += dJ/d(coefficients).  The
+ * stepper keeps the run's state copy and snapshots for the next call where
+ * they are 1 GiB or less; destroying the stepper frees them. */
 int omega_adjoint_run(omega_stepper_t stepper, double t0, double dt, int nsteps,
                       int n_snapshots, int64_t byte_cap, omega_state_t state, omega_state_t obs,
                       const double *weights, double *J, omega_state_t grad, double *param_grad,
@@ -520,7 +522,10 @@ int omega_batch_info(omega_batch_t batch, int *nmembers, int64_t *blocks_per_lau
  * dJ/d(member m's initial state) (overwritten); param_grad[0..4) (may be NULL)
  * += dJ/d(shared coefficients).  At most n_snapshots ensemble states and,
  * when byte_cap > 0, byte_cap bytes of them are stored; the members' states
- * are left unchanged.  Synchronises. */
+ * are left unchanged.  The batch keeps the stacked model, its states and
+ * workspaces for the next call where all of them, snapshots included, are
+ * 1 GiB or less (without the snapshots, where that brings them below it);
+ * destroying the batch frees them.  Synchronises. */
 int omega_batch_adjoint_run(omega_batch_t batch, double t0, int nsteps, int n_snapshots,
                             int64_t byte_cap, const omega_state_t *obs, const double *weights,
                             double *J, omega_state_t *grads, double *param_grad,

@@ -62,7 +62,7 @@ struct omega_batch_s {
   bool use_graph = false;
   std::map<int, hipGraphExec_t> graphs;
   // omega_batch_adjoint_run's stacked mesh, model, stepper and states, kept
-  // for the next call where small (kKeepBytes) and what they were built for
+  // for the next call within kKeepBytes, and what they were built for
   std::shared_ptr<void> stacked;
   struct StackedFor {
     uint64_t mesh = 0;
@@ -682,6 +682,7 @@ struct Owned {
   omega_model_s *model = nullptr;
   omega_stepper_s *st = nullptr;
   omega_state_s *y = nullptr, *obs = nullptr, *grad = nullptr;
+  int64_t bytes = 0; // device memory of all of it
   ~Owned() {
     (void)omega_state_destroy(grad);
     (void)omega_state_destroy(obs);
@@ -737,8 +738,11 @@ int omega_batch_adjoint_run(omega_batch_t B, double t0, int nsteps, int n_snapsh
     const omega_batch_s::StackedFor &sf = B->stacked_for;
     std::shared_ptr<Owned> o = std::static_pointer_cast<Owned>(B->stacked);
     B->stacked.reset(); // a call that fails leaves none behind
+    int64_t start = device_bytes();
     if (!o || sf.mesh != mesh0->uid || sf.M != M || sf.ntr != ntr || sf.terms != M0->terms ||
         !same_params(sf.params, M0->params)) {
+      o.reset();
+      start = device_bytes();
       o = std::make_shared<Owned>();
       o->mesh = new omega_mesh_s();
       o->mesh->dm.host = h0;
@@ -767,10 +771,15 @@ int omega_batch_adjoint_run(omega_batch_t B, double t0, int nsteps, int n_snapsh
                          param_grad, stream));
     stack_fields(o->grad, out, L, false, s);
     OMEGA_HIP_CHECK(hipStreamSynchronize(s));
-    // states, stage states, diagnostics and cotangents: about 100 rows of a
-    // cell and tracer
-    const size_t row = (size_t)h0.ncells * M * L * sizeof(Real);
-    if (row * (100 + 20 * (size_t)ntr) <= kKeepBytes) {
+    // this call allocates for the stacked objects alone, and they only grow
+    o->bytes += device_bytes() - start;
+    if (o->bytes > kKeepBytes) {
+      // without the snapshots it may do
+      start = device_bytes();
+      o->st->adj_run.reset();
+      o->bytes += device_bytes() - start;
+    }
+    if (o->bytes <= kKeepBytes) {
       B->stacked = o;
       B->stacked_for.mesh = mesh0->uid;
       B->stacked_for.M = M;

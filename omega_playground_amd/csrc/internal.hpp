@@ -38,6 +38,13 @@ struct Error : std::runtime_error {
     if (!(cond)) throw ::omega_hip::Error(OMEGA_ERR_ARG, msg);                         \
   } while (0)
 
+// Bytes of device buffers this thread has allocated, less those it has freed:
+// what the objects made in between hold, as a difference.
+inline int64_t &device_bytes() {
+  static thread_local int64_t n = 0;
+  return n;
+}
+
 // Device buffer with RAII ownership.
 template <class T> struct DBuf {
   T *p = nullptr;
@@ -54,14 +61,18 @@ template <class T> struct DBuf {
   ~DBuf() { release(); }
   void alloc(size_t count, bool zero = true) {
     release();
-    n = count;
     if (count) {
       OMEGA_HIP_CHECK(hipMalloc(&p, count * sizeof(T)));
+      device_bytes() += (int64_t)(count * sizeof(T));
+      n = count;
       if (zero) OMEGA_HIP_CHECK(hipMemset(p, 0, count * sizeof(T)));
     }
   }
   void release() {
-    if (p) (void)hipFree(p);
+    if (p) {
+      (void)hipFree(p);
+      device_bytes() -= (int64_t)(n * sizeof(T));
+    }
     p = nullptr;
     n = 0;
   }

@@ -32,9 +32,10 @@ template <class Map> void destroy_graphs(Map &graphs) {
 } // namespace omega_hip
 
 namespace omega_hip {
-// Device memory an object keeps between calls that could free it: more than
-// this is freed when the call ends.
-constexpr size_t kKeepBytes = size_t(1) << 30;
+// Device memory an adjoint run leaves with its stepper, or an ensemble's with
+// its batch, for the next call: where it is more than this all of it is freed
+// when the call ends, otherwise with the object.
+constexpr int64_t kKeepBytes = int64_t(1) << 30;
 uint64_t next_uid();
 } // namespace omega_hip
 
@@ -184,8 +185,8 @@ struct omega_stepper_s {
   // step adjoint: recomputed stage states (RK4 stage inputs 2..4, LSRK stage
   // inputs 2..S), their tendency, the incoming cotangent and stage cotangents
   DBuf<Real> adj_y[4][3], adj_t[3], adj_gy[3], adj_pb[3], adj_kb[3];
-  // omega_adjoint_run's tape and running state, kept for the next call where
-  // small (kKeepBytes)
+  // omega_adjoint_run's tape and running state, kept for the next call within
+  // kKeepBytes
   std::shared_ptr<void> adj_run;
   ~omega_stepper_s() { omega_hip::destroy_graphs(graphs); }
 };

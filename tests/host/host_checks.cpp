@@ -199,8 +199,75 @@ static void rebuild() {
     }
 }
 
+// What adjoint runs keep between calls is within its bound, 1 GiB for a
+// stepper and for an ensemble.
+constexpr size_t kBound = size_t(1) << 30;
+static const double weights[3] = {1, 0, 1};
+
+static void keep_stepper() {
+  for (int kind : {OMEGA_STEPPER_RK4, OMEGA_STEPPER_LSRK})
+    for (int L : {64, 108, 114, 120, 140}) {
+      // the first call's snapshots are too many to keep
+      omega_mesh_t mesh;
+      omega_model_t model;
+      omega_stepper_t st;
+      omega_state_t y, obs, grad;
+      const omega_params p = Ensemble::params(0);
+      ok(omega_mesh_create_planar_hex(256, 256, 1e4, L, OMEGA_ORDER_HILBERT, &mesh));
+      ok(omega_model_create(mesh, &p, &model));
+      ok(omega_stepper_create(model, kind, 5, &st));
+      for (omega_state_t *s : {&y, &obs, &grad}) ok(omega_state_create(mesh, 0, s));
+      size_t held[2];
+      for (int snaps : {12, 1}) {
+        double J;
+        ok(omega_adjoint_run(st, 0.0, 1.0, 12, snaps, 0, y, obs, weights, &J, grad, nullptr, nullptr));
+        held[snaps == 1] = fake::bytes;
+      }
+      std::printf("kind %d, %d levels: %zu bytes kept\n", kind, L, held[1] - held[0]);
+      CHECK(held[1] - held[0] <= kBound);
+      CHECK(L > 64 || held[1] > held[0]);
+      for (omega_state_t s : {y, obs, grad}) ok(omega_state_destroy(s));
+      ok(omega_stepper_destroy(st));
+      ok(omega_model_destroy(model));
+      ok(omega_mesh_destroy(mesh));
+      CHECK(fake::bytes == 0);
+    }
+}
+
+static void keep_ensemble() {
+  for (int kind : {OMEGA_STEPPER_RK4, OMEGA_STEPPER_LSRK})
+    for (int ntr : {1, 4})
+      for (int L : {8, 24, 32, 40, 56, 64}) {
+        omega_params p = Ensemble::params(ntr);
+        p.visc_del4 = 1;
+        p.eddy_diff4 = 1;
+        Ensemble e(4, 64, 64, L, p, kind);
+        std::vector<omega_state_t> obs(4), grads(4);
+        for (int i = 0; i < 4; ++i) {
+          ok(omega_state_create(e.mesh, ntr, &obs[i]));
+          ok(omega_state_create(e.mesh, ntr, &grads[i]));
+        }
+        const size_t before = fake::bytes;
+        double J;
+        for (int call = 0; call < 2; ++call)
+          ok(omega_batch_adjoint_run(e.batch, 0.0, 20, 20, 0, obs.data(), weights, &J, grads.data(),
+                                     nullptr, nullptr));
+        std::printf("kind %d, %d tracers, %d levels: %zu bytes kept\n", kind, ntr, L,
+                    fake::bytes - before);
+        CHECK(fake::bytes - before <= kBound);
+        CHECK(L > 8 || fake::bytes > before);
+        for (int i = 0; i < 4; ++i) {
+          ok(omega_state_destroy(obs[i]));
+          ok(omega_state_destroy(grads[i]));
+        }
+      }
+  CHECK(fake::bytes == 0);
+}
+
 int main(int argc, char **argv) {
-  const std::map<std::string, std::function<void()>> checks = {{"tall", tall}, {"rebuild", rebuild}};
+  const std::map<std::string, std::function<void()>> checks = {{"tall", tall}, {"rebuild", rebuild},
+                                                              {"keep_stepper", keep_stepper},
+                                                              {"keep_ensemble", keep_ensemble}};
   CHECK(argc == 2 && checks.count(argv[1]));
   checks.at(argv[1])();
   std::printf("%s ok\n", argv[1]);
