@@ -21,7 +21,7 @@ using namespace stage;
 template <int N, bool V2, bool V4, bool EMIT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N == 1 ? 4 : 2)))
     k_stage_mom(StageLaunch p) {
-  stage_mom<N, V2, V4, EMIT>(p, xcd_entry(p.tiles));
+  stage_mom<N, V2, V4, EMIT>(p, xcd_entry(p.tiles, p.swz));
 }
 
 // The same leaving the stage input's diagnostics and the rows its tendency
@@ -33,7 +33,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N == 1
 template <int N, bool V2, bool V4>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N == 1 ? 3 : 2)))
     k_stage_mom_pre(StageLaunch p) {
-  stage_mom<N, V2, V4, true, true>(p, xcd_entry(p.tiles));
+  stage_mom<N, V2, V4, true, true>(p, xcd_entry(p.tiles, p.swz));
 }
 
 // A parameter block through the constant address space (no kernel writes one):
@@ -52,7 +52,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N == 1
   const int w = uniform(who[blockIdx.x]);
   if (w < 0) return;
   const StageLaunch &p = constant_at(desc, w);
-  stage_mom<N, V2, false, EMIT>(p, logical_block((int)blockIdx.x - p.block0, p.tiles, 1));
+  stage_mom<N, V2, false, EMIT>(p, logical_block((int)blockIdx.x - p.block0, p.tiles, p.swz));
 }
 
 // The edge Laplacian: of the velocity (FINAL false), then of that result,
@@ -61,7 +61,7 @@ template <int N, bool FINAL, bool EMIT>
 __global__ void __launch_bounds__(256) k_stage_lap(StageLaunch p) {
   int c;
   Ctx x;
-  if (!stage_place(p, xcd_entry(p.tiles), N, c, x)) return;
+  if (!stage_place(p, xcd_entry(p.tiles, p.swz), N, c, x)) return;
   int id[hl::kCells];
   load_cells(p.rec, c, id);
   LapOut<N> o;
@@ -86,7 +86,7 @@ __global__ void __launch_bounds__(256) k_stage_lap(StageLaunch p) {
 template <int N, int LX, int TW, int TH, bool D2, bool D4, bool EMIT>
 __global__ void __launch_bounds__(LX *TW *TH) __attribute__((amdgpu_waves_per_eu(N == 2 ? 3 : 4)))
     k_stage_tile(TileLaunch p) {
-  stage_tile<N, LX, TW, TH, D2, D4, EMIT>(p, xcd_entry(p.work), (int)blockIdx.y * p.per_block);
+  stage_tile<N, LX, TW, TH, D2, D4, EMIT>(p, xcd_entry(p.work, p.swz), (int)blockIdx.y * p.per_block);
 }
 
 template <int N, int LX, int TW, int TH, bool D2, bool D4, bool EMIT>
@@ -95,7 +95,7 @@ __global__ void __launch_bounds__(LX *TW *TH) __attribute__((amdgpu_waves_per_eu
   const int w = uniform(who[blockIdx.x]);
   if (w < 0) return;
   const TileLaunch &p = constant_at(desc, w);
-  stage_tile<N, LX, TW, TH, D2, D4, EMIT>(p, logical_block((int)blockIdx.x - p.block0, p.work, 1), 0);
+  stage_tile<N, LX, TW, TH, D2, D4, EMIT>(p, logical_block((int)blockIdx.x - p.block0, p.work, p.swz), 0);
 }
 
 using StageFn = void (*)(StageLaunch);
@@ -166,6 +166,7 @@ void stage_launch(const MeshView &m, const Launch &lc, int N, const HexCoef &q, 
   p.rows = lc.rows > 0 ? std::min(lc.rows, 256 / p.lx) : 256 / p.lx;
   p.ncb = (m.nc + p.rows - 1) / p.rows;
   p.tiles = p.ncb * nch;
+  p.swz = lc.swizzle;
   p.a = a;
   p.d = d;
   t = TileLaunch{};
@@ -181,6 +182,7 @@ void stage_launch(const MeshView &m, const Launch &lc, int N, const HexCoef &q, 
   t.nc = m.nc;
   t.L = m.L;
   t.per_block = a.ntr;
+  t.swz = lc.swizzle;
   t.a = a;
   t.d = d;
 }

@@ -10,9 +10,11 @@ namespace omega_hip {
 namespace stage {
 
 // Entry b of n for this block: workgroups are dealt to the 8 XCDs
-// round-robin, and each XCD takes a contiguous range of entries, so that
-// neighbouring cells' rows are re-read from one L2.
-__device__ __forceinline__ int xcd_entry(int n) { return logical_block((int)blockIdx.x, n, 1); }
+// round-robin, and with swz each XCD takes a contiguous range of entries, so
+// that neighbouring cells' rows are re-read from one L2.
+__device__ __forceinline__ int xcd_entry(int n, int swz) {
+  return logical_block((int)blockIdx.x, n, swz);
+}
 
 // The cell and levels of this thread at an entry (level chunk, cell block);
 // false: no work here.

@@ -12,6 +12,7 @@ struct StageLaunch {
   HexCoef q;
   const int *rec; // neighbourhood records
   int nc, L, lx, rows, ncb, tiles;
+  int swz;    // each XCD takes a contiguous range of entries
   int block0; // first block in an ensemble's launch
   StageArgs a;
   DiagOut d;
@@ -25,7 +26,7 @@ struct TileLaunch {
   HexCoef q;
   const int *ids; // [tiles][(th + 4)(tw + 4)] cell at each place, row-major
   int nx, ny, tiles_x, nch, work, nc, L, per_block;
-  int block0;
+  int swz, block0;
   StageArgs a;
   DiagOut d;
 };

@@ -2,6 +2,7 @@
 // for the HIP runtime (memory is host memory, a launch is noted and not run),
 // so that what the host code allocates, keeps, launches and does after a
 // failing call can be looked at.  Built and run by tests/test_host_side.py.
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -10,7 +11,7 @@
 #include <string>
 #include <vector>
 
-#include "internal.hpp"
+#include "stage_launch.hpp"
 
 using namespace omega_hip;
 
@@ -33,7 +34,14 @@ int fail_after = -1; // allocations until one fails, -1: none does
 struct Launched {
   dim3 grid, block;
   hipStream_t stream;
+  std::vector<char> arg; // of its first argument, as many bytes as were asked for
+  template <class T> T at() const {
+    T x;
+    std::memcpy(static_cast<void *>(&x), arg.data(), sizeof(T));
+    return x;
+  }
 };
+size_t arg_bytes = 0;
 std::vector<Launched> launches;
 std::map<hipGraphExec_t, int> graphs; // live executables and their replays
 } // namespace fake
@@ -68,13 +76,14 @@ hipError_t hipMemset(void *p, int v, size_t n) {
   if (v || !fake::live.count(p)) std::memset(p, v, n);
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *, dim3 grid, dim3 block, void **, size_t, hipStream_t s) {
-  fake::launches.push_back({grid, block, s});
+hipError_t hipLaunchKernel(const void *, dim3 grid, dim3 block, void **args, size_t, hipStream_t s) {
+  const char *a = static_cast<const char *>(args[0]);
+  fake::launches.push_back({grid, block, s, std::vector<char>(a, a + fake::arg_bytes)});
   return hipSuccess;
 }
 static fake::Launched pushed;
 hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t, hipStream_t s) {
-  pushed = {grid, block, s};
+  pushed = {grid, block, s, {}};
   return hipSuccess;
 }
 hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shared, hipStream_t *s) {
@@ -264,10 +273,41 @@ static void keep_ensemble() {
   CHECK(fake::bytes == 0);
 }
 
+// The launches of f, with as many bytes of their first arguments
+template <class F> static std::vector<fake::Launched> launched(size_t arg_bytes, F &&f) {
+  fake::launches.clear();
+  fake::arg_bytes = arg_bytes;
+  f();
+  fake::arg_bytes = 0;
+  return fake::launches;
+}
+
+// The block order set with omega_model_set_launch reaches the stage kernels,
+// a model's own and an ensemble's.
+static void block_order() {
+  Ensemble e(1, 128, 128, 64, Ensemble::params(2), OMEGA_STEPPER_RK4);
+  omega_state_t tend;
+  ok(omega_state_create(e.mesh, 2, &tend));
+  for (int order : {1, 0}) {
+    ok(omega_model_set_launch(e.models[0], 0, 0, order, -1));
+    const auto own = launched(std::max(sizeof(StageLaunch), sizeof(TileLaunch)), [&] {
+      ok(omega_model_compute_tendency(e.models[0], tend, e.states[0], 0.0, OMEGA_ADD_REPLACE, nullptr));
+    });
+    const auto batch = launched(sizeof(void *), [&] { ok(omega_batch_step(e.batch, nullptr)); });
+    CHECK(own.size() == 2 && batch.size() == 8); // momentum, tracers
+    CHECK(own[0].at<StageLaunch>().swz == order);
+    CHECK(own[1].at<TileLaunch>().swz == order);
+    CHECK(batch[0].at<const StageLaunch *>()->swz == order);
+    CHECK(batch[1].at<const TileLaunch *>()->swz == order);
+  }
+  ok(omega_state_destroy(tend));
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, std::function<void()>> checks = {{"tall", tall}, {"rebuild", rebuild},
                                                               {"keep_stepper", keep_stepper},
-                                                              {"keep_ensemble", keep_ensemble}};
+                                                              {"keep_ensemble", keep_ensemble},
+                                                              {"block_order", block_order}};
   CHECK(argc == 2 && checks.count(argv[1]));
   checks.at(argv[1])();
   std::printf("%s ok\n", argv[1]);

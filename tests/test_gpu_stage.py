@@ -249,3 +249,24 @@ def test_tallest_columns_bitwise(L):
     gs, gt = upload(gm, 1, [columns(a) for a in state]), swe.ShallowWaterState(gm, 1)
     gmodel.compute_tendency(gt, gs, 0.0)
     compare(gt.download(), [columns(a) for a in ref], L)
+
+
+@pytest.mark.parametrize("terms", [79, 127])
+def test_block_order_does_not_change_bits(terms):
+    """Large enough for launches of their own for momentum and tracers: with
+    and without the XCD order, alone and as an ensemble's member."""
+    nx, ny, L, ntr = 72, 70, 64, 2
+    mesh = swe.PlanarHexagonalMesh(nx, ny, 10e3, L)
+    model = swe.ShallowWaterModel(mesh, swe.ShallowWaterParams(**params_dict(10e3, ntr)))
+    model.terms = terms
+    y0, out = rich_state(mesh, L, ntr, 2), []
+    for order in (1, 0):
+        model.set_launch(0, 0, order)
+        s, b = upload(mesh, ntr, y0), swe.Batch("rk4", 4)
+        m = upload(mesh, ntr, y0)
+        b.add(model, m, 20.0)
+        swe.RK4Stepper(model).run(0.0, 20.0, 2, s)
+        b.run(2)
+        out += [s.download(), m.download()]
+    for got in out[1:]:
+        compare(got, out[0], terms)

@@ -22,7 +22,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["tall", "rebuild", "keep_stepper", "keep_ensemble"])
+@pytest.mark.parametrize("what", ["tall", "rebuild", "keep_stepper", "keep_ensemble", "block_order"])
 def test_host_side(program, what):
     r = subprocess.run([program, what], capture_output=True, text=True, timeout=120)
     print(r.stdout, r.stderr, flush=True)
