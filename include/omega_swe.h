@@ -306,8 +306,8 @@ int omega_model_get_terms(omega_model_t model, int *mask);
 /* Launch shape: cells per block (0: fill 256 threads), levels per thread
  * (1 or 2), whether blocks are swizzled so each XCD walks a contiguous
  * stretch of the cell curve (-1 keeps it; models small enough for one launch
- * of all fields per stage run their blocks in order either way), and levels
- * per block (0: all).
+ * of all fields per stage run their blocks in order either way, and fill 256
+ * threads), and levels per block (0: all).
  * No reference counterpart (Kokkos chose its tiles, src/common.hpp:78-104);
  * these are the autotuner's knobs.  Non-positive values keep the current
  * setting unless stated. */

@@ -275,6 +275,7 @@ void build_tables(omega_batch_s *B) {
           const size_t ng = B->groups[own[i]]->members.size();
           const size_t at = ((size_t)p * ns + s) * ng + place[i];
           stage_launch(g.m, M->lc, B->groups[own[i]]->kind.N, coef[i], a, g.d, T.mom[at], T.tile[at]);
+          whole_blocks(T.mom[at]);
           continue;
         }
         g.a = a;

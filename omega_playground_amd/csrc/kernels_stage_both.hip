@@ -64,14 +64,18 @@ int tile_blocks(const TileLaunch &t, int &per_block) {
 // cells, 74 -> 58 at 2304, 80 -> 80 at 4096 where it is two rounds; one
 // layer, 196608 cells, LSRK5: 97 -> 83 at one and a half), beyond them the
 // tracers miss the waves they have alone (142 -> 151 at 9216 cells).
-bool stage_one_launch(int N, const StageLaunch &p, const TileLaunch &t) {
+bool stage_one_launch(int N, const StageLaunch &p0, const TileLaunch &t) {
   int per_block;
+  StageLaunch p = p0;
+  whole_blocks(p);
   return p.tiles + tile_blocks(t, per_block) <= (N == 2 ? 1024 : 2048);
 }
 
-bool launch_stage_both(int N, int lx, const StageLaunch &p, const TileLaunch &t0, bool emit, bool pre,
+bool launch_stage_both(int N, int lx, const StageLaunch &p0, const TileLaunch &t0, bool emit, bool pre,
                        hipStream_t s) {
-  if (!stage_one_launch(N, p, t0)) return false;
+  if (!stage_one_launch(N, p0, t0)) return false;
+  StageLaunch p = p0;
+  whole_blocks(p);
   TileLaunch t = t0;
   const int blocks = p.tiles + tile_blocks(t0, t.per_block), terms = p.a.terms;
   const bool v2 = terms & T_VDEL2, d2 = terms & T_TDEL2, d4 = terms & T_TDEL4;

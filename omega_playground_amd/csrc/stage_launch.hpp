@@ -36,6 +36,15 @@ void stage_launch(const MeshView &m, const Launch &lc, int N, const HexCoef &q, 
                   const DiagOut &d, StageLaunch &p, TileLaunch &t);
 int stage_levels(const MeshView &m, const Launch &lc); // N of a model's launches
 
+// Momentum blocks for a kernel that has 256 threads whatever the model's cells
+// per block (4 cells of 64 levels would leave three of its wavefronts idle).
+inline void whole_blocks(StageLaunch &p) {
+  const int nch = p.tiles / p.ncb;
+  p.rows = 256 / p.lx;
+  p.ncb = (p.nc + p.rows - 1) / p.rows;
+  p.tiles = p.ncb * nch;
+}
+
 // Fewer tiles than this (two blocks per CU) leave the chip short of blocks.
 constexpr int kFewTiles = 512;
 

@@ -303,11 +303,42 @@ static void block_order() {
   ok(omega_state_destroy(tend));
 }
 
+// Cells per block, set or tuned, leave no wavefronts idle where a kernel has
+// 256 threads in any case (models small enough for one launch, ensembles);
+// where momentum has a launch of its own the block is as large as they ask.
+static void tuned_cells() {
+  for (int nx : {16, 128})
+    for (int L : {64, 60, 7})
+      for (int rows : {0, 4, 2}) {
+        Ensemble e(1, nx, nx, L, Ensemble::params(2), OMEGA_STEPPER_RK4);
+        omega_state_t tend;
+        ok(omega_state_create(e.mesh, 2, &tend));
+        ok(omega_model_set_launch(e.models[0], rows, 0, -1, -1));
+        const auto own = launched(sizeof(StageLaunch), [&] {
+          ok(omega_model_compute_tendency(e.models[0], tend, e.states[0], 0.0, OMEGA_ADD_REPLACE, nullptr));
+        });
+        const auto batch = launched(sizeof(void *), [&] { ok(omega_batch_step(e.batch, nullptr)); });
+        const StageLaunch p = own[0].at<StageLaunch>(), q = *batch[0].at<const StageLaunch *>();
+        const bool one = own.size() == 1;
+        std::printf("%d x %d cells, %d levels, rows %d: %zu launches, %d x %d of %u threads; ensemble %d x %d\n",
+                    nx, nx, L, rows, own.size(), p.lx, p.rows, own[0].block.x, q.lx, q.rows);
+        CHECK(one == (nx == 16 || L == 7));
+        CHECK((int)own[0].block.x == (one ? 256 : p.lx * p.rows));
+        if (one) CHECK(p.rows == 256 / p.lx);
+        else CHECK(p.rows == (rows ? rows : 256 / p.lx));
+        CHECK(batch[0].block.x == 256 && q.rows == 256 / q.lx);
+        for (const StageLaunch &x : {p, q}) CHECK(x.tiles >= 1 && (x.tiles / x.ncb) * x.ncb == x.tiles &&
+                                                  x.ncb * x.rows >= x.nc && (x.ncb - 1) * x.rows < x.nc);
+        ok(omega_state_destroy(tend));
+      }
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, std::function<void()>> checks = {{"tall", tall}, {"rebuild", rebuild},
                                                               {"keep_stepper", keep_stepper},
                                                               {"keep_ensemble", keep_ensemble},
-                                                              {"block_order", block_order}};
+                                                              {"block_order", block_order},
+                                                              {"tuned_cells", tuned_cells}};
   CHECK(argc == 2 && checks.count(argv[1]));
   checks.at(argv[1])();
   std::printf("%s ok\n", argv[1]);

@@ -270,3 +270,24 @@ def test_block_order_does_not_change_bits(terms):
         out += [s.download(), m.download()]
     for got in out[1:]:
         compare(got, out[0], terms)
+
+
+@pytest.mark.parametrize("nx,L", [(12, 64), (12, 9), (72, 60)])
+def test_cells_per_block_do_not_change_bits(nx, L):
+    """Set or tuned cells per block where all fields share a launch (12) and
+    where they do not (72), alone and as an ensemble's member."""
+    ntr, out = 2, []
+    mesh = swe.PlanarHexagonalMesh(nx, nx, 10e3, L)
+    model = swe.ShallowWaterModel(mesh, swe.ShallowWaterParams(**params_dict(10e3, ntr)))
+    model.terms = 79
+    y0 = rich_state(mesh, L, ntr, 2)
+    for rows in (256, 4, 2, 1):
+        print("case", nx, L, rows, flush=True)
+        model.set_launch(rows)
+        s, m, b = upload(mesh, ntr, y0), upload(mesh, ntr, y0), swe.Batch("lsrk", 5)
+        b.add(model, m, 20.0)
+        swe.LSRKStepper(model, 5).run(0.0, 20.0, 2, s)
+        b.run(2)
+        out += [s.download(), m.download()]
+    for got in out[1:]:
+        compare(got, out[0])

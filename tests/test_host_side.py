@@ -22,7 +22,8 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["tall", "rebuild", "keep_stepper", "keep_ensemble", "block_order"])
+@pytest.mark.parametrize("what", ["tall", "rebuild", "keep_stepper", "keep_ensemble", "block_order",
+                                  "tuned_cells"])
 def test_host_side(program, what):
     r = subprocess.run([program, what], capture_output=True, text=True, timeout=120)
     print(r.stdout, r.stderr, flush=True)
