@@ -333,33 +333,42 @@ int omega_model_autotune(omega_model_t model, omega_state_t state, int reps, dou
  * mesh is a regular hexagonal mesh verified against the built-in stencil
  * pattern and nlayers is a multiple of 64 (or 16 / 32 with two levels per
  * thread), 1 forces the general kernels.  omega_model_kernel_variant
- * reports what runs: 6 linear model, 2 specialised, 1 general.  No reference
- * counterpart (performance control only; both give the same bits). */
+ * reports the family: 6 linear model, 2 specialised, 1 general; where bit 5 of
+ * omega_model_kernel_flags is set, that is the family of the kernels with
+ * stored diagnostics.  No reference counterpart (performance control only;
+ * both give the same bits). */
 int omega_model_set_variant(omega_model_t model, int variant);
 int omega_model_kernel_variant(omega_model_t model, int *in_use);
-/* Forms of the two-cells-per-wavefront kernels this model runs: bit 0 set
- * when every coefficient table (mesh and model) is bit-identical at each
- * stencil slot, so a wavefront's two cells share one scalar read of each;
- * bit 1 set when all [rows][levels] arrays have < 2^24 rows, each < 2^24
- * bytes, and < 4 GiB, so row addresses are 32-bit offsets from the array
- * base; bit 2 set when
- * the tendency VJP runs its slot-uniform form (regular hexagonal
- * numbering, an even layer count, every adjoint table bit-identical at
- * each stencil slot; known after the model's first adjoint call); bit 3
- * set when the pair tendency kernel (64k layers) runs a form compiled for
- * the model's term set (7, 15, 79 or 127, both tendencies on); bit 4 set
- * when a step adjoint's stage recomputation also writes the rows its
- * tendency VJPs linearise about (edge PV sums, thickness fluxes and their
- * edges-on-edge sums; the one-cell-per-row kernels at 16 or 32 layers, and
- * the pair kernel with bits 0 and 1), so those VJPs skip their pre-pass.  No reference counterpart (introspection
- * for tests and tuning; the forward results are the same bits either way,
- * and so are the VJP's state cotangents). */
+/* Which kernels this model runs, and in which forms.  Bit 5 set: tendencies of
+ * all fields and steps run the stage kernels, which store no diagnostics in
+ * between (any layer count; a regular hexagonal mesh that closes without a
+ * shift, every coefficient of mesh and model uniform, both tendencies and the
+ * three basic terms on, no drag, forms 7; single-field tendencies, the
+ * auxiliary state alone and a scratch evaluation with momentum del4 still use
+ * the others).  Bits 0, 1 and 3 describe the two-cells-per-wavefront kernels
+ * with stored diagnostics, which a tendency runs where bit 5 is not set: bit 0
+ * set when every coefficient table (mesh and model) is bit-identical at each
+ * stencil slot, so a wavefront's two cells share one scalar read of each; bit
+ * 1 set when all [rows][levels] arrays have < 2^24 rows, each < 2^24 bytes,
+ * and < 4 GiB, so row addresses are 32-bit offsets from the array base; bit 3
+ * set when their tendency kernel (64k layers) has a form compiled for the
+ * model's term set (7, 15, 79 or 127, both tendencies on).  Bit 2 set when the
+ * tendency VJP runs its slot-uniform form (regular hexagonal numbering, an
+ * even layer count, every adjoint table bit-identical at each stencil slot;
+ * known after the model's first adjoint call).  Bit 4 set when a step
+ * adjoint's stage recomputation also writes the rows its tendency VJPs
+ * linearise about (edge PV sums, thickness fluxes and their edges-on-edge
+ * sums: the stage kernels; without them the one-cell-per-row kernels at 16 or
+ * 32 layers, and the pair kernel with bits 0 and 1), so those VJPs skip their
+ * pre-pass.  No reference counterpart (introspection for tests and tuning; the
+ * forward results are the same bits either way, and so are the VJP's state
+ * cotangents). */
 int omega_model_kernel_flags(omega_model_t model, int *flags);
 /* Which of those forms the model may use (bit 0 shared coefficients, bit 1
  * 32-bit offsets, bit 2 the compiled-in term sets, bit 3 the VJP rows
  * written by the stage recomputation; default 15); clearing a bit forces
- * the per-cell, 64-bit, run-time-terms or separate pre-pass form (tests,
- * tuning). */
+ * the per-cell, 64-bit, run-time-terms or separate pre-pass form, and any of
+ * the first three the kernels with stored diagnostics (tests, tuning). */
 int omega_model_set_kernel_forms(omega_model_t model, int forms);
 /* ----------------------------------------------------------------------
  * Time steppers (src/time_integration/time_stepper.hpp:8-38)
@@ -380,8 +389,11 @@ int omega_stepper_coeffs(omega_stepper_t stepper, int *nstages, double *a, doubl
 
 /* Replaces TimeStepper::do_step(t, dt, state)
  * (src/time_integration/rk4.cpp:28-104, src/time_integration/lsrk.cpp:36-89).
- * Without an additional-tendency hook each stage is one diagnostics launch
- * and one fused tendency + stage-update launch. */
+ * Without an additional-tendency hook a stage is fused with its update: one
+ * launch of momentum and thickness and one of the tracers (both in one where
+ * the model is small; two more with momentum del4) where bit 5 of
+ * omega_model_kernel_flags is set, else a diagnostics launch and a tendency
+ * launch (on general meshes one more for the edges' means). */
 int omega_stepper_do_step(omega_stepper_t stepper, double t, double dt, omega_state_t state,
                           omega_stream_t stream);
 

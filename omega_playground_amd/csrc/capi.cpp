@@ -833,16 +833,17 @@ int omega_model_kernel_flags(omega_model_t M, int *flags) {
     const MeshView mv = M->view();
     const ModelCoef mc = M->coef();
     const AdjLayout &al = M->mesh->adj;
+    HexCoef q;
     // the VJP's slot-uniform form (known once the adjoint tables exist)
     const bool adj_uni = al.built && al.fixed && al.uni && M->ect_uniform && mv.coef_uni &&
                          mc.uniform && mv.L % 2 == 0;
-    // the pair tendency kernel's compiled-in term set runs for this model
+    // the pair tendency kernel, where it runs, has this model's term set compiled in
     const bool tset = mv.term_sets && mv.coef_uni && mc.uniform && mv.off32 && mv.hexu_ok &&
                       !M->linear && !general_only(M) && hex_usable(mv, M->lc) &&
                       M->lc.lpt != 1 && mv.L % 64 == 0 && hex_term_set(M->terms) &&
                       !M->params.disable_h_tendency && !M->params.disable_vn_tendency;
     *flags = (mv.coef_uni && mc.uniform ? 1 : 0) | (mv.off32 ? 2 : 0) | (adj_uni ? 4 : 0) |
-             (tset ? 8 : 0) | (stage_writes_pre(M) ? 16 : 0);
+             (tset ? 8 : 0) | (stage_writes_pre(M) ? 16 : 0) | (M->stage_coef(q) ? 32 : 0);
   });
 }
 

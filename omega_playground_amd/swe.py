@@ -564,7 +564,9 @@ class ShallowWaterModel:
         tendency VJP's slot-uniform form (after the first adjoint call);
         bit 3: the pair tendency kernel compiled for the model's term set;
         bit 4: a step adjoint's stage recomputation writes the rows its
-        tendency VJPs linearise about."""
+        tendency VJPs linearise about; bit 5: tendencies and steps run the
+        stage kernels, which store no diagnostics (bits 0, 1 and 3 then
+        describe kernels that they do not run)."""
         v = C.c_int()
         check(lib().omega_model_kernel_flags(self._h, C.byref(v)))
         return v.value

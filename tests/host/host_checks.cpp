@@ -333,12 +333,64 @@ static void tuned_cells() {
       }
 }
 
+// Bit 5 of the kernel flags is set exactly where a tendency launches the
+// stage kernels (no diagnostics launch), whatever else is said.
+static void reports() {
+  struct Case {
+    const char *what;
+    int L, stage;
+    std::function<void(omega_params &)> params;
+    std::function<void(omega_model_t)> set;
+  };
+  auto none = [](auto) {};
+  auto f = [](omega_model_t m) {
+    std::vector<double> f((size_t)16 * 16 * 2, 1e-4);
+    f[3] = 2e-4;
+    ok(omega_model_set_f_vertex(m, f.data()));
+  };
+  const std::vector<Case> cases = {
+      {"default", 64, 1, [](omega_params &) {}, none},
+      {"any layer count", 7, 1, [](omega_params &) {}, none},
+      {"every term", 64, 1, [](omega_params &p) { p.visc_del2 = p.visc_del4 = p.eddy_diff2 = p.eddy_diff4 = 1; }, none},
+      {"forms", 64, 0, [](omega_params &) {}, [](omega_model_t m) { ok(omega_model_set_kernel_forms(m, 3)); }},
+      {"variant", 64, 0, [](omega_params &) {}, [](omega_model_t m) { ok(omega_model_set_variant(m, 1)); }},
+      {"no PV term", 64, 0, [](omega_params &) {}, [](omega_model_t m) { ok(omega_model_set_terms(m, 6)); }},
+      {"drag", 64, 0, [](omega_params &) {}, [](omega_model_t m) { ok(omega_model_set_terms(m, 128 + 7)); }},
+      {"f per vertex", 64, 0, [](omega_params &) {}, f},
+      {"a tendency off", 64, 0, [](omega_params &p) { p.disable_vn_tendency = 1; }, none},
+  };
+  for (const Case &c : cases) {
+    omega_params p = Ensemble::params(1);
+    c.params(p);
+    Ensemble e(1, 16, 16, c.L, p, OMEGA_STEPPER_RK4);
+    c.set(e.models[0]);
+    int flags;
+    ok(omega_model_kernel_flags(e.models[0], &flags));
+    omega_state_t tend;
+    ok(omega_state_create(e.mesh, 1, &tend));
+    ok(omega_timing_enable(1));
+    ok(omega_timing_reset());
+    ok(omega_model_compute_tendency(e.models[0], tend, e.states[0], 0.0, OMEGA_ADD_REPLACE, nullptr));
+    double ms;
+    int64_t diag = 0, tends = 0;
+    ok(omega_timing_read("diag", &ms, &diag));
+    ok(omega_timing_read("tend", &ms, &tends));
+    ok(omega_timing_enable(0));
+    std::printf("%s: flags %d, %d diagnostics launches\n", c.what, flags, (int)diag);
+    CHECK(tends == 1);
+    CHECK(((flags >> 5) & 1) == c.stage);
+    if (!p.disable_vn_tendency) CHECK((diag == 0) == (c.stage == 1));
+    ok(omega_state_destroy(tend));
+  }
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, std::function<void()>> checks = {{"tall", tall}, {"rebuild", rebuild},
                                                               {"keep_stepper", keep_stepper},
                                                               {"keep_ensemble", keep_ensemble},
                                                               {"block_order", block_order},
-                                                              {"tuned_cells", tuned_cells}};
+                                                              {"tuned_cells", tuned_cells},
+                                                              {"reports", reports}};
   CHECK(argc == 2 && checks.count(argv[1]));
   checks.at(argv[1])();
   std::printf("%s ok\n", argv[1]);
