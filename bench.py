@@ -262,11 +262,11 @@ def batched_bench(nmembers: int = 48, nsteps: int = 50, specs=None, label=None, 
     """The ensemble workload: 48 seeded members (nx in {32..192}, 16/32/64
     layers, 1-4 tracers, double vortex with offset centres and random dH),
     LSRK5, 50 steps, del2 viscosity 1e3 and tracer del4 1e9 as the forward
-    workload; one autotuned, graph-captured launch per stage phase for the
-    whole ensemble against a sequential per-member loop (each member its own
-    graph-captured stepper) on the same GPU.  Per-stage bandwidth: the
-    members' algorithmic bytes (18 S per cell-layer-step for LSRK5, S =
-    8 (4 + ntr) B) over the time, as a fraction of the 8 TB/s peak."""
+    workload; the ensemble's graph-captured launches against a sequential
+    per-member loop (each member its own graph-captured stepper) on the same
+    GPU.  Per-stage bandwidth: the members' algorithmic bytes (18 S per
+    cell-layer-step for LSRK5, S = 8 (4 + ntr) B) over the time, as a fraction
+    of the 8 TB/s peak."""
     specs = specs if specs is not None else wl.ensemble_members(nmembers, seed=0)
     nmembers = len(specs)
     members = []
@@ -336,14 +336,17 @@ def batched_bench(nmembers: int = 48, nsteps: int = 50, specs=None, label=None, 
         all(np.array_equal(a, b) for a, b in zip(sb.download(), sl.download()))
         for sb, sl in zip(states_b, states_l))
     info = batch.info()
+    # members on the stage kernels (kernel flag bit 5, no momentum del4) run
+    # launches of their own, to which these shapes do not apply
+    shaped = any(not m[1].kernel_flags() & 32 or m[1].terms & 16 for m in members)
     return {
         "workload": label or (f"{nmembers} members, nx in {{32..192}}, 16/32/64 layers, 1-4 "
                               f"tracers, LSRK5, {nsteps} steps, double vortex, del2 visc 1e3, "
                               f"tracer del4 1e9"),
         "cell_layers": info["cell_layers"],
         "blocks_per_launch": info["blocks_per_launch"],
-        "launch": list(batch.get_launch()),
-        "persistent_blocks_per_cu": batch.get_persistent(),
+        "launch": list(batch.get_launch()) if shaped else None,
+        "persistent_blocks_per_cu": batch.get_persistent() if shaped else None,
         "batched_GBs": alg / t_batch / 1e9,
         "batched_frac": alg / t_batch / 1e9 / HBM_PEAK_GBS,
         "looped_GBs": alg / t_loop / 1e9,

@@ -317,9 +317,10 @@ int omega_model_get_launch(omega_model_t model, int *rows_per_block, int *levels
                            int *xcd_swizzle, int *levels_per_block);
 /* Times reps tendency evaluations of state for each launch shape (cells per
  * block: the default fill, 4 or 2; levels per thread 2 or 1; XCD swizzle on
- * or off), keeps the fastest; *best_ms = its time per evaluation; then
- * times the diagnostics launch alone for its own cells per block (as the
- * tendency launch, the default fill, 4 or 2).  With the environment
+ * or off; where a stage is one launch of all fields only the levels per
+ * thread), keeps the fastest; *best_ms = its time per evaluation; then, where
+ * a tendency has a diagnostics launch, times that for its own cells per block
+ * (as the tendency launch, the default fill, 4 or 2).  With the environment
  * variable OMEGA_TUNE_CACHE naming a file, a choice recorded there for the
  * same model shape (cells, layers, tracers, terms, kernel family) is
  * applied without timing, and a new choice is appended.
@@ -504,9 +505,11 @@ int omega_batch_set_graph(omega_batch_t batch, int enable);
  * del4 pre-pass, tendency + update) is one launch over every member; members
  * on the regular hexagonal mesh run the pattern-specialised operators and
  * the others the general ones inside it.  Members whose models take the stage
- * kernels without stored diagnostics (regular mesh, uniform coefficients, no
+ * kernels without stored diagnostics (bit 5 of omega_model_kernel_flags, no
  * momentum del4) have launches of their own, one for momentum and one for
- * tracers per set of terms, with the shape their models' launches have. */
+ * tracers per set of terms, with 256 threads and the levels per lane and block
+ * order of their models: this setting, the persistent grid and the autotuner
+ * below are for the others. */
 int omega_batch_set_launch(omega_batch_t batch, int threads, int levels_per_thread);
 int omega_batch_get_launch(omega_batch_t batch, int *threads, int *levels_per_thread);
 /* Persistent grid: 0 (default) launches one block per table entry (a
@@ -522,7 +525,8 @@ int omega_batch_get_persistent(omega_batch_t batch, int *blocks_per_cu);
  * shape's time per step.  When the environment variable OMEGA_TUNE_CACHE
  * names a file, a choice recorded there for the same ensemble (stepper and
  * each member's cells, layers, tracers, terms and kernel kind) is applied
- * without timing, and a new choice is appended to the file. */
+ * without timing, and a new choice is appended to the file.  Where the shapes
+ * apply to no member, the setting stays and *best_ms is its time. */
 int omega_batch_autotune(omega_batch_t batch, int reps, double *best_ms, omega_stream_t stream);
 int omega_batch_info(omega_batch_t batch, int *nmembers, int64_t *blocks_per_launch,
                      int64_t *cell_layers);

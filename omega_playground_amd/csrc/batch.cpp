@@ -98,6 +98,12 @@ Real *state_buf(omega_state_s *S, int c, int f) {
   return S->ptr(f);
 }
 
+// Members on the stage kernels without stored diagnostics; their launches have
+// the shapes of their models' own.
+bool in_group(const omega_model_s *M, HexCoef &q) {
+  return !(M->terms & T_VDEL4) && M->stage_coef(q);
+}
+
 void build_tables(omega_batch_s *B) {
   OMEGA_REQUIRE(!B->mem.empty(), "batch: no members");
   // a build that fails leaves neither tables to step with nor graphs that
@@ -130,7 +136,7 @@ void build_tables(omega_batch_s *B) {
     }
     mb.cur0 = S->cur;
     mb.gen = M->gen;
-    if (!(M->terms & T_VDEL4) && M->stage_coef(coef[i])) {
+    if (in_group(M, coef[i])) {
       const MeshView mv = M->view();
       const StageKind k{stage_levels(mv, M->lc), mv.tile.lx, (M->terms & T_VDEL2) != 0,
                         (M->terms & T_TDEL2) != 0, (M->terms & T_TDEL4) != 0};
@@ -509,7 +515,8 @@ int omega_batch_get_launch(omega_batch_t B, int *threads, int *levels_per_thread
 // was.  With OMEGA_TUNE_CACHE naming a file, a choice recorded there for
 // the same ensemble signature (stepper, and per member: cells, layers,
 // tracers, terms, kernel kind) is applied without timing, and a new choice
-// is appended to it.
+// is appended to it.  Where every member has the launches of its group none
+// of it applies: the setting stays, is timed once and not recorded.
 int omega_batch_autotune(omega_batch_t B, int reps, double *best_ms, omega_stream_t stream) {
   return guarded([&] {
     OMEGA_REQUIRE(B && !B->mem.empty(), "batch: no members");
@@ -518,16 +525,25 @@ int omega_batch_autotune(omega_batch_t B, int reps, double *best_ms, omega_strea
     bool even_layers = true;
     for (auto &mb : B->mem) even_layers = even_layers && mb->M->mesh->dm.host.nlayers % 2 == 0;
     // the ensemble's signature for the tuning cache
-    std::string sig = std::to_string(B->kind) + "/" + std::to_string(B->nstages);
+    // (stored: with the kind that a member on the stage kernels would have on
+    // the others, as in records from before they had one of their own)
+    std::string sig = std::to_string(B->kind) + "/" + std::to_string(B->nstages), stored = sig;
+    bool shapes = false; // some member runs the launches that have them
     for (auto &mb : B->mem) {
       const HostMesh &hm = mb->M->mesh->dm.host;
       const bool hx = hex_usable(mb->M->mesh->dm.view(), mb->M->lc) && !general_only(mb->M);
-      sig += ";" + std::to_string(hm.ncells) + ":" + std::to_string(hm.nlayers) + ":" +
-             std::to_string(mb->M->params.ntracers) + ":" + std::to_string(mb->M->terms) + ":" +
-             (hx ? "h" : "g");
+      HexCoef q;
+      const bool grouped = in_group(mb->M, q);
+      shapes = shapes || !grouped;
+      const std::string member = ";" + std::to_string(hm.ncells) + ":" +
+                                 std::to_string(hm.nlayers) + ":" +
+                                 std::to_string(mb->M->params.ntracers) + ":" +
+                                 std::to_string(mb->M->terms) + ":";
+      sig += member + (grouped ? "s" : hx ? "h" : "g");
+      stored += member + (hx ? "h" : "g");
     }
     const char *cache = std::getenv("OMEGA_TUNE_CACHE");
-    if (cache && *cache) {
+    auto recorded = [&](const std::string &wanted) {
       std::ifstream in(cache);
       std::string line;
       while (std::getline(in, line)) {
@@ -535,17 +551,19 @@ int omega_batch_autotune(omega_batch_t B, int reps, double *best_ms, omega_strea
         std::string key;
         int n = 0, t = 0, pc = -1;
         double ms = -1;
-        if (!(ls >> key >> n >> t >> pc >> ms) || key != sig) continue;
+        if (!(ls >> key >> n >> t >> pc >> ms) || key != wanted) continue;
         if ((n == 1 || (n == 2 && even_layers)) && (t == 64 || t == 128 || t == 256) && pc >= 0) {
           B->N = n;
           B->threads = t;
           B->per_cu = pc;
           B->built = false;
           if (best_ms) *best_ms = ms;
-          return;
+          return true;
         }
       }
-    }
+      return false;
+    };
+    if (cache && *cache && (recorded(sig) || recorded(stored))) return;
     // save every member's state
     std::vector<std::array<DBuf<Real>, 3>> saved(B->mem.size());
     std::vector<int> cur(B->mem.size());
@@ -561,8 +579,9 @@ int omega_batch_autotune(omega_batch_t B, int reps, double *best_ms, omega_strea
     }
     double best = -1;
     int bestN = B->N, bestT = B->threads, bestP = B->per_cu;
+    if (!shapes) best = time_steps(B, reps, s);
     for (int N : {2, 1}) {
-      if (N == 2 && !even_layers) continue;
+      if (!shapes || (N == 2 && !even_layers)) continue;
       for (int T : {256, 128, 64})
         for (int P : {0, 4, 8, 16}) {
           B->N = N;
@@ -592,7 +611,7 @@ int omega_batch_autotune(omega_batch_t B, int reps, double *best_ms, omega_strea
                                          hipMemcpyDeviceToDevice, s));
     }
     OMEGA_HIP_CHECK(hipStreamSynchronize(s));
-    if (cache && *cache) {
+    if (shapes && cache && *cache) {
       std::ofstream out(cache, std::ios::app);
       if (out) out << sig << " " << bestN << " " << bestT << " " << bestP << " " << best << "\n";
     }

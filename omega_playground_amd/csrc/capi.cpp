@@ -8,6 +8,7 @@
 #include <sstream>
 
 #include "objects.hpp"
+#include "stage_launch.hpp"
 
 using namespace omega_hip;
 
@@ -691,12 +692,13 @@ int omega_model_set_launch(omega_model_t M, int rows, int lpt, int swizzle, int 
   });
 }
 
-// Times reps tendency evaluations of `state` (diagnostics + tendency
-// launches) for each launch shape -- cells per block (the default fill, 4,
-// 2), levels per thread (2 when the layer count is even, 1) and the XCD
-// swizzle (on, off) -- and keeps the fastest.  OMEGA_TUNE_CACHE works as for
-// omega_batch_autotune, keyed by the model's cells, layers, tracers, terms
-// and kernel family.
+// Times reps tendency evaluations of `state` for each launch shape -- cells
+// per block (the default fill, 4, 2), levels per thread (2 when the layer
+// count is even, 1) and the XCD swizzle (on, off) -- and keeps the fastest.
+// Models small enough for one launch of all fields have only the levels per
+// thread to choose, and only a stored diagnostics launch has its own cells per
+// block.  OMEGA_TUNE_CACHE works as for omega_batch_autotune, keyed by the
+// model's cells, layers, tracers, terms and kernel family.
 int omega_model_autotune(omega_model_t M, omega_state_t state, int reps, double *best_ms,
                          omega_stream_t stream) {
   return guarded([&] {
@@ -706,12 +708,16 @@ int omega_model_autotune(omega_model_t M, omega_state_t state, int reps, double 
     hipStream_t s = as_stream(stream);
     const HostMesh &hm = M->mesh->dm.host;
     const MeshView mv = M->view();
-    const std::string sig = "model;" + std::to_string(hm.ncells) + ":" +
-                            std::to_string(hm.nlayers) + ":" +
-                            std::to_string(M->params.ntracers) + ":" + std::to_string(M->terms) +
-                            ":" + (M->linear ? "l" : hex_usable(mv, M->lc) ? "h" : "g");
+    HexCoef q;
+    const bool stage = M->stage_coef(q); // the stage kernels
+    const std::string shape = "model;" + std::to_string(hm.ncells) + ":" +
+                              std::to_string(hm.nlayers) + ":" +
+                              std::to_string(M->params.ntracers) + ":" +
+                              std::to_string(M->terms) + ":";
+    const std::string stored = shape + (M->linear ? "l" : hex_usable(mv, M->lc) ? "h" : "g");
+    const std::string sig = stage ? shape + "s" : stored;
     const char *cache = std::getenv("OMEGA_TUNE_CACHE");
-    if (cache && *cache) {
+    auto recorded = [&](const std::string &wanted) {
       std::ifstream in(cache);
       std::string line;
       while (std::getline(in, line)) {
@@ -719,7 +725,7 @@ int omega_model_autotune(omega_model_t M, omega_state_t state, int reps, double 
         std::string key;
         int r = 0, l = 0, w = 0, dr = -1;
         double ms = -1;
-        if (!(ls >> key >> r >> l >> w >> ms) || key != sig) continue;
+        if (!(ls >> key >> r >> l >> w >> ms) || key != wanted) continue;
         if (!(ls >> dr) || dr < -1 || dr > 256) dr = -1;
         if (r >= 0 && r <= 256 && (l == 1 || (l == 2 && hm.nlayers % 2 == 0))) {
           M->lc.rows = r;
@@ -728,10 +734,14 @@ int omega_model_autotune(omega_model_t M, omega_state_t state, int reps, double 
           M->lc.drows = dr;
           M->touch();
           if (best_ms) *best_ms = ms;
-          return;
+          return true;
         }
       }
-    }
+      return false;
+    };
+    // records from before the stage kernels had a family of their own still
+    // hold for their models, where there is none of them
+    if (cache && *cache && (recorded(sig) || (stage && recorded(stored)))) return;
     DBuf<Real> t0(state->n[0]), t1(state->n[1]), t2(state->n[2]);
     hipEvent_t a, b;
     OMEGA_HIP_CHECK(hipEventCreate(&a));
@@ -741,8 +751,12 @@ int omega_model_autotune(omega_model_t M, omega_state_t state, int reps, double 
     Launch pick = keep;
     for (int lpt : {2, 1}) {
       if (lpt == 2 && hm.nlayers % 2 != 0) continue;
+      Launch lpt_only = keep;
+      lpt_only.lpt = lpt;
+      const bool one = stage && stage_shares_launch(mv, lpt_only, M->terms, M->params.ntracers);
       for (int rows : {0, 4, 2})
         for (int swz : {1, 0}) {
+          if (one && (rows || !swz)) continue; // the launch has neither
           M->lc = keep;
           M->lc.rows = rows;
           M->lc.lpt = lpt;
@@ -765,17 +779,25 @@ int omega_model_autotune(omega_model_t M, omega_state_t state, int reps, double 
           }
         }
     }
-    // then the diagnostics launch's own block height, timed alone
-    {
+    // then the diagnostics launch's own block height, timed alone (with the
+    // tendency where that comes with edge means, whose launch has it too)
+    if (!stage) {
+      const bool means = M->fh_e.p && mv.ccx;
+      auto diag = [&] {
+        if (means)
+          compute_tendency_ptrs(M, t0.p, t1.p, t2.p, state->ptr(0), state->ptr(1), state->ptr(2),
+                                0.0, OMEGA_ADD_REPLACE, s, 7);
+        else run_diag(M, state->ptr(0), state->ptr(1), state->ptr(2), s);
+      };
       double dbest = -1;
       int dpick = -1;
       for (int dr : {-1, 0, 4, 2}) {
         if (dr >= 0 && dr == pick.rows) continue;
         M->lc = pick;
         M->lc.drows = dr;
-        run_diag(M, state->ptr(0), state->ptr(1), state->ptr(2), s);
+        diag();
         OMEGA_HIP_CHECK(hipEventRecord(a, s));
-        for (int i = 0; i < reps; ++i) run_diag(M, state->ptr(0), state->ptr(1), state->ptr(2), s);
+        for (int i = 0; i < reps; ++i) diag();
         OMEGA_HIP_CHECK(hipEventRecord(b, s));
         OMEGA_HIP_CHECK(hipEventSynchronize(b));
         float ms = 0;

@@ -187,6 +187,17 @@ void stage_launch(const MeshView &m, const Launch &lc, int N, const HexCoef &q, 
   t.d = d;
 }
 
+bool stage_shares_launch(const MeshView &m, const Launch &lc, int terms, int ntr) {
+  if (ntr <= 0 || (terms & T_VDEL4)) return false;
+  StageArgs a{};
+  a.ntr = ntr;
+  const int N = stage_levels(m, lc);
+  StageLaunch p;
+  TileLaunch t;
+  stage_launch(m, lc, N, HexCoef{}, a, DiagOut{}, p, t);
+  return stage_one_launch(N, p, t);
+}
+
 void launch_stage_hex(const MeshView &m, const Launch &lc, const HexCoef &q, const StageArgs &a,
                       const DiagOut &d, bool emit, hipStream_t s, const PreOut *pre) {
   TimerScope ts("tend", s);

@@ -51,6 +51,8 @@ constexpr int kFewTiles = 512;
 // Both in one launch, where that is the faster one (kernels_stage_both.hip);
 // false: nothing launched.
 bool stage_one_launch(int N, const StageLaunch &p, const TileLaunch &t);
+// whether the stages of a model take it
+bool stage_shares_launch(const MeshView &m, const Launch &lc, int terms, int ntr);
 bool launch_stage_both(int N, int lx, const StageLaunch &p, const TileLaunch &t, bool emit, bool pre,
                        hipStream_t s);
 

@@ -6,10 +6,14 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <fstream>
 #include <functional>
+#include <iterator>
 #include <map>
 #include <string>
 #include <vector>
+
+#include <unistd.h>
 
 #include "stage_launch.hpp"
 
@@ -384,13 +388,81 @@ static void reports() {
   }
 }
 
+static std::string contents(const std::string &path) {
+  std::ifstream in(path);
+  return std::string(std::istreambuf_iterator<char>(in), {});
+}
+
+// The tuners time shapes that change what runs and nothing else, and their
+// records tell the stage kernels from the others; records of the others are
+// still read where there is none of the stage kernels.
+static void tuning() {
+  char dir[] = "/tmp/omega_tuning_XXXXXX";
+  CHECK(mkdtemp(dir));
+  const std::string cache = std::string(dir) + "/cache";
+  setenv("OMEGA_TUNE_CACHE", cache.c_str(), 1);
+  // cells, levels, shapes to time: levels per lane, and cells per block and
+  // block order where momentum has a launch of its own
+  struct Size {
+    int nx, L, launches, shapes;
+  };
+  for (const Size &c : {Size{16, 64, 1, 2}, Size{16, 7, 1, 1}, Size{128, 64, 2, 12}}) {
+    for (const char *forms : {"s", "h", ""}) {
+      std::remove(cache.c_str());
+      Ensemble e(1, c.nx, c.nx, c.L, Ensemble::params(2), OMEGA_STEPPER_RK4);
+      const std::string key = "model;" + std::to_string(c.nx * c.nx) + ":" + std::to_string(c.L) + ":2:7:";
+      const std::string old = c.L == 64 ? "h" : "g";
+      // another family's record comes first in the file
+      if (*forms) std::ofstream(cache) << key << old << " 4 1 0 9.5 -1\n";
+      if (*forms == 's') std::ofstream(cache, std::ios::app) << key << "s 2 1 1 0.5 -1\n";
+      double ms = 0;
+      const auto n = launched(0, [&] { ok(omega_model_autotune(e.models[0], e.states[0], 3, &ms, nullptr)); });
+      std::printf("%d x %d cells, %d levels, records '%s': %zu launches, %g ms\n%s", c.nx, c.nx, c.L, forms,
+                  n.size(), ms, contents(cache).c_str());
+      int rows, lpt, order;
+      ok(omega_model_get_launch(e.models[0], &rows, &lpt, &order, nullptr));
+      if (*forms == 's') CHECK(n.empty() && ms == 0.5 && rows == 2 && order == 1);
+      else if (*forms) CHECK(n.empty() && ms == 9.5 && rows == 4 && order == 0);
+      else {
+        CHECK((int)n.size() == c.shapes * c.launches * (1 + 3));
+        CHECK(contents(cache).rfind(key + "s ", 0) == 0);
+      }
+    }
+  }
+  // an ensemble of such members alone: nothing to choose
+  std::remove(cache.c_str());
+  {
+    Ensemble e(3, 16, 16, 64, Ensemble::params(2), OMEGA_STEPPER_RK4);
+    ok(omega_batch_set_launch(e.batch, 128, 1));
+    double ms = 0;
+    const auto n = launched(0, [&] { ok(omega_batch_autotune(e.batch, 3, &ms, nullptr)); });
+    int threads, lpt;
+    ok(omega_batch_get_launch(e.batch, &threads, &lpt));
+    std::printf("ensemble: %zu launches, %g ms, %d threads\n", n.size(), ms, threads);
+    CHECK(n.size() == 4 * 2 * (1 + 3) && ms > 0 && threads == 128 && lpt == 1);
+    CHECK(contents(cache).empty());
+  }
+  // with a member on the other kernels: every shape
+  {
+    Ensemble e(3, 16, 16, 64, Ensemble::params(2), OMEGA_STEPPER_RK4);
+    ok(omega_model_set_kernel_forms(e.models[1], 3));
+    const auto n = launched(0, [&] { ok(omega_batch_autotune(e.batch, 3, nullptr, nullptr)); });
+    CHECK(n.size() == 24 * 4 * (2 + 2) * (1 + 3));
+    CHECK(contents(cache).rfind("0/4;256:64:2:7:s;256:64:2:7:h;256:64:2:7:s ", 0) == 0);
+  }
+  std::remove(cache.c_str());
+  CHECK(rmdir(dir) == 0);
+  unsetenv("OMEGA_TUNE_CACHE");
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, std::function<void()>> checks = {{"tall", tall}, {"rebuild", rebuild},
                                                               {"keep_stepper", keep_stepper},
                                                               {"keep_ensemble", keep_ensemble},
                                                               {"block_order", block_order},
                                                               {"tuned_cells", tuned_cells},
-                                                              {"reports", reports}};
+                                                              {"reports", reports},
+                                                              {"tuning", tuning}};
   CHECK(argc == 2 && checks.count(argv[1]));
   checks.at(argv[1])();
   std::printf("%s ok\n", argv[1]);
