@@ -507,7 +507,7 @@ int omega_batch_set_graph(omega_batch_t batch, int enable);
  * the others the general ones inside it.  Members whose models take the stage
  * kernels without stored diagnostics (bit 5 of omega_model_kernel_flags, no
  * momentum del4) have launches of their own, one for momentum and one for
- * tracers per set of terms, with 256 threads and the levels per lane and block
+ * tracers for those of each number of levels per lane, with 256 threads and the levels per lane and block
  * order of their models: this setting, the persistent grid and the autotuner
  * below are for the others. */
 int omega_batch_set_launch(omega_batch_t batch, int threads, int levels_per_thread);

@@ -2,9 +2,10 @@
 // mesh, layer count, tracer count, coefficients and time step -- advanced
 // together.  Members on the stage kernels without stored diagnostics
 // (kernels_stage.hip) have one momentum and one tracer launch per stage and
-// set of terms (16 mixed members, 64 layers at most, LSRK5: 2.05 -> 1.23 ms
-// per step against the launches below).  For the others every stage phase (diagnostics, momentum del4 pre-pass,
-// tendency + update) is one launch over all members' blocks, driven by a
+// number of levels per lane (16 mixed members, 64 layers at most, LSRK5: 2.05
+// -> 0.97 ms per step against the launches below).  For the others every stage
+// phase (diagnostics, momentum del4 pre-pass, tendency + update) is one launch
+// over all members' blocks, driven by a
 // table of per-member descriptors built once per (step parity, stage); the
 // step can be captured in a HIP graph.  The stage updates are the fused
 // epilogues of the single-model steppers (rk4.cpp:28-104, lsrk.cpp:36-89),
@@ -48,8 +49,8 @@ struct omega_batch_s {
   bool any_vdel4 = false;
   DBuf<int> blk;
   DBuf<BatchMember> desc; // [parity][stage][member]
-  // members on the stage kernels without stored diagnostics, by what their
-  // launches have compiled in; the tables above hold the others
+  // members on the stage kernels without stored diagnostics, by the levels per
+  // lane of their launches; the tables above hold the others
   struct Group {
     StageKind kind;
     std::vector<int> members;
@@ -138,13 +139,19 @@ void build_tables(omega_batch_s *B) {
     mb.gen = M->gen;
     if (in_group(M, coef[i])) {
       const MeshView mv = M->view();
-      const StageKind k{stage_levels(mv, M->lc), mv.tile.lx, (M->terms & T_VDEL2) != 0,
-                        (M->terms & T_TDEL2) != 0, (M->terms & T_TDEL4) != 0};
+      const bool v2 = M->terms & T_VDEL2, d2 = M->terms & T_TDEL2, d4 = M->terms & T_TDEL4;
+      StageKind k{stage_levels(mv, M->lc), v2, mv.tile.lx, d2, d4};
       size_t j = 0;
-      while (j < B->groups.size() && !(B->groups[j]->kind == k)) ++j;
+      while (j < B->groups.size() && B->groups[j]->kind.N != k.N) ++j;
       if (j == B->groups.size()) {
         B->groups.push_back(std::make_unique<omega_batch_s::Group>());
         B->groups[j]->kind = k;
+      }
+      StageKind &g = B->groups[j]->kind;
+      if (g.v2 != k.v2) g.v2 = kAny;
+      if (g.lx != k.lx || g.d2 != k.d2 || g.d4 != k.d4) {
+        g.lx = g.d2 = kAny;
+        g.d4 = g.d4 || k.d4;
       }
       B->groups[j]->members.push_back(i);
       own[i] = (int)j;

@@ -43,16 +43,25 @@ template <class T> __device__ __forceinline__ const T &constant_at(const T *t, i
   return *(const T *)((const __attribute__((address_space(4))) T *)t + i);
 }
 
-// Ensemble forms: block b belongs to member who[b] (-1: none), whose parameter
+// Ensemble form: block b belongs to member who[b] (-1: none), whose parameter
 // block is read in place through scalar loads and whose blocks start at a
 // multiple of 8, so that each XCD takes a contiguous eighth of every member.
-template <int N, bool V2, bool EMIT>
+// Members of any terms share the launch (StageKind): with a launch for each
+// set of terms small members waited for one another, 24 members of 576 cells
+// with 8 sets of terms and 3 layer counts 1660 us per LSRK5 step, 107 so.
+template <int N, int V2, bool EMIT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N == 1 ? 4 : 2)))
     k_batch_mom(const StageLaunch *__restrict__ desc, const int *__restrict__ who) {
   const int w = uniform(who[blockIdx.x]);
   if (w < 0) return;
   const StageLaunch &p = constant_at(desc, w);
-  stage_mom<N, V2, false, EMIT>(p, logical_block((int)blockIdx.x - p.block0, p.tiles, p.swz));
+  const int entry = logical_block((int)blockIdx.x - p.block0, p.tiles, p.swz);
+  if constexpr (V2 != kAny) {
+    stage_mom<N, V2 != 0, false, EMIT>(p, entry);
+  } else {
+    if (p.a.terms & T_VDEL2) stage_mom<N, true, false, EMIT>(p, entry);
+    else stage_mom<N, false, false, EMIT>(p, entry);
+  }
 }
 
 // The edge Laplacian: of the velocity (FINAL false), then of that result,
@@ -86,16 +95,52 @@ __global__ void __launch_bounds__(256) k_stage_lap(StageLaunch p) {
 template <int N, int LX, int TW, int TH, bool D2, bool D4, bool EMIT>
 __global__ void __launch_bounds__(LX *TW *TH) __attribute__((amdgpu_waves_per_eu(N == 2 ? 3 : 4)))
     k_stage_tile(TileLaunch p) {
-  stage_tile<N, LX, TW, TH, D2, D4, EMIT>(p, xcd_entry(p.work, p.swz), (int)blockIdx.y * p.per_block);
+  __shared__ TileRows<N, LX, TW, TH, D4> rows;
+  stage_tile<N, LX, TW, TH, D2, D4, EMIT>(p, xcd_entry(p.work, p.swz), (int)blockIdx.y * p.per_block,
+                                          rows);
 }
 
-template <int N, int LX, int TW, int TH, bool D2, bool D4, bool EMIT>
-__global__ void __launch_bounds__(LX *TW *TH) __attribute__((amdgpu_waves_per_eu(N == 2 ? 3 : 4)))
+// Ensemble form (k_batch_mom); tiles of all shapes share the LDS.  D4: some
+// member has del4 (without it the bodies leave room for four waves per SIMD).
+template <int N, int LX, int TW, int TH, int D2, bool D4, bool EMIT>
+__device__ __forceinline__ void batch_tile(const TileLaunch &p, int entry, char *mem) {
+  auto body = [&](auto D2_, auto D4_) {
+    constexpr bool d2 = decltype(D2_)::value, d4 = decltype(D4_)::value;
+    // without del4 there is no Laplacian to emit
+    stage_tile<N, LX, TW, TH, d2, d4, EMIT && d4>(p, entry, 0,
+                                                  *reinterpret_cast<TileRows<N, LX, TW, TH, d4> *>(mem));
+  };
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+  if constexpr (D2 != kAny) {
+    body(std::bool_constant<D2 != 0>{}, std::bool_constant<D4>{});
+  } else {
+    const bool d2 = p.a.terms & T_TDEL2;
+    if (D4 && (p.a.terms & T_TDEL4)) {
+      if (d2) body(yes, std::bool_constant<D4>{});
+      else body(no, std::bool_constant<D4>{});
+    } else if (d2) {
+      body(yes, no);
+    } else {
+      body(no, no);
+    }
+  }
+}
+
+template <int N, int LX, int D2, bool D4, bool EMIT>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N == 2 && (D4 || D2 != kAny) ? 3 : 4)))
     k_batch_tile(const TileLaunch *__restrict__ desc, const int *__restrict__ who) {
+  constexpr size_t of[3] = {sizeof(TileRows<N, 4, 8, 8, D4>), sizeof(TileRows<N, 2, 16, 8, D4>),
+                            sizeof(TileRows<N, 1, 16, 16, D4>)};
+  __shared__ alignas(16) char mem[LX == 4 ? of[0] : LX == 2 ? of[1] : LX == 1 ? of[2]
+                                                                  : std::max({of[0], of[1], of[2]})];
   const int w = uniform(who[blockIdx.x]);
   if (w < 0) return;
   const TileLaunch &p = constant_at(desc, w);
-  stage_tile<N, LX, TW, TH, D2, D4, EMIT>(p, logical_block((int)blockIdx.x - p.block0, p.work, p.swz), 0);
+  const int entry = logical_block((int)blockIdx.x - p.block0, p.work, p.swz);
+  if (LX == 4 || (LX == kAny && p.lx == 4)) batch_tile<N, 4, 8, 8, D2, D4, EMIT>(p, entry, mem);
+  else if (LX == 2 || (LX == kAny && p.lx == 2)) batch_tile<N, 2, 16, 8, D2, D4, EMIT>(p, entry, mem);
+  else batch_tile<N, 1, 16, 16, D2, D4, EMIT>(p, entry, mem);
 }
 
 using StageFn = void (*)(StageLaunch);
@@ -111,34 +156,21 @@ template <int N> StageFn pick_pre(bool v2, bool v4) {
 }
 
 // without del4 there is no Laplacian to emit
-template <int N, int LX, int TW, int TH, bool EMIT, bool BATCH> auto pick_shape(bool d2, bool d4) {
-  if constexpr (BATCH) {
-    if (d4)
-      return d2 ? k_batch_tile<N, LX, TW, TH, true, true, EMIT>
-                : k_batch_tile<N, LX, TW, TH, false, true, EMIT>;
-    return d2 ? k_batch_tile<N, LX, TW, TH, true, false, false>
-              : k_batch_tile<N, LX, TW, TH, false, false, false>;
-  } else {
-    if (d4)
-      return d2 ? k_stage_tile<N, LX, TW, TH, true, true, EMIT>
-                : k_stage_tile<N, LX, TW, TH, false, true, EMIT>;
-    return d2 ? k_stage_tile<N, LX, TW, TH, true, false, false>
-              : k_stage_tile<N, LX, TW, TH, false, false, false>;
-  }
+template <int N, int LX, int TW, int TH, bool EMIT> auto pick_shape(bool d2, bool d4) {
+  if (d4)
+    return d2 ? k_stage_tile<N, LX, TW, TH, true, true, EMIT>
+              : k_stage_tile<N, LX, TW, TH, false, true, EMIT>;
+  return d2 ? k_stage_tile<N, LX, TW, TH, true, false, false>
+            : k_stage_tile<N, LX, TW, TH, false, false, false>;
 }
-template <bool BATCH, int N, bool EMIT> auto pick_tile_of(int lx, bool d2, bool d4) {
-  if (lx == 4) return pick_shape<N, 4, 8, 8, EMIT, BATCH>(d2, d4);
-  if (lx == 2) return pick_shape<N, 2, 16, 8, EMIT, BATCH>(d2, d4);
-  return pick_shape<N, 1, 16, 16, EMIT, BATCH>(d2, d4);
+template <int N, bool EMIT> auto pick_tile_of(int lx, bool d2, bool d4) {
+  if (lx == 4) return pick_shape<N, 4, 8, 8, EMIT>(d2, d4);
+  if (lx == 2) return pick_shape<N, 2, 16, 8, EMIT>(d2, d4);
+  return pick_shape<N, 1, 16, 16, EMIT>(d2, d4);
 }
-template <bool BATCH> auto pick_tile(int N, int lx, bool d2, bool d4, bool emit) {
-  if (N == 2) return emit ? pick_tile_of<BATCH, 2, true>(lx, d2, d4) : pick_tile_of<BATCH, 2, false>(lx, d2, d4);
-  return emit ? pick_tile_of<BATCH, 1, true>(lx, d2, d4) : pick_tile_of<BATCH, 1, false>(lx, d2, d4);
-}
-
-template <int N> auto pick_batch_mom(bool v2, bool emit) {
-  if (emit) return v2 ? k_batch_mom<N, true, true> : k_batch_mom<N, false, true>;
-  return v2 ? k_batch_mom<N, true, false> : k_batch_mom<N, false, false>;
+auto pick_tile(int N, int lx, bool d2, bool d4, bool emit) {
+  if (N == 2) return emit ? pick_tile_of<2, true>(lx, d2, d4) : pick_tile_of<2, false>(lx, d2, d4);
+  return emit ? pick_tile_of<1, true>(lx, d2, d4) : pick_tile_of<1, false>(lx, d2, d4);
 }
 
 constexpr int kTileThreads = 256; // every tile shape's
@@ -182,6 +214,7 @@ void stage_launch(const MeshView &m, const Launch &lc, int N, const HexCoef &q, 
   t.nc = m.nc;
   t.L = m.L;
   t.per_block = a.ntr;
+  t.lx = tv.lx;
   t.swz = lc.swizzle;
   t.a = a;
   t.d = d;
@@ -233,7 +266,7 @@ void launch_stage_hex(const MeshView &m, const Launch &lc, const HexCoef &q, con
     // where the tiles alone leave the chip short of blocks each tracer has
     // its own
     if (t.work < kFewTiles) t.per_block = 1;
-    hipLaunchKernelGGL(pick_tile<false>(N, m.tile.lx, d2, d4, emit),
+    hipLaunchKernelGGL(pick_tile(N, m.tile.lx, d2, d4, emit),
                        dim3(t.work, (a.ntr + t.per_block - 1) / t.per_block), dim3(kTileThreads), 0,
                        s, t);
   }
@@ -262,19 +295,42 @@ bool launch_stage_rows(const MeshView &m, const Launch &lc, const HexCoef &q, St
   return true;
 }
 
+namespace {
+using BatchMomFn = void (*)(const StageLaunch *, const int *);
+using BatchTileFn = void (*)(const TileLaunch *, const int *);
+
+template <int N, bool EMIT> BatchMomFn pick_batch_mom(const StageKind &k) {
+  if (k.v2 == kAny) return k_batch_mom<N, kAny, EMIT>;
+  return k.v2 ? k_batch_mom<N, 1, EMIT> : k_batch_mom<N, 0, EMIT>;
+}
+template <int N, int LX> BatchTileFn pick_batch_shape(int d2, bool d4, bool emit) {
+  if (!d4) return d2 ? k_batch_tile<N, LX, 1, false, false> : k_batch_tile<N, LX, 0, false, false>;
+  if (emit) return d2 ? k_batch_tile<N, LX, 1, true, true> : k_batch_tile<N, LX, 0, true, true>;
+  return d2 ? k_batch_tile<N, LX, 1, true, false> : k_batch_tile<N, LX, 0, true, false>;
+}
+template <int N> BatchTileFn pick_batch_tile(const StageKind &k, bool emit) {
+  if (k.lx == 4) return pick_batch_shape<N, 4>(k.d2, k.d4, emit);
+  if (k.lx == 2) return pick_batch_shape<N, 2>(k.d2, k.d4, emit);
+  if (k.lx == 1) return pick_batch_shape<N, 1>(k.d2, k.d4, emit);
+  if (!k.d4) return k_batch_tile<N, kAny, kAny, false, false>;
+  return emit ? k_batch_tile<N, kAny, kAny, true, true> : k_batch_tile<N, kAny, kAny, true, false>;
+}
+} // namespace
+
 void launch_stage_batch(const StageKind &k, const StageLaunch *desc, const int *who, int n, bool emit,
                         hipStream_t s) {
   TimerScope ts("batch_tend", s);
-  hipLaunchKernelGGL(k.N == 2 ? pick_batch_mom<2>(k.v2, emit) : pick_batch_mom<1>(k.v2, emit),
-                     dim3(n), dim3(256), 0, s, desc, who);
+  const BatchMomFn f = k.N == 2 ? (emit ? pick_batch_mom<2, true>(k) : pick_batch_mom<2, false>(k))
+                                : (emit ? pick_batch_mom<1, true>(k) : pick_batch_mom<1, false>(k));
+  hipLaunchKernelGGL(f, dim3(n), dim3(256), 0, s, desc, who);
   OMEGA_HIP_CHECK(hipGetLastError());
 }
 
 void launch_tile_batch(const StageKind &k, const TileLaunch *desc, const int *who, int n, bool emit,
                        hipStream_t s) {
   TimerScope ts("batch_tracers", s);
-  hipLaunchKernelGGL(pick_tile<true>(k.N, k.lx, k.d2, k.d4, emit), dim3(n), dim3(kTileThreads), 0, s,
-                     desc, who);
+  const BatchTileFn f = k.N == 2 ? pick_batch_tile<2>(k, emit) : pick_batch_tile<1>(k, emit);
+  hipLaunchKernelGGL(f, dim3(n), dim3(kTileThreads), 0, s, desc, who);
   OMEGA_HIP_CHECK(hipGetLastError());
 }
 

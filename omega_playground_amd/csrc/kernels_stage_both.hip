@@ -22,8 +22,9 @@ __global__ void __launch_bounds__(256)
     stage_mom<N, V2, false, E != kNothing, E == kPre>(p, b);
   } else {
     // tiles of all tracers of a group, then the next group
+    __shared__ TileRows<N, LX, TW, TH, D4> rows;
     const int w = b - p.tiles, group = uniform(w / t.work);
-    stage_tile<N, LX, TW, TH, D2, D4, E != kNothing>(t, w - group * t.work, group * t.per_block);
+    stage_tile<N, LX, TW, TH, D2, D4, E != kNothing>(t, w - group * t.work, group * t.per_block, rows);
   }
 }
 

@@ -91,6 +91,15 @@ __device__ __forceinline__ void stage_mom(const StageLaunch &p, int entry) {
   epilogue<N>(a, a.h, idx, T);
 }
 
+// A tile's rows in LDS: thickness, tracer ratio and Laplacian, and its cells
+template <int N, int LX, int TW, int TH, bool D4> struct TileRows {
+  static constexpr int HALO = D4 ? 2 : 1;
+  static constexpr int NP = (TW + 2 * HALO) * (TH + 2 * HALO), PLANE = NP * LX * N;
+  alignas(16) double h[PLANE];
+  double ratio[PLANE], lap[D4 ? PLANE : 1];
+  int ids[NP];
+};
+
 // ---------------------------------------------------------------------------
 // Tracers: a block stages a tile of the lattice, TW x TH cells with one ring
 // of halo (two with del4) and LX lanes of N levels, in LDS, so that a
@@ -105,14 +114,15 @@ __device__ __forceinline__ void stage_mom(const StageLaunch &p, int entry) {
 // SIMD faster than four with 13 registers spilled (6.3 against 7.0).
 // ---------------------------------------------------------------------------
 template <int N, int LX, int TW, int TH, bool D2, bool D4, bool EMIT>
-__device__ __forceinline__ void stage_tile(const TileLaunch &p, int w, int l0) {
+__device__ __forceinline__ void stage_tile(const TileLaunch &p, int w, int l0,
+                                           TileRows<N, LX, TW, TH, D4> &rows) {
   constexpr int HALO = D4 ? 2 : 1, PW = TW + 2 * HALO, PH = TH + 2 * HALO, NP = PW * PH;
   constexpr int CELLS = TW * TH, R = (NP + CELLS - 1) / CELLS;
   constexpr int RING = 2 * (TW + 2) + 2 * TH; // the first ring round the tile
   static_assert(RING <= CELLS, "one place of the ring per row of lanes");
-  constexpr int S = LX * N, PLANE = NP * S; // doubles per place and per array
-  __shared__ double Hs[PLANE], Ns[PLANE], Ds[D4 ? PLANE : 1];
-  __shared__ int ids[NP];
+  constexpr int S = LX * N; // doubles per place and array
+  double *const Hs = rows.h, *const Ns = rows.ratio, *const Ds = rows.lap;
+  int *const ids = rows.ids;
   const int tile = uniform(w / p.nch), ch = w - tile * p.nch;
   const int ln = (int)threadIdx.x % LX, row = (int)threadIdx.x / LX;
   const int L = p.L, k = (ch * LX + ln) * N;

@@ -186,6 +186,15 @@ struct Ensemble {
   }
 };
 
+// The launches of f, with as many bytes of their first arguments
+template <class F> static std::vector<fake::Launched> launched(size_t arg_bytes, F &&f) {
+  fake::launches.clear();
+  fake::arg_bytes = arg_bytes;
+  f();
+  fake::arg_bytes = 0;
+  return fake::launches;
+}
+
 // A step whose tables cannot be rebuilt fails and leaves no graph of the old
 // ones; the step after it does all of its work.
 static void rebuild() {
@@ -193,14 +202,13 @@ static void rebuild() {
     for (int fail = 0;; ++fail) {
       Ensemble e(2, 6, 4, 8, Ensemble::params(1), OMEGA_STEPPER_RK4);
       ok(omega_batch_set_graph(e.batch, graph));
-      ok(omega_batch_step(e.batch, nullptr));
+      const size_t want = launched(0, [&] { ok(omega_batch_step(e.batch, nullptr)); }).size();
       fake::launches.clear();
       ok(omega_model_set_terms(e.models[1], 7 + 8)); // the tables are now out of date
       fake::fail_after = fail;
       const bool failed = omega_batch_step(e.batch, nullptr) != OMEGA_OK;
       fake::fail_after = -1;
       std::printf("graph %d, allocation %d fails: %d\n", graph, fail, (int)failed);
-      const size_t want = 4 * (2 + 2); // momentum and tracers of two sets of terms per stage
       if (!failed) {
         CHECK(fake::launches.size() == want && fail > 0);
         break;
@@ -275,15 +283,6 @@ static void keep_ensemble() {
         }
       }
   CHECK(fake::bytes == 0);
-}
-
-// The launches of f, with as many bytes of their first arguments
-template <class F> static std::vector<fake::Launched> launched(size_t arg_bytes, F &&f) {
-  fake::launches.clear();
-  fake::arg_bytes = arg_bytes;
-  f();
-  fake::arg_bytes = 0;
-  return fake::launches;
 }
 
 // The block order set with omega_model_set_launch reaches the stage kernels,
@@ -455,6 +454,44 @@ static void tuning() {
   unsetenv("OMEGA_TUNE_CACHE");
 }
 
+// An ensemble's stage is two launches for all its members of even layer counts
+// and two for those of odd ones, whatever their terms, layers and tiles.
+static void few_launches() {
+  omega_batch_t batch;
+  ok(omega_batch_create(OMEGA_STEPPER_RK4, 4, &batch));
+  std::vector<omega_mesh_t> meshes;
+  std::vector<omega_model_t> models;
+  std::vector<omega_state_t> states;
+  auto add = [&](int L, int ntr, int terms) {
+    omega_mesh_t mesh;
+    omega_model_t m;
+    omega_state_t s;
+    const omega_params p = Ensemble::params(ntr);
+    ok(omega_mesh_create_planar_hex(10, 8, 1e4, L, OMEGA_ORDER_HILBERT, &mesh));
+    ok(omega_model_create(mesh, &p, &m));
+    ok(omega_model_set_terms(m, terms));
+    ok(omega_state_create(mesh, ntr, &s));
+    ok(omega_batch_add(batch, m, s, 10.0, nullptr));
+    meshes.push_back(mesh);
+    models.push_back(m);
+    states.push_back(s);
+  };
+  for (int L : {2, 4, 8, 64})
+    for (int terms : {7, 15, 39, 47, 71, 79, 103, 111}) add(L, 1 + L % 3, terms);
+  size_t n = launched(0, [&] { ok(omega_batch_step(batch, nullptr)); }).size();
+  std::printf("even layer counts: %zu launches a step\n", n);
+  CHECK(n == 4 * 2);
+  for (int L : {1, 5})
+    for (int terms : {7, 111}) add(L, 2, terms);
+  n = launched(0, [&] { ok(omega_batch_step(batch, nullptr)); }).size();
+  std::printf("and odd ones: %zu launches a step\n", n);
+  CHECK(n == 4 * 4);
+  ok(omega_batch_destroy(batch));
+  for (auto s : states) ok(omega_state_destroy(s));
+  for (auto m : models) ok(omega_model_destroy(m));
+  for (auto m : meshes) ok(omega_mesh_destroy(m));
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, std::function<void()>> checks = {{"tall", tall}, {"rebuild", rebuild},
                                                               {"keep_stepper", keep_stepper},
@@ -462,7 +499,8 @@ int main(int argc, char **argv) {
                                                               {"block_order", block_order},
                                                               {"tuned_cells", tuned_cells},
                                                               {"reports", reports},
-                                                              {"tuning", tuning}};
+                                                              {"tuning", tuning},
+                                                              {"few_launches", few_launches}};
   CHECK(argc == 2 && checks.count(argv[1]));
   checks.at(argv[1])();
   std::printf("%s ok\n", argv[1]);

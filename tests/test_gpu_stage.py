@@ -291,3 +291,29 @@ def test_cells_per_block_do_not_change_bits(nx, L):
         out += [s.download(), m.download()]
     for got in out[1:]:
         compare(got, out[0])
+
+
+@pytest.mark.parametrize("kind", ["rk4", "lsrk"])
+@pytest.mark.parametrize("del4", [True, False])
+def test_ensemble_of_any_terms_and_layers_bitwise(kind, del4):
+    """Members of every set of terms, tile shape and levels per lane share
+    their launches and end with the bits of their solo steps."""
+    b, members = swe.Batch(kind, 5), []
+    sets = [7 + x for x in (0, 8, 32, 40) + ((64, 72, 96, 104) if del4 else ())]
+    for L in (1, 2, 3, 4, 10, 66):
+        for i, terms in enumerate(sets):
+            nx, ny, ntr = 8 + i, 10 + 2 * (L % 3), (i + L) % 4
+            mesh = swe.PlanarHexagonalMesh(nx, ny, 10e3, L)
+            model = swe.ShallowWaterModel(mesh, swe.ShallowWaterParams(**params_dict(10e3, ntr)))
+            model.terms = terms
+            y0 = rich_state(mesh, L, ntr, L + i)
+            s = upload(mesh, ntr, y0)
+            b.add(model, s, 15.0)
+            members.append((mesh, model, ntr, y0, s))
+    print("case", kind, del4, len(members), flush=True)
+    b.set_graph(True)
+    b.run(3)
+    for mesh, model, ntr, y0, s in members:
+        solo = upload(mesh, ntr, y0)
+        (swe.RK4Stepper(model) if kind == "rk4" else swe.LSRKStepper(model, 5)).run(0.0, 15.0, 3, solo)
+        compare(s.download(), solo.download(), mesh.nlayers, model.terms)
