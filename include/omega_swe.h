@@ -508,8 +508,10 @@ int omega_batch_set_graph(omega_batch_t batch, int enable);
  * kernels without stored diagnostics (bit 5 of omega_model_kernel_flags, no
  * momentum del4) have launches of their own, one for momentum and one for
  * tracers for those of each number of levels per lane, with 256 threads and the levels per lane and block
- * order of their models: this setting, the persistent grid and the autotuner
- * below are for the others. */
+ * order of their models, beside those of the others on a stream of the
+ * batch's (next to others and below 262144 cells and levels in all they run
+ * with them): this setting, the persistent grid and the autotuner below are
+ * for the others. */
 int omega_batch_set_launch(omega_batch_t batch, int threads, int levels_per_thread);
 int omega_batch_get_launch(omega_batch_t batch, int *threads, int *levels_per_thread);
 /* Persistent grid: 0 (default) launches one block per table entry (a

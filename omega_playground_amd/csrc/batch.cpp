@@ -60,6 +60,10 @@ struct omega_batch_s {
     DBuf<TileLaunch> tile;
   };
   std::vector<std::unique_ptr<Group>> groups;
+  // where there are both, the groups' launches run beside the others' on a
+  // stream of the batch's own, from fork to join
+  hipStream_t side = nullptr;
+  hipEvent_t fork = nullptr, join = nullptr;
   bool use_graph = false;
   std::map<int, hipGraphExec_t> graphs;
   // omega_batch_adjoint_run's stacked mesh, model, stepper and states, kept
@@ -71,7 +75,15 @@ struct omega_batch_s {
     omega_params params{};
   } stacked_for;
 
-  ~omega_batch_s() { drop_graphs(); }
+  ~omega_batch_s() {
+    drop_graphs();
+    if (side) {
+      (void)hipStreamSynchronize(side);
+      (void)hipStreamDestroy(side);
+    }
+    for (hipEvent_t e : {fork, join})
+      if (e) (void)hipEventDestroy(e);
+  }
   void drop_graphs() { destroy_graphs(graphs); }
 };
 
@@ -99,10 +111,31 @@ Real *state_buf(omega_state_s *S, int c, int f) {
   return S->ptr(f);
 }
 
-// Members on the stage kernels without stored diagnostics; their launches have
-// the shapes of their models' own.
-bool in_group(const omega_model_s *M, HexCoef &q) {
-  return !(M->terms & T_VDEL4) && M->stage_coef(q);
+// Which members run the stage kernels without stored diagnostics (their
+// coefficients in coef), in launches of their own beside those of the others.
+//
+// Where there are others and all members together are less than one round of
+// resident blocks (512, of 512 cells and levels), the others' launches take
+// them along at no cost, and a member of a few blocks next to them stays on
+// one XCD; us per LSRK5 step, a general member of 144 cells, 8 layers, with 16
+// lattice members of 576 cells, 16 layers: 295 so, 331 in launches of their
+// own (147000 cells and levels); 4 general members of 2304 cells, 16 layers
+// with 8 lattice members of 256 cells, 16 layers 394 and 397 (180000), of 1024
+// cells, 32 layers 685 and 437 (410000).
+std::vector<char> grouped_members(const omega_batch_s *B, std::vector<HexCoef> &coef) {
+  const size_t nm = B->mem.size();
+  std::vector<char> in(nm, 0);
+  coef.resize(nm);
+  size_t work = 0;
+  bool others = false;
+  for (size_t i = 0; i < nm; ++i) {
+    const omega_model_s *M = B->mem[i]->M;
+    in[i] = !(M->terms & T_VDEL4) && M->stage_coef(coef[i]);
+    others = others || !in[i];
+    work += (size_t)M->mesh->dm.host.ncells * M->mesh->dm.host.nlayers;
+  }
+  if (others && work < 512 * 512) std::fill(in.begin(), in.end(), 0);
+  return in;
 }
 
 void build_tables(omega_batch_s *B) {
@@ -115,7 +148,8 @@ void build_tables(omega_batch_s *B) {
   std::vector<int> blk;
   std::vector<BatchMember> geo(nm);
   std::vector<int> own(nm, -1); // group of a member on the stage kernels
-  std::vector<HexCoef> coef(nm);
+  std::vector<HexCoef> coef;
+  const std::vector<char> grouped = grouped_members(B, coef);
   B->groups.clear();
   B->any_vdel4 = false;
   for (int i = 0; i < nm; ++i) {
@@ -137,7 +171,7 @@ void build_tables(omega_batch_s *B) {
     }
     mb.cur0 = S->cur;
     mb.gen = M->gen;
-    if (in_group(M, coef[i])) {
+    if (grouped[i]) {
       const MeshView mv = M->view();
       const bool v2 = M->terms & T_VDEL2, d2 = M->terms & T_TDEL2, d4 = M->terms & T_TDEL4;
       StageKind k{stage_levels(mv, M->lc), v2, mv.tile.lx, d2, d4};
@@ -330,6 +364,11 @@ void build_tables(omega_batch_s *B) {
   if (B->desc.n != tab.size()) B->desc.alloc(tab.size());
   OMEGA_HIP_CHECK(hipMemcpy(B->desc.p, tab.data(), tab.size() * sizeof(BatchMember),
                             hipMemcpyHostToDevice));
+  if (!B->groups.empty() && B->ntable) {
+    if (!B->fork) OMEGA_HIP_CHECK(hipEventCreateWithFlags(&B->fork, hipEventDisableTiming));
+    if (!B->join) OMEGA_HIP_CHECK(hipEventCreateWithFlags(&B->join, hipEventDisableTiming));
+    if (!B->side) OMEGA_HIP_CHECK(hipStreamCreateWithFlags(&B->side, hipStreamNonBlocking));
+  }
   B->parity = 0;
   B->built = true;
 }
@@ -361,23 +400,36 @@ void step_launches(omega_batch_s *B, int parity, hipStream_t s) {
       carry_extra_tracers(mb->M, S, s);
       S->cur = keep;
     }
-  const int pers = persistent_blocks(B);
-  for (int st = 0; st < B->nstages; ++st) {
-    const BatchMember *d = B->desc.p + ((size_t)parity * B->nstages + st) * nm;
-    const int *g = B->blk.p;
-    const int n = B->ntable;
+  const int pers = persistent_blocks(B), n = B->ntable;
+  const int *g = B->blk.p;
+  // Members are independent for the whole step, so the groups' launches do not
+  // wait for the others' (us per LSRK5 step, a general member of 144 cells, 8
+  // layers, with 16 lattice members of 1024 cells, 32 layers: 502 one after the
+  // other, 388 so; of 2304 cells, 64 layers: 1136 and 850).
+  const bool both = !B->groups.empty() && n;
+  const hipStream_t gs = both ? B->side : s;
+  if (both) {
+    OMEGA_HIP_CHECK(hipEventRecord(B->fork, s));
+    OMEGA_HIP_CHECK(hipStreamWaitEvent(gs, B->fork, 0));
+  }
+  for (int st = 0; st < B->nstages; ++st)
     for (auto &gp : B->groups) {
       // the last stage leaves its input's diagnostics in the models' buffers
       const omega_batch_s::Group &G = *gp;
       const size_t at = ((size_t)parity * B->nstages + st) * G.members.size();
       const bool emit = st + 1 == B->nstages;
-      launch_stage_batch(G.kind, G.mom.p + at, G.wmom.p, G.nmom, emit, s);
-      if (G.ntile) launch_tile_batch(G.kind, G.tile.p + at, G.wtile.p, G.ntile, emit, s);
+      launch_stage_batch(G.kind, G.mom.p + at, G.wmom.p, G.nmom, emit, gs);
+      if (G.ntile) launch_tile_batch(G.kind, G.tile.p + at, G.wtile.p, G.ntile, emit, gs);
     }
-    if (!n) continue;
+  for (int st = 0; st < B->nstages && n; ++st) {
+    const BatchMember *d = B->desc.p + ((size_t)parity * B->nstages + st) * nm;
     launch_batch_diag(d, g, n, B->threads, B->N, pers, B->kinds, s);
     if (B->any_vdel4) launch_batch_vdel4(d, g, n, B->threads, B->N, pers, s);
     launch_batch_tend(d, g, n, B->threads, B->N, pers, B->kinds, B->tset, s);
+  }
+  if (both) {
+    OMEGA_HIP_CHECK(hipEventRecord(B->join, gs));
+    OMEGA_HIP_CHECK(hipStreamWaitEvent(s, B->join, 0));
   }
 }
 
@@ -536,17 +588,18 @@ int omega_batch_autotune(omega_batch_t B, int reps, double *best_ms, omega_strea
     // the others, as in records from before they had one of their own)
     std::string sig = std::to_string(B->kind) + "/" + std::to_string(B->nstages), stored = sig;
     bool shapes = false; // some member runs the launches that have them
-    for (auto &mb : B->mem) {
+    std::vector<HexCoef> coef;
+    const std::vector<char> in = grouped_members(B, coef);
+    for (size_t i = 0; i < in.size(); ++i) {
+      const auto &mb = B->mem[i];
       const HostMesh &hm = mb->M->mesh->dm.host;
       const bool hx = hex_usable(mb->M->mesh->dm.view(), mb->M->lc) && !general_only(mb->M);
-      HexCoef q;
-      const bool grouped = in_group(mb->M, q);
-      shapes = shapes || !grouped;
+      shapes = shapes || !in[i];
       const std::string member = ";" + std::to_string(hm.ncells) + ":" +
                                  std::to_string(hm.nlayers) + ":" +
                                  std::to_string(mb->M->params.ntracers) + ":" +
                                  std::to_string(mb->M->terms) + ":";
-      sig += member + (grouped ? "s" : hx ? "h" : "g");
+      sig += member + (in[i] ? "s" : hx ? "h" : "g");
       stored += member + (hx ? "h" : "g");
     }
     const char *cache = std::getenv("OMEGA_TUNE_CACHE");

@@ -48,6 +48,15 @@ struct Launched {
 size_t arg_bytes = 0;
 std::vector<Launched> launches;
 std::map<hipGraphExec_t, int> graphs; // live executables and their replays
+// streams that wait for another's work so far, with the number of launches
+// before each wait
+struct Wait {
+  hipStream_t stream, on;
+  size_t at;
+};
+std::vector<Wait> waits;
+std::map<hipEvent_t, hipStream_t> events;
+int streams = 0;
 } // namespace fake
 
 extern "C" {
@@ -106,12 +115,24 @@ hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *s) {
   return *s = hipStreamCaptureStatusNone, hipSuccess;
 }
-hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return *s = nullptr, hipSuccess; }
+static char *handle() {
+  static char *next = nullptr;
+  return ++next;
+}
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
+  ++fake::streams;
+  return *s = reinterpret_cast<hipStream_t>(handle()), hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t) { return --fake::streams, hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
+  CHECK(fake::events.count(e));
+  fake::waits.push_back({s, fake::events[e], fake::launches.size()});
+  return hipSuccess;
+}
 hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
 hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g) { return *g = nullptr, hipSuccess; }
 hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t, hipGraphNode_t *, char *, size_t) {
-  static char *next = nullptr;
-  *e = reinterpret_cast<hipGraphExec_t>(++next);
+  *e = reinterpret_cast<hipGraphExec_t>(handle());
   fake::graphs[*e] = 0;
   return hipSuccess;
 }
@@ -125,9 +146,10 @@ hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t) {
   ++fake::graphs[e];
   return hipSuccess;
 }
-hipError_t hipEventCreate(hipEvent_t *e) { return *e = nullptr, hipSuccess; }
-hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t *e) { return *e = reinterpret_cast<hipEvent_t>(handle()), hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCreate(e); }
+hipError_t hipEventDestroy(hipEvent_t e) { return fake::events.erase(e), hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { return fake::events[e] = s, hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { return *ms = 1, hipSuccess; }
 }
@@ -443,11 +465,11 @@ static void tuning() {
   }
   // with a member on the other kernels: every shape
   {
-    Ensemble e(3, 16, 16, 64, Ensemble::params(2), OMEGA_STEPPER_RK4);
+    Ensemble e(3, 128, 128, 64, Ensemble::params(2), OMEGA_STEPPER_RK4);
     ok(omega_model_set_kernel_forms(e.models[1], 3));
     const auto n = launched(0, [&] { ok(omega_batch_autotune(e.batch, 3, nullptr, nullptr)); });
     CHECK(n.size() == 24 * 4 * (2 + 2) * (1 + 3));
-    CHECK(contents(cache).rfind("0/4;256:64:2:7:s;256:64:2:7:h;256:64:2:7:s ", 0) == 0);
+    CHECK(contents(cache).rfind("0/4;16384:64:2:7:s;16384:64:2:7:h;16384:64:2:7:s ", 0) == 0);
   }
   std::remove(cache.c_str());
   CHECK(rmdir(dir) == 0);
@@ -492,6 +514,37 @@ static void few_launches() {
   for (auto m : meshes) ok(omega_mesh_destroy(m));
 }
 
+// Next to others small members run the others' kernels: no launches more.
+// Members on the stage kernels do not wait for those on the others: their
+// launches run on a stream of the batch's, which starts after what came before
+// the step and ends before what comes after it.
+static void side_by_side() {
+  const int streams = fake::streams;
+  {
+    Ensemble e(3, 16, 16, 64, Ensemble::params(1), OMEGA_STEPPER_RK4);
+    ok(omega_model_set_kernel_forms(e.models[1], 3));
+    CHECK(launched(0, [&] { ok(omega_batch_step(e.batch, nullptr)); }).size() == 4 * 2);
+  }
+  {
+    Ensemble e(3, 128, 128, 64, Ensemble::params(1), OMEGA_STEPPER_RK4);
+    const hipStream_t s = reinterpret_cast<hipStream_t>(handle());
+    fake::waits.clear();
+    for (const auto &l : launched(0, [&] { ok(omega_batch_step(e.batch, reinterpret_cast<omega_stream_t>(s))); }))
+      CHECK(l.stream == s);
+    CHECK(fake::waits.empty());
+    ok(omega_model_set_kernel_forms(e.models[1], 3));
+    const auto n = launched(0, [&] { ok(omega_batch_step(e.batch, reinterpret_cast<omega_stream_t>(s))); });
+    CHECK(n.size() == 4 * (2 + 2) && fake::waits.size() == 2);
+    const auto &from = fake::waits[0], &to = fake::waits[1];
+    CHECK(from.on == s && from.stream != s && from.at == 0);
+    CHECK(to.on == from.stream && to.stream == s && to.at == n.size());
+    size_t side = 0;
+    for (const auto &l : n) side += l.stream == from.stream;
+    CHECK(side == 4 * 2);
+  }
+  CHECK(fake::streams == streams);
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, std::function<void()>> checks = {{"tall", tall}, {"rebuild", rebuild},
                                                               {"keep_stepper", keep_stepper},
@@ -500,7 +553,8 @@ int main(int argc, char **argv) {
                                                               {"tuned_cells", tuned_cells},
                                                               {"reports", reports},
                                                               {"tuning", tuning},
-                                                              {"few_launches", few_launches}};
+                                                              {"few_launches", few_launches},
+                                                              {"side_by_side", side_by_side}};
   CHECK(argc == 2 && checks.count(argv[1]));
   checks.at(argv[1])();
   std::printf("%s ok\n", argv[1]);

@@ -317,3 +317,32 @@ def test_ensemble_of_any_terms_and_layers_bitwise(kind, del4):
         solo = upload(mesh, ntr, y0)
         (swe.RK4Stepper(model) if kind == "rk4" else swe.LSRKStepper(model, 5)).run(0.0, 15.0, 3, solo)
         compare(s.download(), solo.download(), mesh.nlayers, model.terms)
+
+
+@pytest.mark.parametrize("kind", ["rk4", "lsrk"])
+@pytest.mark.parametrize("graph", [True, False])
+def test_ensemble_side_by_side_bitwise(kind, graph):
+    """Members on the stage kernels beside members on the others (momentum
+    del4, kernel forms), too large to share launches: several replays with
+    uploads, downloads and solo steps between them."""
+    b, members = swe.Batch(kind, 5), []
+    for i, (nx, L, ntr, terms, forms) in enumerate(((66, 64, 1, 79, 15), (12, 8, 2, 127, 15),
+                                                    (40, 5, 3, 111, 15), (12, 64, 1, 15, 3))):
+        mesh = swe.PlanarHexagonalMesh(nx, nx, 10e3, L)
+        model = swe.ShallowWaterModel(mesh, swe.ShallowWaterParams(**params_dict(10e3, ntr)))
+        model.terms = terms
+        model.set_kernel_forms(forms)
+        y0 = rich_state(mesh, L, ntr, i)
+        s, solo = upload(mesh, ntr, y0), upload(mesh, ntr, y0)
+        b.add(model, s, 15.0)
+        st = swe.RK4Stepper(model) if kind == "rk4" else swe.LSRKStepper(model, 5)
+        members.append((s, solo, st))
+    b.set_graph(graph)
+    for again in range(4):
+        print("case", kind, graph, again, flush=True)
+        b.run(2)
+        for i, (s, solo, st) in enumerate(members):
+            st.run(0.0, 15.0, 2, solo)
+            got = s.download()
+            compare(got, solo.download(), again, i)
+            s.upload(*got)
