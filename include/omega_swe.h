@@ -487,7 +487,8 @@ int omega_adjoint_run(omega_stepper_t stepper, double t0, double dt, int nsteps,
  * every member by one do_step of the batch's stepper kind, with each stage
  * phase (diagnostics, momentum del4 pre-pass, tendency + update) a single
  * launch over all members.  Each member's state ends bit-identical to
- * stepping it alone.  Members must not have an additional-tendency hook.
+ * stepping it alone, also where members share a model (its auxiliary state is
+ * then the first one's).  Members must not have an additional-tendency hook.
  * -------------------------------------------------------------------- */
 typedef struct omega_batch_s *omega_batch_t;
 
@@ -507,8 +508,8 @@ int omega_batch_set_graph(omega_batch_t batch, int enable);
  * the others the general ones inside it.  Members whose models take the stage
  * kernels without stored diagnostics (bit 5 of omega_model_kernel_flags, no
  * momentum del4) have launches of their own, one for momentum and one for
- * tracers for those of each number of levels per lane, with 256 threads and the levels per lane and block
- * order of their models, beside those of the others on a stream of the
+ * tracers for those of each number of levels per lane, with 256 threads and
+ * the levels per lane and block order of their models, beside those of the others on a stream of the
  * batch's (next to others and below 262144 cells and levels in all they run
  * with them): this setting, the persistent grid and the autotuner below are
  * for the others. */

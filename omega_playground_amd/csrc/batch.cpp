@@ -34,6 +34,7 @@ struct omega_batch_s {
     DBuf<Real> acc[3], p1[3], p2[3]; // RK4
     DBuf<Real> tend[3];              // LSRK
     uint64_t gen = 0;                // model configuration the tables hold
+    omega_model_s::DiagSet diag;     // where an earlier member has the same model
   };
   std::vector<std::unique_ptr<Member>> mem;
   int N = 2;         // levels per lane
@@ -136,6 +137,30 @@ std::vector<char> grouped_members(const omega_batch_s *B, std::vector<HexCoef> &
   }
   if (others && work < 512 * 512) std::fill(in.begin(), in.end(), 0);
   return in;
+}
+
+// Where member i's diagnostics go: to its model's buffers, or, if an earlier
+// member has the same model, to buffers of its own (the launches step both).
+DiagOut member_diag(omega_batch_s *B, int i) {
+  omega_model_s *M = B->mem[i]->M;
+  DiagOut d = M->diag();
+  bool shared = false;
+  for (int j = 0; j < i; ++j) shared = shared || B->mem[j]->M == M;
+  if (!shared) return d;
+  auto own = [](DBuf<Real> &b, const DBuf<Real> &like) {
+    if (b.n != like.n) b.alloc(like.n);
+    return b.p;
+  };
+  omega_model_s::DiagSet &s = B->mem[i]->diag;
+  d.rvort_v = own(s.rvort_v, M->rvort_v);
+  d.inv_thick_v = own(s.inv_thick_v, M->inv_thick_v);
+  d.ke_c = own(s.ke_c, M->ke_c);
+  d.div_c = own(s.div_c, M->div_c);
+  d.trdel2_c = own(s.trdel2_c, M->trdel2_c);
+  d.vdel2_e = own(s.vdel2_e, M->vdel2_e);
+  d.vdel2_rv_v = own(s.vdel2_rv_v, M->vdel2_rv_v);
+  d.vdel2_div_c = own(s.vdel2_div_c, M->vdel2_div_c);
+  return d;
 }
 
 void build_tables(omega_batch_s *B) {
@@ -263,6 +288,8 @@ void build_tables(omega_batch_s *B) {
     gt[j].tile.resize((size_t)2 * ns * mem.size());
     for (size_t q = 0; q < mem.size(); ++q) place[mem[q]] = (int)q;
   }
+  std::vector<DiagOut> diag(nm);
+  for (int i = 0; i < nm; ++i) diag[i] = member_diag(B, i);
   std::vector<BatchMember> tab((size_t)2 * ns * nm);
   for (int p = 0; p < 2; ++p)
     for (int s = 0; s < ns; ++s)
@@ -273,7 +300,7 @@ void build_tables(omega_batch_s *B) {
         BatchMember g = geo[i];
         g.m = M->view();
         g.mc = M->coef();
-        g.d = M->diag();
+        g.d = diag[i];
         StageArgs a{};
         a.terms = M->terms;
         a.do_h = !M->params.disable_h_tendency;

@@ -10,11 +10,13 @@
 #include <functional>
 #include <iterator>
 #include <map>
+#include <set>
 #include <string>
 #include <vector>
 
 #include <unistd.h>
 
+#include "batch.hpp"
 #include "stage_launch.hpp"
 
 using namespace omega_hip;
@@ -545,6 +547,39 @@ static void side_by_side() {
   CHECK(fake::streams == streams);
 }
 
+// Members of one model have diagnostics of their own: no two members of a
+// launch write the same rows.
+static void one_model() {
+  for (int terms : {7, 7 + 16}) { // the stage kernels' ensemble launches, the others'
+    omega_mesh_t mesh;
+    omega_model_t model;
+    omega_batch_t batch;
+    std::vector<omega_state_t> states(3);
+    const omega_params p = Ensemble::params(1);
+    ok(omega_mesh_create_planar_hex(12, 10, 1e4, 64, OMEGA_ORDER_HILBERT, &mesh));
+    ok(omega_model_create(mesh, &p, &model));
+    ok(omega_model_set_terms(model, terms));
+    ok(omega_batch_create(OMEGA_STEPPER_RK4, 4, &batch));
+    for (auto &s : states) {
+      ok(omega_state_create(mesh, 1, &s));
+      ok(omega_batch_add(batch, model, s, 10.0, nullptr));
+    }
+    const auto n = launched(sizeof(void *), [&] { ok(omega_batch_step(batch, nullptr)); });
+    std::set<const double *> rows;
+    for (int i = 0; i < 3; ++i) {
+      const DiagOut &d = terms == 7 ? n[6].at<const StageLaunch *>()[i].d : n[0].at<const BatchMember *>()[i].d;
+      for (const double *x : {d.rvort_v, d.inv_thick_v, d.ke_c, d.div_c, d.trdel2_c}) CHECK(x && rows.insert(x).second);
+      if (terms != 7)
+        for (const double *x : {d.vdel2_e, d.vdel2_rv_v, d.vdel2_div_c}) CHECK(x && rows.insert(x).second);
+    }
+    ok(omega_batch_destroy(batch));
+    for (auto s : states) ok(omega_state_destroy(s));
+    ok(omega_model_destroy(model));
+    ok(omega_mesh_destroy(mesh));
+    CHECK(fake::bytes == 0);
+  }
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, std::function<void()>> checks = {{"tall", tall}, {"rebuild", rebuild},
                                                               {"keep_stepper", keep_stepper},
@@ -554,7 +589,8 @@ int main(int argc, char **argv) {
                                                               {"reports", reports},
                                                               {"tuning", tuning},
                                                               {"few_launches", few_launches},
-                                                              {"side_by_side", side_by_side}};
+                                                              {"side_by_side", side_by_side},
+                                                              {"one_model", one_model}};
   CHECK(argc == 2 && checks.count(argv[1]));
   checks.at(argv[1])();
   std::printf("%s ok\n", argv[1]);

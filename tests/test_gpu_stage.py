@@ -346,3 +346,25 @@ def test_ensemble_side_by_side_bitwise(kind, graph):
             got = s.download()
             compare(got, solo.download(), again, i)
             s.upload(*got)
+
+
+@pytest.mark.parametrize("terms", [79, 127])
+@pytest.mark.parametrize("L", [7, 64])
+def test_ensemble_of_one_model_bitwise(terms, L):
+    """Members that share a model: the stage kernels (79) and, with momentum
+    del4, the kernels that store the diagnostics."""
+    ntr, n = 2, 5
+    mesh = swe.PlanarHexagonalMesh(14, 12, 10e3, L)
+    model = swe.ShallowWaterModel(mesh, swe.ShallowWaterParams(**params_dict(10e3, ntr)))
+    model.terms = terms
+    y0 = [rich_state(mesh, L, ntr, i) for i in range(n)]
+    b, states = swe.Batch("lsrk", 5), [upload(mesh, ntr, y) for y in y0]
+    for s in states:
+        b.add(model, s, 15.0)
+    b.run(3)
+    aux = model.aux_array("ke_cell")
+    for i in reversed(range(n)):
+        solo = upload(mesh, ntr, y0[i])
+        swe.LSRKStepper(model, 5).run(0.0, 15.0, 3, solo)
+        compare(states[i].download(), solo.download(), i)
+    assert same_bits(aux, model.aux_array("ke_cell"))
