@@ -277,7 +277,10 @@ void launch_stage_hex(const MeshView &m, const Launch &lc, const HexCoef &q, con
 // adjoint's PV pass then reads the edges-on-edge sums instead of forming them
 // (step adjoint at nx=256, 64 layers, 1 tracer: 2286 -> 2272 us).  The tracers'
 // Laplacian comes along in the same launch (6-step gradient at 1920 cells, 20
-// layers: 1600 -> 1557 us) but is not worth a tile launch of its own.
+// layers: 1600 -> 1557 us) but is not worth a tile launch of its own, nor with
+// two levels per lane one in which a block takes all tracers of its tile: us
+// per tendency VJP with tracer del4, 64 layers, 102 against 105 at 2304 cells,
+// 2 tracers, but 107, 115, 134 against 106, 113, 127 at 4096 cells, 1, 2 and 4.
 bool launch_stage_rows(const MeshView &m, const Launch &lc, const HexCoef &q, StageArgs a,
                        const DiagOut &d, const PreOut &pre, hipStream_t s) {
   a.epi = EPI_NONE;
@@ -290,6 +293,7 @@ bool launch_stage_rows(const MeshView &m, const Launch &lc, const HexCoef &q, St
     const int N = stage_levels(m, lc);
     stage_launch(m, lc, N, q, a, d, p, t);
     if ((a.terms & T_VDEL4) || !stage_one_launch(N, p, t)) return false;
+    if (N == 2 && t.work >= kFewTiles) return false;
   }
   launch_stage_hex(m, lc, q, a, d, true, s, &pre);
   return true;

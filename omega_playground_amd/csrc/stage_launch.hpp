@@ -46,7 +46,12 @@ inline void whole_blocks(StageLaunch &p) {
   p.tiles = p.ncb * nch;
 }
 
-// Fewer tiles than this (two blocks per CU) leave the chip short of blocks.
+// Fewer tiles than this (two blocks per CU) leave the chip short of blocks, so
+// each tracer has blocks of its own; us per RK4 step with del4, a block for all
+// tracers of a tile or for each: one layer, 4 tracers 50 against 36 at 144
+// tiles, 69 against 66 at 400, but 81 against 98 at 576; 64 layers 60 against
+// 48 at 128 tiles, 71 against 62 at 200, 89 against 98 at 288 (2 tracers 69
+// against 63), 116 against 123 at 512.
 constexpr int kFewTiles = 512;
 
 // Both in one launch, where that is the faster one (kernels_stage_both.hip);

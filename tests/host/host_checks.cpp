@@ -580,6 +580,34 @@ static void one_model() {
   }
 }
 
+// A tendency VJP with tracer del4 takes its diagnostics from the stage kernels
+// where their launch has a block for each tracer of a tile, and without del4
+// at any size.
+static void vjp_rows() {
+  struct Case {
+    int nx, L, ntr, terms, diag;
+  };
+  for (const Case &c : {Case{48, 64, 2, 79, 0}, Case{64, 64, 1, 79, 1}, Case{64, 64, 9, 79, 1},
+                        Case{64, 64, 9, 15, 0}, Case{80, 25, 4, 79, 0}, Case{128, 64, 2, 79, 1},
+                        Case{128, 64, 2, 15, 0}}) {
+    Ensemble e(1, c.nx, c.nx, c.L, Ensemble::params(c.ntr), OMEGA_STEPPER_RK4);
+    ok(omega_model_set_terms(e.models[0], c.terms));
+    omega_state_t cot[2];
+    for (auto &s : cot) ok(omega_state_create(e.mesh, c.ntr, &s));
+    ok(omega_timing_enable(1));
+    ok(omega_timing_reset());
+    ok(omega_model_tendency_vjp(e.models[0], e.states[0], cot[0], cot[1], nullptr, nullptr));
+    double ms;
+    int64_t diag = 0;
+    ok(omega_timing_read("diag", &ms, &diag));
+    ok(omega_timing_enable(0));
+    std::printf("%d x %d cells, %d levels, %d tracers, terms %d: %d\n", c.nx, c.nx, c.L, c.ntr, c.terms,
+                (int)diag);
+    CHECK(diag == c.diag);
+    for (auto &s : cot) ok(omega_state_destroy(s));
+  }
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, std::function<void()>> checks = {{"tall", tall}, {"rebuild", rebuild},
                                                               {"keep_stepper", keep_stepper},
@@ -590,7 +618,8 @@ int main(int argc, char **argv) {
                                                               {"tuning", tuning},
                                                               {"few_launches", few_launches},
                                                               {"side_by_side", side_by_side},
-                                                              {"one_model", one_model}};
+                                                              {"one_model", one_model},
+                                                              {"vjp_rows", vjp_rows}};
   CHECK(argc == 2 && checks.count(argv[1]));
   checks.at(argv[1])();
   std::printf("%s ok\n", argv[1]);

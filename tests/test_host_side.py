@@ -24,7 +24,7 @@ def program(tmp_path_factory):
 
 @pytest.mark.parametrize("what", ["tall", "rebuild", "keep_stepper", "keep_ensemble", "block_order",
                                   "tuned_cells", "reports", "tuning", "few_launches",
-                                  "side_by_side", "one_model"])
+                                  "side_by_side", "one_model", "vjp_rows"])
 def test_host_side(program, what):
     r = subprocess.run([program, what], capture_output=True, text=True, timeout=120)
     print(r.stdout, r.stderr, flush=True)
