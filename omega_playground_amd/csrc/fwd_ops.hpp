@@ -432,11 +432,13 @@ __device__ __forceinline__ void cell_tend(const MeshView &m, const ModelCoef &mc
 // lookup) instead of its two cells' and two vertices' rows (7 rows, three
 // lookups in a chain), and no cell forms its neighbours' inverse thicknesses.
 // Same values and summation order.  160 x 120 cells, 32 layers, 2 tracers,
-// del2 mixing: 664 -> 475 us per RK4 step; what is left is the rows' delivery
+// del2 mixing: 664 -> 510 us per RK4 step; what is left is the rows' delivery
 // through L1 and the tables read per lane.
 // ---------------------------------------------------------------------------
 constexpr int kSlots = 5; // PV slots whose rows are loaded together
-constexpr int kSides = 2; // cell edges likewise (three cost a wave per SIMD: 518 against 475 us per step)
+// cell edges likewise (three cost a wave per SIMD: 518 against 475 us per step,
+// both stepping one state over and over)
+constexpr int kSides = 2;
 
 // the means of edge e (thickness_aux.hpp:33-52, vorticity_aux.hpp:118-132)
 template <int N>

@@ -7,7 +7,7 @@
 // rows per cell (nx=512, 64 layers, 4 tracers, del2 viscosity, tracer del4):
 // 2.37 -> 1.57 ms per RK4 stage, 68 -> 44 rows per cell through HBM.  At 60
 // layers, where that pair ran the general kernels, 0.250 -> 0.077 ms (150 x
-// 94 cells, 3 tracers); one layer, 512 x 384 cells: 0.135 -> 0.019 ms.
+// 94 cells, 3 tracers); one layer, 512 x 384 cells: 0.135 -> 0.016 ms.
 #include <algorithm>
 
 #include "stage_blocks.hpp"

@@ -28,9 +28,9 @@ __device__ __forceinline__ bool stage_place(const StageLaunch &p, int entry, int
 }
 
 // Momentum and thickness.  Two levels per lane at two waves per SIMD (228
-// registers) take 0.70 ms at nx=512, 64 layers (3.6 TB/s; the vector units
-// half busy, the rest latency), one level per lane at four waves 0.83 ms (the
-// same rows in twice the load instructions).
+// registers) take 0.68 ms per stage at nx=512, 64 layers (2.25 GB, 3.3 TB/s;
+// the vector units half busy, the rest latency), one level per lane at four
+// waves 0.83 ms (the same rows in twice the load instructions).
 // V4: subtract the del4 rows (p.x) the Laplacian launches left.
 template <int N, bool V2, bool V4, bool EMIT, bool PRE = false>
 __device__ __forceinline__ void stage_mom(const StageLaunch &p, int entry) {
