@@ -55,7 +55,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N == 1
   const int w = uniform(who[blockIdx.x]);
   if (w < 0) return;
   const StageLaunch &p = constant_at(desc, w);
-  const int entry = logical_block((int)blockIdx.x - p.block0, p.tiles, p.swz);
+  const int entry = block_entry((int)blockIdx.x - p.block0, p.tiles, p.swz);
   if constexpr (V2 != kAny) {
     stage_mom<N, V2 != 0, false, EMIT>(p, entry);
   } else {
@@ -95,9 +95,11 @@ __global__ void __launch_bounds__(256) k_stage_lap(StageLaunch p) {
 template <int N, int LX, int TW, int TH, bool D2, bool D4, bool EMIT>
 __global__ void __launch_bounds__(LX *TW *TH) __attribute__((amdgpu_waves_per_eu(N == 2 ? 3 : 4)))
     k_stage_tile(TileLaunch p) {
-  __shared__ TileRows<N, LX, TW, TH, D4> rows;
-  stage_tile<N, LX, TW, TH, D2, D4, EMIT>(p, xcd_entry(p.work, p.swz), (int)blockIdx.y * p.per_block,
-                                          rows);
+  using R = TileRows<N, LX, TW, TH, D4>;
+  __shared__ double h[R::ROWS], ratio[R::ROWS], lap[R::LAPS];
+  __shared__ int ids[R::PLACES];
+  stage_tile<N, LX, TW, TH, D2, D4, EMIT>(p, xcd_entry(p.work, p.swz), (int)blockIdx.y * p.per_block, h,
+                                          ratio, lap, ids);
 }
 
 // Ensemble form (k_batch_mom); tiles of all shapes share the LDS.  D4: some
@@ -107,8 +109,8 @@ __device__ __forceinline__ void batch_tile(const TileLaunch &p, int entry, char 
   auto body = [&](auto D2_, auto D4_) {
     constexpr bool d2 = decltype(D2_)::value, d4 = decltype(D4_)::value;
     // without del4 there is no Laplacian to emit
-    stage_tile<N, LX, TW, TH, d2, d4, EMIT && d4>(p, entry, 0,
-                                                  *reinterpret_cast<TileRows<N, LX, TW, TH, d4> *>(mem));
+    auto &r = *reinterpret_cast<TileRows<N, LX, TW, TH, d4> *>(mem);
+    stage_tile<N, LX, TW, TH, d2, d4, EMIT && d4>(p, entry, 0, r.h, r.ratio, r.lap, r.ids);
   };
   constexpr std::true_type yes{};
   constexpr std::false_type no{};
@@ -137,7 +139,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N == 2
   const int w = uniform(who[blockIdx.x]);
   if (w < 0) return;
   const TileLaunch &p = constant_at(desc, w);
-  const int entry = logical_block((int)blockIdx.x - p.block0, p.work, p.swz);
+  const int entry = block_entry((int)blockIdx.x - p.block0, p.work, p.swz);
   if (LX == 4 || (LX == kAny && p.lx == 4)) batch_tile<N, 4, 8, 8, D2, D4, EMIT>(p, entry, mem);
   else if (LX == 2 || (LX == kAny && p.lx == 2)) batch_tile<N, 2, 16, 8, D2, D4, EMIT>(p, entry, mem);
   else batch_tile<N, 1, 16, 16, D2, D4, EMIT>(p, entry, mem);

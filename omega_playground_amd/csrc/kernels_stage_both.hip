@@ -22,9 +22,12 @@ __global__ void __launch_bounds__(256)
     stage_mom<N, V2, false, E != kNothing, E == kPre>(p, b);
   } else {
     // tiles of all tracers of a group, then the next group
-    __shared__ TileRows<N, LX, TW, TH, D4> rows;
+    using R = TileRows<N, LX, TW, TH, D4>;
+    __shared__ double h[R::ROWS], ratio[R::ROWS], lap[R::LAPS];
+    __shared__ int ids[R::PLACES];
     const int w = b - p.tiles, group = uniform(w / t.work);
-    stage_tile<N, LX, TW, TH, D2, D4, E != kNothing>(t, w - group * t.work, group * t.per_block, rows);
+    stage_tile<N, LX, TW, TH, D2, D4, E != kNothing>(t, w - group * t.work, group * t.per_block, h,
+                                                     ratio, lap, ids);
   }
 }
 

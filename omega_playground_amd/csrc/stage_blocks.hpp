@@ -9,12 +9,15 @@
 namespace omega_hip {
 namespace stage {
 
-// Entry b of n for this block: workgroups are dealt to the 8 XCDs
-// round-robin, and with swz each XCD takes a contiguous range of entries, so
-// that neighbouring cells' rows are re-read from one L2.
-__device__ __forceinline__ int xcd_entry(int n, int swz) {
-  return logical_block((int)blockIdx.x, n, swz);
+// Entry of block b of n: workgroups are dealt to the 8 XCDs round-robin, and
+// with swz each XCD takes a contiguous range of entries, so that neighbouring
+// cells' rows are re-read from one L2.  (Chosen without a branch, which cost
+// 0.1 us of a 5 us launch.)
+__device__ __forceinline__ int block_entry(int b, int n, int swz) {
+  const int e = logical_block(b, n, 1);
+  return swz ? e : b;
 }
+__device__ __forceinline__ int xcd_entry(int n, int swz) { return block_entry((int)blockIdx.x, n, swz); }
 
 // The cell and levels of this thread at an entry (level chunk, cell block);
 // false: no work here.
@@ -91,13 +94,15 @@ __device__ __forceinline__ void stage_mom(const StageLaunch &p, int entry) {
   epilogue<N>(a, a.h, idx, T);
 }
 
-// A tile's rows in LDS: thickness, tracer ratio and Laplacian, and its cells
+// A tile's LDS: rows of thickness, tracer ratio and (D4) Laplacian at its places,
+// and the cells there
 template <int N, int LX, int TW, int TH, bool D4> struct TileRows {
   static constexpr int HALO = D4 ? 2 : 1;
-  static constexpr int NP = (TW + 2 * HALO) * (TH + 2 * HALO), PLANE = NP * LX * N;
-  alignas(16) double h[PLANE];
-  double ratio[PLANE], lap[D4 ? PLANE : 1];
-  int ids[NP];
+  static constexpr int PLACES = (TW + 2 * HALO) * (TH + 2 * HALO), ROWS = PLACES * LX * N,
+                       LAPS = D4 ? ROWS : 1;
+  alignas(16) double h[ROWS];
+  double ratio[ROWS], lap[LAPS];
+  int ids[PLACES];
 };
 
 // ---------------------------------------------------------------------------
@@ -114,15 +119,13 @@ template <int N, int LX, int TW, int TH, bool D4> struct TileRows {
 // SIMD faster than four with 13 registers spilled (6.3 against 7.0).
 // ---------------------------------------------------------------------------
 template <int N, int LX, int TW, int TH, bool D2, bool D4, bool EMIT>
-__device__ __forceinline__ void stage_tile(const TileLaunch &p, int w, int l0,
-                                           TileRows<N, LX, TW, TH, D4> &rows) {
+__device__ __forceinline__ void stage_tile(const TileLaunch &p, int w, int l0, double *Hs, double *Ns,
+                                           double *Ds, int *ids) {
   constexpr int HALO = D4 ? 2 : 1, PW = TW + 2 * HALO, PH = TH + 2 * HALO, NP = PW * PH;
   constexpr int CELLS = TW * TH, R = (NP + CELLS - 1) / CELLS;
   constexpr int RING = 2 * (TW + 2) + 2 * TH; // the first ring round the tile
   static_assert(RING <= CELLS, "one place of the ring per row of lanes");
   constexpr int S = LX * N; // doubles per place and array
-  double *const Hs = rows.h, *const Ns = rows.ratio, *const Ds = rows.lap;
-  int *const ids = rows.ids;
   const int tile = uniform(w / p.nch), ch = w - tile * p.nch;
   const int ln = (int)threadIdx.x % LX, row = (int)threadIdx.x / LX;
   const int L = p.L, k = (ch * LX + ln) * N;
