@@ -484,9 +484,8 @@ int omega_adjoint_run(omega_stepper_t stepper, double t0, double dt, int nsteps,
  * Ensembles.  No reference counterpart: the reference steps one model at a
  * time.  Members are (model, state, dt) triples with their own meshes,
  * layer counts, tracer counts and coefficients; one batch step advances
- * every member by one do_step of the batch's stepper kind, with each stage
- * phase (diagnostics, momentum del4 pre-pass, tendency + update) a single
- * launch over all members.  Each member's state ends bit-identical to
+ * every member by one do_step of the batch's stepper kind, in a few launches
+ * per stage over all members (omega_batch_set_launch).  Each member's state ends bit-identical to
  * stepping it alone, also where members share a model (its auxiliary state is
  * then the first one's).  Members must not have an additional-tendency hook.
  * -------------------------------------------------------------------- */

@@ -786,8 +786,8 @@ def adjoint_run(stepper: "_Stepper", t0: float, dt: float, nsteps: int, state: S
 # Ensembles (no reference counterpart)
 # ---------------------------------------------------------------------------
 class Batch:
-    """Ensemble of independent (model, state, dt) members advanced together,
-    one launch per stage phase for all members."""
+    """Ensemble of independent (model, state, dt) members advanced together, in
+    a few launches per stage over all members."""
 
     def __init__(self, kind: str = "lsrk", nstages: int = 5):
         h = C.c_void_p()
