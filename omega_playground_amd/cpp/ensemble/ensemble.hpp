@@ -1,9 +1,9 @@
 // Ensembles of independent members (no reference counterpart: the
 // reference steps one model at a time).  A member is a model, its state and
 // its dt; an Ensemble step advances every member by one step of the
-// ensemble's stepper kind in a few launches per stage over all members, and each member's state ends bit-identical to stepping it alone.  The
-// Ensemble keeps references to the members' models and states: keep them
-// alive.
+// ensemble's stepper kind in a few launches per stage over all members, and
+// each member's state ends bit-identical to stepping it alone.  The Ensemble
+// keeps references to the members' models and states: keep them alive.
 #pragma once
 
 #include <vector>
